@@ -1,0 +1,96 @@
+"""The pipelined loop of the gemm tiles (ttm_gemm.hip, PIPE).
+
+On the CPU: the ragged last slice of an interior tile (load_ragged), whose
+vectors are read at moved, in-range addresses and shifted and masked at the
+store, takes exactly the elements of the slice and no read leaves its operand.
+On the GPU: contractions around the lengths where the loop starts and where
+its last slices change (whole and ragged), every view, both B orientations,
+against the FP64 brute force, normwise <= 4 n_q eps.
+"""
+import itertools
+
+import numpy as np
+import pytest
+
+import refcases as rc
+from test_tile_bounds_cpu import gemm_configs
+
+
+def _shift_mask(v, d, nvalid, zero=None):
+    return [(v[x + d] if x + d < len(v) else v[x]) if x < nvalid else zero for x in range(len(v))]
+
+
+@pytest.mark.parametrize("cfg", [c for c in gemm_configs() if not c[7]], ids=lambda c: "-".join(map(str, c)))
+def test_ragged_slice_takes_its_elements(cfg):
+    t, vec, JT, NT, WM, BK, tn, bcol, _ = cfg
+    BM, BN = WM * 16 * JT, (4 // WM) * 16 * NT
+    for nq, m in itertools.product((BK + 1, BK + vec - 1, 2 * BK + 3, 3 * BK - 1), (BM, BM + vec)):
+        w, outer = (1, BN) if tn else (BN, 1)
+        l0 = nq // BK * BK
+        j0 = 0 if m == BM else BM  # the second row block of m = BM + vec reads rows past m in place of none
+
+        def along(row, l):  # (addresses, kept elements) of a vector along l
+            lc = min(l, nq - vec)
+            nvalid = 0 if l >= nq else min(vec, nq - l)
+            return _shift_mask([row + lc + x for x in range(vec)], l - lc, nvalid), row + lc
+
+        def across(col, l, step):
+            start = col + min(l, nq - 1) * step
+            return _shift_mask([start + x for x in range(vec)], 0, vec if l < nq else 0), start
+
+        for v in range(BK * BN // vec):
+            if tn:
+                n, r = v // (BK // vec), v % (BK // vec) * vec
+                kept, start = along(n * nq, l0 + r)
+                want = [n * nq + l0 + r + x if l0 + r + x < nq else None for x in range(vec)]
+            else:
+                r, n = v // (BN // vec), v % (BN // vec) * vec
+                kept, start = across(n, l0 + r, w)
+                want = [n + x + (l0 + r) * w if l0 + r < nq else None for x in range(vec)]
+            assert kept == want and 0 <= start and start + vec <= outer * nq * w
+        for v in range(BK * BM // vec):
+            if bcol:
+                if (m - j0) % vec and j0 + BM > m:
+                    continue
+                r, j = v // (BM // vec), j0 + v % (BM // vec) * vec
+                jc = j if j + vec <= m else m - vec
+                kept, start = across(jc, l0 + r, m)
+                want = [jc + x + (l0 + r) * m if l0 + r < nq else None for x in range(vec)]
+            else:
+                j, r = j0 + v // (BK // vec), v % (BK // vec) * vec
+                jc = min(j, m - 1)
+                kept, start = along(jc * nq, l0 + r)
+                want = [jc * nq + l0 + r + x if l0 + r + x < nq else None for x in range(vec)]
+            assert kept == want and 0 <= start and start + vec <= m * nq
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,nqs", [(np.float32, (95, 96, 97, 112, 127, 192, 193, 225)),
+                                       (np.float64, (383, 384, 385, 399, 416, 433))])
+def test_contractions_around_the_pipelined_loop(gpu, oracle, dtype, nqs):
+    import torch
+    import ttm_amd
+    tdt = torch.float32 if dtype == np.float32 else torch.float64
+    rng = np.random.default_rng(71)
+    for nq, m, view in itertools.product(nqs, (10, 20, 40, 130), ("tn", "nn", "pad")):
+        na, pia, q = {"tn": ([nq, 300], [1, 2], 1), "nn": ([260, nq], [1, 2], 2),
+                      "pad": ([131, nq, 2], [1, 2, 3], 2)}[view]
+        wa = rc.dense_strides(na, pia)
+        nc = list(na)
+        nc[q - 1] = m
+        wc = rc.dense_strides(nc, pia)
+        a = rng.uniform(-1, 1, int(np.prod(na))).astype(dtype)
+        Bm = rng.uniform(-1, 1, (m, nq)).astype(dtype)
+        A = torch.from_numpy(a).to(gpu)
+        for colmajor in (False, True):
+            b = (Bm.T if colmajor else Bm).reshape(-1).copy()
+            label = f"{np.dtype(dtype).name} {view} nq={nq} m={m} col={colmajor}"
+            print(label, flush=True)
+            C = torch.full((int(np.prod(nc)),), float("nan"), dtype=tdt, device=gpu)
+            ttm_amd.force_kernel("gemm")
+            ttm_amd.ttm_raw(q, len(na), A, na, wa, pia, torch.from_numpy(b).to(gpu), [m, nq],
+                            [1, 2] if colmajor else [2, 1], C, nc, wc)
+            torch.cuda.synchronize()
+            c64 = oracle.ttm_brute_f64(q, a, na, wa, b, m, colmajor, nc, wc)
+            err = rc.normwise_error(C.cpu().numpy(), c64, a, b)
+            assert err <= 4 * nq * rc.eps(dtype), (label, ttm_amd.last_kernel(), err)

@@ -184,7 +184,8 @@ struct TileShape
 // PAD (NN view only): slabs of any width w and element-aligned A and C (a_len:
 // elements of A from a to its end; A holds at least VEC); off, the NN view requires
 // w % VEC == 0 and 16-byte aligned A and C (wp == w).
-template <class T, int JT, int NT, int WAVES_M, int BK, int VIEW, bool BCOL, bool PAD = false>
+// PIPE: the interior tiles' slices run in the pipelined loop below.
+template <class T, int JT, int NT, int WAVES_M, int BK, int VIEW, bool BCOL, bool PAD = false, bool PIPE = false>
 __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__restrict__ b, T *__restrict__ c,
                                           uint64_t ncols, uint64_t nq, uint64_t ld, uint64_t w, uint64_t wp,
                                           uint64_t m, uint64_t j0, uint64_t n0, unsigned flags, uint64_t a_len,
@@ -238,53 +239,62 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     constexpr int B_VECS = BK * BM / VEC;
     constexpr int B_PER = (B_VECS + 255) / 256;
 
-    // per-thread fixed part of the A addresses; NN vectors are VEC padded
-    // columns of one slab, of which a_nv are real (i < w)
-    uint64_t a_base[A_PER];
-    bool a_ok[A_PER];
-    int a_row[A_PER], a_col[A_PER], a_nv[A_PER];
+    // Per-thread places of the vectors within the tile and the fixed part of
+    // the A addresses; NN vectors are VEC padded columns of one slab, of which
+    // a_nv are real (i < w).
+    struct Place
+    {
+        uint64_t a_base[A_PER];
+        bool a_ok[A_PER];
+        int a_row[A_PER], a_col[A_PER], a_nv[A_PER];
+        int b_row[B_PER], b_col[B_PER];
+        bool b_in[B_PER];
+    };
+    auto place = [&](int t) {
+        Place g;
 #pragma unroll
-    for (int e = 0; e < A_PER; ++e) {
-        int const v = tid + 256 * e;
-        a_ok[e] = v < A_VECS;
-        a_nv[e] = VEC;
-        if constexpr (!TN) {
-            a_row[e] = v / (BN / VEC);
-            a_col[e] = (v % (BN / VEC)) * VEC;
-            uint64_t const n = n0 + a_col[e];
-            a_ok[e] = a_ok[e] && n < ncols;
-            if constexpr (PAD) {
-                uint64_t const k = a_ok[e] ? n / wp : 0;
-                uint64_t const i = a_ok[e] ? n - k * wp : 0;
-                a_ok[e] = a_ok[e] && i < w;
-                a_nv[e] = a_ok[e] ? (int)(w - i < (uint64_t)VEC ? w - i : VEC) : 0;
-                a_base[e] = a_ok[e] ? k * ld * w + i : 0;
+        for (int e = 0; e < A_PER; ++e) {
+            int const v = t + 256 * e;
+            g.a_ok[e] = v < A_VECS;
+            g.a_nv[e] = VEC;
+            if constexpr (!TN) {
+                g.a_row[e] = v / (BN / VEC);
+                g.a_col[e] = (v % (BN / VEC)) * VEC;
+                uint64_t const n = n0 + g.a_col[e];
+                g.a_ok[e] = g.a_ok[e] && n < ncols;
+                if constexpr (PAD) {
+                    uint64_t const k = g.a_ok[e] ? n / wp : 0;
+                    uint64_t const i = g.a_ok[e] ? n - k * wp : 0;
+                    g.a_ok[e] = g.a_ok[e] && i < w;
+                    g.a_nv[e] = g.a_ok[e] ? (int)(w - i < (uint64_t)VEC ? w - i : VEC) : 0;
+                    g.a_base[e] = g.a_ok[e] ? k * ld * w + i : 0;
+                } else {
+                    uint64_t const k = g.a_ok[e] ? n / w : 0;
+                    g.a_base[e] = k * ld * w + (g.a_ok[e] ? n - k * w : 0);
+                }
             } else {
-                uint64_t const k = a_ok[e] ? n / w : 0;
-                a_base[e] = k * ld * w + (a_ok[e] ? n - k * w : 0);
+                g.a_col[e] = v / (BK / VEC);         // column n within the tile
+                g.a_row[e] = (v % (BK / VEC)) * VEC; // first l within the slice
+                uint64_t const n = n0 + g.a_col[e];
+                g.a_ok[e] = g.a_ok[e] && n < ncols;
+                g.a_base[e] = g.a_ok[e] ? n * ld : 0;
             }
-        } else {
-            a_col[e] = v / (BK / VEC);          // column n within the tile
-            a_row[e] = (v % (BK / VEC)) * VEC;  // first l within the slice
-            uint64_t const n = n0 + a_col[e];
-            a_ok[e] = a_ok[e] && n < ncols;
-            a_base[e] = a_ok[e] ? n * ld : 0;
         }
-    }
-    int b_row[B_PER], b_col[B_PER];
-    bool b_in[B_PER];
 #pragma unroll
-    for (int e = 0; e < B_PER; ++e) {
-        int const v = tid + 256 * e;
-        b_in[e] = v < B_VECS;
-        if constexpr (BCOL) {
-            b_row[e] = v / (BM / VEC);
-            b_col[e] = (v % (BM / VEC)) * VEC;
-        } else {
-            b_col[e] = v / (BK / VEC);
-            b_row[e] = (v % (BK / VEC)) * VEC;
+        for (int e = 0; e < B_PER; ++e) {
+            int const v = t + 256 * e;
+            g.b_in[e] = v < B_VECS;
+            if constexpr (BCOL) {
+                g.b_row[e] = v / (BM / VEC);
+                g.b_col[e] = (v % (BM / VEC)) * VEC;
+            } else {
+                g.b_col[e] = v / (BK / VEC);
+                g.b_row[e] = (v % (BK / VEC)) * VEC;
+            }
         }
-    }
+        return g;
+    };
+    Place const pl = place(tid);
     bool const b_vec_ok = (flags & TILE_B_VEC) != 0 && (BCOL ? (m % VEC == 0) : (ld % VEC == 0));
 
     // Register sets of slices in flight: two for tiles of at most 32 rows per
@@ -319,25 +329,25 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
         if (!a_vec) {
             bool whole = n0 + BN <= ncols && rows_ok;
 #pragma unroll
-            for (int e = 0; e < A_PER; ++e) whole = whole && a_nv[e] == VEC;
+            for (int e = 0; e < A_PER; ++e) whole = whole && pl.a_nv[e] == VEC;
             full = __syncthreads_and(whole ? 1 : 0) != 0;
         }
     }
     uint64_t a_fix[A_PER]; // A offset of the thread's vector in slice 0
 #pragma unroll
-    for (int e = 0; e < A_PER; ++e) a_fix[e] = TN ? a_base[e] + a_row[e] : a_base[e] + (uint64_t)a_row[e] * w;
+    for (int e = 0; e < A_PER; ++e) a_fix[e] = TN ? pl.a_base[e] + pl.a_row[e] : pl.a_base[e] + (uint64_t)pl.a_row[e] * w;
     uint64_t const a_step = TN ? 1 : w; // A offset per contraction index
 
-    auto load_tiles = [&](uint64_t l0, auto set) {
+    auto load_tiles = [&](Place const &g, uint64_t l0, auto set) {
         constexpr int S = decltype(set)::value;
 #pragma unroll
         for (int e = 0; e < A_PER; ++e) {
             ra[S][e] = vzero<V>();
             ra_dm[S][e] = DM_WHOLE;
             if constexpr (!TN) {
-                uint64_t const l = l0 + a_row[e];
+                uint64_t const l = l0 + g.a_row[e];
                 if (!PAD || a_vec) {
-                    if (a_ok[e] && l < nq) ra[S][e] = load_a(a + a_base[e] + l * w);
+                    if (g.a_ok[e] && l < nq) ra[S][e] = load_a(a + g.a_base[e] + l * w);
                 } else {
                     // Branch-free: the VEC elements from the vector's first
                     // (element-aligned) address; rows of a slab are
@@ -350,12 +360,12 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                     // the read then starts before `a`, still inside A, which
                     // holds at least VEC elements)
                     uint64_t const lc = l < nq ? l : nq - 1;
-                    int64_t const addr = (int64_t)(a_base[e] + lc * w);
+                    int64_t const addr = (int64_t)(g.a_base[e] + lc * w);
                     int64_t const lim = (int64_t)a_len - VEC;
                     int64_t const ac = addr < lim ? addr : lim;
                     V const v = ldg<typename Gt::vec_u>(a + ac);
                     ra[S][e] = v;
-                    ra_dm[S][e] = (int)(addr - ac) | (l < nq ? a_nv[e] : 0) << 8;
+                    ra_dm[S][e] = (int)(addr - ac) | (l < nq ? g.a_nv[e] : 0) << 8;
                 }
             } else if (nq >= (uint64_t)VEC) {
                 // One in-bounds vector per thread and no divergent branch (a
@@ -364,28 +374,28 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                 // that would run past the row end is read as the row's last
                 // VEC elements and shifted into place; elements past the row
                 // end, and rows past the last column (read as row 0), are zero.
-                uint64_t const l = l0 + a_row[e];
+                uint64_t const l = l0 + g.a_row[e];
                 uint64_t const last = nq - VEC;
                 uint64_t const lc = l < last ? l : last;
-                V const v = ldg<typename Gt::vec_u>(a + a_base[e] + lc);
-                int const nvalid = (!a_ok[e] || l >= nq) ? 0 : (int)(nq - l < (uint64_t)VEC ? nq - l : VEC);
+                V const v = ldg<typename Gt::vec_u>(a + g.a_base[e] + lc);
+                int const nvalid = (!g.a_ok[e] || l >= nq) ? 0 : (int)(nq - l < (uint64_t)VEC ? nq - l : VEC);
                 ra[S][e] = v;
                 ra_dm[S][e] = (int)(l - lc) | nvalid << 8;
             } else {
-                uint64_t const l = l0 + a_row[e];
-                if (a_ok[e] && l < nq) {
+                uint64_t const l = l0 + g.a_row[e];
+                if (g.a_ok[e] && l < nq) {
                     if (a_vec) {
                         // nq % VEC == 0: a vector is wholly in or out of range
-                        ra[S][e] = load_a(a + a_base[e] + l);
+                        ra[S][e] = load_a(a + g.a_base[e] + l);
                     } else if (l + VEC <= nq) {
                         // element-aligned vector inside the row
-                        V const v = ldg<typename Gt::vec_u>(a + a_base[e] + l);
+                        V const v = ldg<typename Gt::vec_u>(a + g.a_base[e] + l);
                         ra[S][e] = v;
                     } else {
                         // the row's last, partial vector
 #pragma unroll
                         for (int x = 0; x < VEC; ++x)
-                            if (l + x < nq) ra[S][e][x] = ldg<T>(a + a_base[e] + l + x);
+                            if (l + x < nq) ra[S][e][x] = ldg<T>(a + g.a_base[e] + l + x);
                     }
                 }
             }
@@ -394,10 +404,10 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
         for (int e = 0; e < B_PER; ++e) {
             rb[S][e] = vzero<V>();
             rb_dm[S][e] = DM_WHOLE;
-            if (!b_in[e]) continue;
+            if (!g.b_in[e]) continue;
             if constexpr (BCOL) {
-                uint64_t const l = l0 + b_row[e];
-                uint64_t const j = j0 + b_col[e];
+                uint64_t const l = l0 + g.b_row[e];
+                uint64_t const j = j0 + g.b_col[e];
                 if (l < nq) {
                     if (j + VEC <= m) {
                         // element-aligned vector inside column l (16-byte aligned when m % VEC == 0)
@@ -412,9 +422,9 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
             } else if (nq >= (uint64_t)VEC) {
                 // as the TN rows of A; rows past m read row m - 1 (their
                 // products are never stored)
-                uint64_t const j = j0 + b_col[e];
+                uint64_t const j = j0 + g.b_col[e];
                 uint64_t const jc = j < m ? j : m - 1;
-                uint64_t const l = l0 + b_row[e];
+                uint64_t const l = l0 + g.b_row[e];
                 uint64_t const last = nq - VEC;
                 uint64_t const lc = l < last ? l : last;
                 V const v = ldg<typename Gt::vec_u>(b + jc * ld + lc);
@@ -422,8 +432,8 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                 rb[S][e] = v;
                 rb_dm[S][e] = (int)(l - lc) | nvalid << 8;
             } else {
-                uint64_t const j = j0 + b_col[e];
-                uint64_t const l = l0 + b_row[e];
+                uint64_t const j = j0 + g.b_col[e];
+                uint64_t const l = l0 + g.b_row[e];
                 if (j < m) {
                     if (l + VEC <= nq) {
                         // element-aligned vector inside row j (16-byte aligned when ld % VEC == 0)
@@ -445,6 +455,15 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     // vectors past B_VECS (BM * BK < 256 * VEC) re-read the tile's first
     // vector, B(j0, l0), which is in range, and are not stored.
     static_assert(A_VECS % 256 == 0, "every thread loads whole A vectors");
+    uint64_t b_fix[B_PER]; // B offset of the thread's vector in slice 0
+#pragma unroll
+    for (int e = 0; e < B_PER; ++e) {
+        uint64_t const jj = pl.b_in[e] ? (uint64_t)pl.b_col[e] : 0;
+        uint64_t const ll = pl.b_in[e] ? (uint64_t)pl.b_row[e] : 0;
+        uint64_t const j = j0 + jj;
+        b_fix[e] = BCOL ? (j + VEC <= m ? j : m - VEC) + ll * m : (j < m ? j : m - 1) * ld + ll;
+    }
+    uint64_t const b_step = BCOL ? m : 1; // B offset per contraction index
     auto load_full = [&](uint64_t l0, auto set) {
         constexpr int S = decltype(set)::value;
 #pragma unroll
@@ -467,13 +486,40 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
         }
 #pragma unroll
         for (int e = 0; e < B_PER; ++e) {
-            uint64_t const jj = b_in[e] ? (uint64_t)b_col[e] : 0;
-            uint64_t const ll = b_in[e] ? (uint64_t)b_row[e] : 0;
-            uint64_t const j = j0 + jj;
-            T const *bp = BCOL ? b + (j + VEC <= m ? j : m - VEC) + (l0 + ll) * m
-                               : b + (j < m ? j : m - 1) * ld + l0 + ll;
+            T const *bp = b + b_fix[e] + l0 * b_step;
             if (VIEW == VIEW_TT || b_vec_ok) rb[S][e] = ldg<V>(bp);
             else rb[S][e] = ldg<typename Gt::vec_u>(bp);
+        }
+    };
+    // The ragged last slice of an interior tile (nq % BK != 0, at least one
+    // whole slice before it): the same vectors read at in-range addresses,
+    // with the shift and the count of valid elements kept for the store.
+    // Vectors along n (or j) are whole or past the last index; vectors along
+    // l are moved back to the row's last VEC elements.
+    auto load_ragged = [&](uint64_t l0, auto set) {
+        constexpr int S = decltype(set)::value;
+        using VU = typename Gt::vec_u;
+        auto along_l = [&](const T *row, uint64_t l, V &v, int &dm) {
+            uint64_t const lc = l < nq - VEC ? l : nq - VEC;
+            v = ldg<VU>(row + lc);
+            int const nvalid = l >= nq ? 0 : (int)(nq - l < (uint64_t)VEC ? nq - l : VEC);
+            dm = (int)(l - lc) | nvalid << 8;
+        };
+        auto across_l = [&](const T *col, uint64_t l, uint64_t step, V &v, int &dm) {
+            v = ldg<VU>(col + (l < nq ? l : nq - 1) * step);
+            dm = l < nq ? DM_WHOLE : 0;
+        };
+#pragma unroll
+        for (int e = 0; e < A_PER; ++e) {
+            uint64_t const l = l0 + pl.a_row[e];
+            if constexpr (TN) along_l(a + a_fix[e] - pl.a_row[e], l, ra[S][e], ra_dm[S][e]);
+            else across_l(a + a_fix[e] - (uint64_t)pl.a_row[e] * w, l, w, ra[S][e], ra_dm[S][e]);
+        }
+#pragma unroll
+        for (int e = 0; e < B_PER; ++e) {
+            uint64_t const ll = pl.b_in[e] ? (uint64_t)pl.b_row[e] : 0;
+            if constexpr (BCOL) across_l(b + b_fix[e] - ll * m, l0 + ll, m, rb[S][e], rb_dm[S][e]);
+            else along_l(b + b_fix[e] - ll, l0 + ll, rb[S][e], rb_dm[S][e]);
         }
     };
 
@@ -485,35 +531,33 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     // are conflict-free (32- and 64-bank models; 4-way for BK = 32 without it),
     // the double stores 2-way as before, the fragment reads unchanged.
     auto tn_swz = [](int l) { return NT * (((l >> 3) * 3) & 3); };
-    // full_tag false: the slice came from load_tiles (shift and mask the TN
-    // rows of A and the rows of a row-major B here).
-    auto store_tiles = [&](int buf, auto set, auto full_tag) {
+    // full_tag false: the slice came from load_tiles or load_ragged (shift and
+    // mask the vectors here).
+    auto store_tiles = [&](Place const &g, int buf, auto set, auto full_tag) {
         constexpr int S = decltype(set)::value;
         constexpr bool GUARDED = !decltype(full_tag)::value;
 #pragma unroll
         for (int e = 0; e < A_PER; ++e) {
-            if (tid + 256 * e >= A_VECS) continue;
             if constexpr (!TN) {
-                V const v = (PAD && GUARDED && !a_vec)
-                                ? shift_mask(ra[S][e], ra_dm[S][e] & 0xff, ra_dm[S][e] >> 8)
-                                : ra[S][e];
-                *reinterpret_cast<V *>(&sA[buf][a_row[e] * LDA + a_col[e]]) = v;
+                V const v = GUARDED ? shift_mask(ra[S][e], ra_dm[S][e] & 0xff, ra_dm[S][e] >> 8) : ra[S][e];
+                *reinterpret_cast<V *>(&sA[buf][g.a_row[e] * LDA + g.a_col[e]]) = v;
             } else {
                 V const v = GUARDED ? shift_mask(ra[S][e], ra_dm[S][e] & 0xff, ra_dm[S][e] >> 8) : ra[S][e];
 #pragma unroll
                 for (int x = 0; x < VEC; ++x)
-                    sA[buf][(a_row[e] + x) * LDA + (a_col[e] ^ tn_swz(a_row[e] + x))] = v[x];
+                    sA[buf][(g.a_row[e] + x) * LDA + (g.a_col[e] ^ tn_swz(g.a_row[e] + x))] = v[x];
             }
         }
 #pragma unroll
         for (int e = 0; e < B_PER; ++e) {
-            if (!b_in[e]) continue;
+            if (B_VECS % 256 != 0 && !g.b_in[e]) continue;
             if constexpr (BCOL) {
-                *reinterpret_cast<V *>(&sB[buf][b_row[e] * LDB + b_col[e]]) = rb[S][e];
+                V const v = GUARDED ? shift_mask(rb[S][e], rb_dm[S][e] & 0xff, rb_dm[S][e] >> 8) : rb[S][e];
+                *reinterpret_cast<V *>(&sB[buf][g.b_row[e] * LDB + g.b_col[e]]) = v;
             } else {
                 V const v = GUARDED ? shift_mask(rb[S][e], rb_dm[S][e] & 0xff, rb_dm[S][e] >> 8) : rb[S][e];
 #pragma unroll
-                for (int x = 0; x < VEC; ++x) sB[buf][(b_row[e] + x) * LDB + b_col[e]] = v[x];
+                for (int x = 0; x < VEC; ++x) sB[buf][(g.b_row[e] + x) * LDB + g.b_col[e]] = v[x];
             }
         }
     };
@@ -546,23 +590,23 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     using I1 = std::integral_constant<int, PF - 1>;
     // Slices [sb, se) of the contraction; starts and ends with all waves
     // synchronised and both LDS buffers free.
-    auto kloop = [&](auto full_tag, uint64_t sb, uint64_t se) {
+    auto kloop = [&](Place const &g, auto full_tag, uint64_t sb, uint64_t se) {
         constexpr bool FULL = decltype(full_tag)::value;
         auto load = [&](uint64_t s, auto set) {
             if constexpr (FULL) load_full(s * BK, set);
-            else load_tiles(s * BK, set);
+            else load_tiles(g, s * BK, set);
         };
         uint64_t const n = se - sb;
         if constexpr (PF == 1) {
             load(sb, I0());
-            store_tiles(0, I0(), full_tag);
+            store_tiles(g, 0, I0(), full_tag);
             __syncthreads();
             for (uint64_t s = 0; s < n; ++s) {
                 int const buf = (int)(s & 1);
                 bool const more = s + 1 < n;
                 if (more) load(sb + s + 1, I0());
                 multiply(buf);
-                if (more) store_tiles(buf ^ 1, I0(), full_tag);
+                if (more) store_tiles(g, buf ^ 1, I0(), full_tag);
                 __syncthreads();
             }
         } else {
@@ -571,31 +615,151 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
             // buffer only after the barrier that ended its slice's products.
             load(sb, I0());
             if (n > 1) load(sb + 1, I1());
-            store_tiles(0, I0(), full_tag);
+            store_tiles(g, 0, I0(), full_tag);
             __syncthreads();
             for (uint64_t s = 0; s < n; s += 2) {
                 if (s + 2 < n) load(sb + s + 2, I0());
                 multiply(0);
-                if (s + 1 < n) store_tiles(1, I1(), full_tag);
+                if (s + 1 < n) store_tiles(g, 1, I1(), full_tag);
                 __syncthreads();
                 if (s + 1 < n) {
                     if (s + 3 < n) load(sb + s + 3, I1());
                     multiply(1);
-                    if (s + 2 < n) store_tiles(0, I0(), full_tag);
+                    if (s + 2 < n) store_tiles(g, 0, I0(), full_tag);
                     __syncthreads();
                 }
+            }
+        }
+    };
+    // PIPE: the slices of an interior tile with every wait off the matrix
+    // cores' path.  The plain loop above waits for LDS at the head of each
+    // group of MFMAs and stores a slice in one burst; the two waves of a SIMD
+    // run their groups in step, so both wait at once (matrix cores busy 84 %
+    // of the cycles in the 128 x 128 tiles).  Here the fragments of step
+    // kk + 1 are read while step kk multiplies (two register sets), the stores
+    // of slice s + 1 and the loads of slice s + 1 + PF go one by one between
+    // the MFMAs of the last two steps, and the barrier and the first fragments
+    // of the next slice come in the middle of the last step.  A 1024x1024x512,
+    // m = 1024: float64 16.85 -> 14.87 ms (q = 2) and 17.1 -> 15.05 ms (q = 1),
+    // float32 8.37 -> 7.55 ms and 8.30 -> 7.53 ms (0.92-0.94 of the matrix
+    // peak); bursts of loads and stores between whole steps measured 15.8 /
+    // 16.1 / 8.05 / 8.06 ms, loads three steps earlier 8.0-8.3 ms in float32.
+    // A wave passes the barrier of slice s after its last fragment of buffer
+    // s & 1 has arrived (the wait counts reads too) and its part of slice
+    // s + 1 is stored; buffer s & 1 is overwritten only in slice s + 1, behind
+    // that barrier.
+    auto lds_barrier = [&]() {
+        __builtin_amdgcn_s_waitcnt(0xC07F); // lgkmcnt(0): vector-memory loads stay in flight
+        asm volatile("s_barrier" ::: "memory");
+    };
+    T fa[2][JT], fb[2][NT];
+    auto fragments = [&](int buf, int kk, int set) {
+        int const kr = kk * 4 + lr;
+        lds_read<T, JT>(&sB[buf][kr * LDB + b_off], fa[set]);
+        lds_read<T, NT>(&sA[buf][kr * LDA + (TN ? (a_off ^ tn_swz(kr)) : a_off)], fb[set]);
+    };
+    auto products = [&](int set, int jt0, int jt1) {
+#pragma unroll
+        for (int jt = jt0; jt < jt1; ++jt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[jt][nt] = Gt::mfma(fa[set][jt], fb[set][nt], acc[jt][nt]);
+    };
+    // Slice s (in LDS buffer BUF, its first fragments in set 0).  LOAD: load
+    // slice s + 1 + PF into the registers that the store of slice s + 1 frees;
+    // TAIL: near the end, where a slice may be the ragged one or not exist.
+    uint64_t const nwhole = nq / BK;
+    auto slice = [&](auto buf_tag, auto tail_tag, uint64_t s) {
+        constexpr int BUF = decltype(buf_tag)::value;
+        constexpr bool TAIL = decltype(tail_tag)::value;
+        constexpr int STEPS = BK / 4;
+        static_assert(STEPS % 2 == 0 && STEPS >= 4, "set 0 is free at the end of a slice");
+        using Set = std::integral_constant<int, PF == 2 ? BUF ^ 1 : 0>;
+        constexpr int JH = (JT + 1) / 2; // row tiles ahead of the barrier in the last step
+        bool const more = !TAIL || s + 1 < nslices;
+#pragma unroll
+        for (int kk = 0; kk < STEPS; ++kk) {
+            bool const last = kk + 1 == STEPS;
+            if (!last) fragments(BUF, kk + 1, (kk + 1) & 1);
+            if (kk + 2 == STEPS && more) {
+                if (TAIL && s + 1 == nwhole) store_tiles(pl, BUF ^ 1, Set(), std::false_type());
+                else store_tiles(pl, BUF ^ 1, Set(), std::true_type());
+            }
+            if (last) {
+                uint64_t const t = s + 1 + PF;
+                if (!TAIL || t < nwhole) load_full(t * BK, Set());
+                else if (t < nslices) load_ragged(t * BK, Set());
+            }
+            products(kk & 1, 0, last ? JH : JT);
+            // one memory instruction after each MFMA
+            if constexpr (!TAIL) {
+#pragma unroll
+                for (int i = 0; i < (last ? JH : JT) * NT; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                // MFMA
+                    if (!last) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);     // LDS read
+                    if (kk + 2 == STEPS) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0); // LDS write
+                    if (last) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);      // global load
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (more) {
+            lds_barrier();
+            fragments(BUF ^ 1, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        products((STEPS - 1) & 1, JH, JT);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto kloop_pipe = [&]() {
+        using B0 = std::integral_constant<int, 0>;
+        using B1 = std::integral_constant<int, 1>;
+        auto load = [&](uint64_t t, auto set) {
+            if (t < nwhole) load_full(t * BK, set);
+            else if (t < nslices) load_ragged(t * BK, set);
+        };
+        load_full(0, I0());
+        if constexpr (PF == 2) load(1, I1());
+        store_tiles(pl, 0, I0(), std::true_type());
+        load(PF, I0());
+        lds_barrier();
+        fragments(0, 0, 0);
+        uint64_t s = 0;
+        for (; s + 2 + PF < nwhole; s += 2) {
+            slice(B0(), std::false_type(), s);
+            slice(B1(), std::false_type(), s + 1);
+        }
+        if constexpr (PF == 2) {
+            for (; s < nslices; s += 2) {
+                slice(B0(), std::true_type(), s);
+                if (s + 1 < nslices) slice(B1(), std::true_type(), s + 1);
+            }
+        } else {
+            // rolled: the large tiles have no registers to spare for copies
+            for (; s < nslices; ++s) {
+                int const buf = (int)(s & 1);
+                bool const more = s + 1 < nslices;
+                multiply(buf);
+                if (more) {
+                    if (s + 1 == nwhole) store_tiles(pl, buf ^ 1, I0(), std::false_type());
+                    else store_tiles(pl, buf ^ 1, I0(), std::true_type());
+                    load(s + 2, I0());
+                }
+                lds_barrier();
             }
         }
     };
     if constexpr (VIEW == VIEW_TT) {
         // grouped chain stages (contractions of 16..256): one loop per tile,
         // unguarded only when every slice is whole
-        if (full && nq % BK == 0) kloop(std::true_type(), 0, nslices);
-        else kloop(std::false_type(), 0, nslices);
+        if (full && nq % BK == 0) kloop(pl, std::true_type(), 0, nslices);
+        else kloop(pl, std::false_type(), 0, nslices);
+    } else if constexpr (PIPE) {
+        if (full && nwhole > 0) kloop_pipe();
+        else kloop(pl, std::false_type(), 0, nslices);
     } else {
-        uint64_t const nwhole = full ? nq / BK : 0; // slices with unguarded loads
-        if (nwhole > 0) kloop(std::true_type(), 0, nwhole);
-        if (nwhole < nslices) kloop(std::false_type(), nwhole, nslices);
+        uint64_t const n = full ? nwhole : 0; // slices with unguarded loads
+        if (n > 0) kloop(pl, std::true_type(), 0, n);
+        if (n < nslices) kloop(pl, std::false_type(), n, nslices);
     }
 
     // ---- epilogue ---------------------------------------------------------
@@ -689,7 +853,7 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
 // the contraction and writes its partial product, in C's layout, at
 // c + s * c_split (the partials are summed by k_sum_splits); with one split
 // the block writes C itself.
-template <class T, int JT, int NT, int WAVES_M, int BK, bool TN, bool BCOL, bool PAD = false>
+template <class T, bool PIPE, int JT, int NT, int WAVES_M, int BK, bool TN, bool BCOL, bool PAD>
 __global__ __launch_bounds__(256, 2) void k_gemm(const T *__restrict__ a, const T *__restrict__ b,
                                               T *__restrict__ c, uint64_t ncols, uint64_t nq, uint64_t w,
                                               uint64_t wp, uint64_t m, unsigned nj, unsigned total, uint64_t kc,
@@ -704,7 +868,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm(const T *__restrict__ a, const 
     uint64_t const len = nq - l0 < kc ? nq - l0 : kc;
     // elements of A from the split's first row to the end of A (PAD reads)
     uint64_t const a_len = TN ? 0 : (ncols / wp) * nq * w - l0 * w;
-    gemm_tile<T, JT, NT, WAVES_M, BK, TN ? VIEW_TN : VIEW_NN, BCOL, PAD>(
+    gemm_tile<T, JT, NT, WAVES_M, BK, TN ? VIEW_TN : VIEW_NN, BCOL, PAD, PIPE>(
         a + l0 * (TN ? 1 : w), b + l0 * (BCOL ? m : 1), c + (uint64_t)blockIdx.y * c_split, ncols, len, nq, w, wp,
         m, (uint64_t)jb * S::BM, (uint64_t)nb * S::BN, flags, a_len, sA, sB);
 }
@@ -899,21 +1063,37 @@ Split split_for(const Fold &f, bool is_double, const Geom &g, unsigned want)
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// Blocks whose contraction (of one split) has at least this many indices take
+// the pipelined loop; its start and its last slices cost more than the plain
+// loop's.  Measured against the plain loop on [n, K, n] x_2 with n = 512:
+// float32 128-row blocks 1.04x at K = 96 and 0.97x at 64; 32- and 48-row
+// blocks 1.03x at 256 and 0.98x at 128; float64 128-row blocks 1.03x at 512,
+// 0.99-1.02x at 256 and 0.92x at 128 (256 registers, some spilled outside
+// the loop), 16- and 50-row blocks 1.07x at 515 and 0.99x at 255.
+bool gemm_pipelined(const Config &cfg, bool is_double, uint64_t len)
+{
+    return len >= (is_double ? 384u : cfg.waves_m == 2 ? 96u : 192u);
+}
+
 template <class T, int JT, int NT, int WM, int BK, bool TN, bool BCOL>
 void launch_cfg(const Fold &f, const Geom &g, const Split &sp, unsigned flags, const T *a, const T *b, T *c,
                 hipStream_t s)
 {
     unsigned const total = g.nj * g.nn;
     uint64_t const c_split = sp.splits > 1 ? f.numel_c() : 0;
-    if constexpr (!TN) {
-        if (g.pad) {
-            hipLaunchKernelGGL((k_gemm<T, JT, NT, WM, BK, TN, BCOL, true>), dim3(total, sp.splits), dim3(256), 0, s,
-                               a, b, c, g.ncols, f.nq, f.w, g.wp, f.m, g.nj, total, sp.kc, c_split, flags);
-            return;
-        }
+    auto run = [&](auto pad, auto pipe) {
+        hipLaunchKernelGGL((k_gemm<T, decltype(pipe)::value, JT, NT, WM, BK, TN, BCOL, decltype(pad)::value>),
+                           dim3(total, sp.splits), dim3(256), 0, s, a, b, c, g.ncols, f.nq, f.w, g.wp, f.m, g.nj,
+                           total, sp.kc, c_split, flags);
+    };
+    bool const pipe = gemm_pipelined(g.cfg, sizeof(T) == 8, sp.kc);
+    using Y = std::true_type;
+    using N = std::false_type;
+    if (!TN && g.pad) {
+        if constexpr (!TN) pipe ? run(Y(), Y()) : run(Y(), N());
+    } else {
+        pipe ? run(N(), Y()) : run(N(), N());
     }
-    hipLaunchKernelGGL((k_gemm<T, JT, NT, WM, BK, TN, BCOL>), dim3(total, sp.splits), dim3(256), 0, s, a, b, c,
-                       g.ncols, f.nq, f.w, g.wp, f.m, g.nj, total, sp.kc, c_split, flags);
 }
 
 template <class T, bool TN, bool BCOL>
@@ -954,8 +1134,9 @@ std::string gemm_symbol(const Fold &f, bool is_double, bool aligned)
     uint64_t const vec = is_double ? 2 : 4;
     bool const pad = f.w != 1 && (!aligned || f.w % vec != 0);
     char buf[128];
-    std::snprintf(buf, sizeof buf, "k_gemm<%s, %d, %d, %d, %d, %s, %s, %s>", is_double ? "double" : "float", cfg.jt,
-                  cfg.nt, cfg.waves_m, cfg.bk, f.w == 1 ? "true" : "false", f.b_colmajor ? "true" : "false",
+    std::snprintf(buf, sizeof buf, "k_gemm<%s, %s, %d, %d, %d, %d, %s, %s, %s>", is_double ? "double" : "float",
+                  gemm_pipelined(cfg, is_double, split_for(f, is_double, geom(f, is_double), 0).kc) ? "true" : "false",
+                  cfg.jt, cfg.nt, cfg.waves_m, cfg.bk, f.w == 1 ? "true" : "false", f.b_colmajor ? "true" : "false",
                   pad ? "true" : "false");
     return buf;
 }
