@@ -753,8 +753,8 @@ std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision
     }
     case Kernel::gemm: return gemm_symbol(f, is_double, aligned);
     case Kernel::skinny: return skinny_symbol(f, is_double);
-    case Kernel::lowp: return lowp_symbol(f, prec, false);
-    case Kernel::lowp_generic: return lowp_symbol(f, prec, true);
+    case Kernel::lowp: return lowp_symbol(f, prec, false, aligned);
+    case Kernel::lowp_generic: return lowp_symbol(f, prec, true, aligned);
     default: return "";
     }
 }
@@ -771,7 +771,7 @@ Kernel choose_kernel(const Fold &f, bool is_double, ttm_precision_t prec, bool a
 {
     if (prec != TTM_PREC_DEFAULT) {
         if (is_double || prec > TTM_PREC_FP16X2) return Kernel::none;
-        bool const lp_ok = lowp_supports(f, aligned);
+        bool const lp_ok = lowp_supports(f, aligned) || lowp_any_supports(f, prec);
         if (force == Kernel::generic || force == Kernel::lowp_generic || !lp_ok) return Kernel::lowp_generic;
         return Kernel::lowp;
     }
@@ -817,6 +817,19 @@ unsigned launch_splits(Kernel k, const Fold &f, bool is_double, unsigned want)
     return k == Kernel::gemm ? gemm_split(f, is_double, want).splits : skinny_splits(f, is_double, want);
 }
 
+namespace
+{
+bool stream_capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+} // namespace
+
 ttm_status_t launch_f32(const Fold &f, const float *a, const float *b, float *c, ttm_precision_t prec,
                         hipStream_t stream, Kernel force, LaunchInfo *info, unsigned want_splits)
 {
@@ -832,8 +845,18 @@ ttm_status_t launch_f32(const Fold &f, const float *a, const float *b, float *c,
     }
     bool const ac_aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(c)) & 15u) == 0;
     if (k == Kernel::lowp || k == Kernel::lowp_generic) {
-        if (info) *info = LaunchInfo{k, 1, ac_aligned};
-        return launch_lowp(f, a, b, c, prec, stream, k == Kernel::lowp_generic);
+        bool generic = k == Kernel::lowp_generic;
+        // without room for the converted operands, or while the stream is
+        // captured (no allocation there): one thread per element
+        bool const any = !generic && !lowp_supports(f, aligned);
+        if (any && (!lowp_any_fits(f, prec) || (!scratch_bound() && stream_capturing(stream)))) generic = true;
+        ttm_status_t st = launch_lowp(f, a, b, c, prec, stream, generic);
+        if (any && !generic && st == TTM_ERR_ALLOC) {
+            generic = true;
+            st = launch_lowp(f, a, b, c, prec, stream, true);
+        }
+        if (info) *info = LaunchInfo{generic ? Kernel::lowp_generic : Kernel::lowp, 1, aligned};
+        return st;
     }
     if (want_splits == 0) want_splits = tuned_splits(k, f, false);
     if (info) *info = LaunchInfo{k, launch_splits(k, f, false, want_splits), ac_aligned};

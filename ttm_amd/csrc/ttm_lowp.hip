@@ -806,16 +806,16 @@ __device__ __forceinline__ void lowp_tile(const float *__restrict__ a, const flo
 // product): plane p at bs + p * plane, row j at j * ldb, zero outside m x nq.
 // One thread per 8 consecutive l of a row.
 template <int MODE>
-__global__ __launch_bounds__(256) void k_lowp_split_b(const float *__restrict__ b, typename Lp<MODE>::op *__restrict__ bs,
-                                                      uint64_t m, uint64_t nq, uint64_t bsj, uint64_t bsl, uint64_t ldb,
-                                                      uint64_t rows, uint64_t plane, const int *__restrict__ exps)
+__device__ __forceinline__ void split_b_block(unsigned block, const float *__restrict__ b, typename Lp<MODE>::op *__restrict__ bs,
+                                              uint64_t m, uint64_t nq, uint64_t bsj, uint64_t bsl, uint64_t ldb,
+                                              uint64_t rows, uint64_t plane, int eb)
 {
     using L = Lp<MODE>;
     using v2 = typename L::v2;
     using v8 = typename L::v8;
     constexpr int P = L::PARTS;
     uint64_t const groups = ldb / 8;
-    uint64_t const idx = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    uint64_t const idx = (uint64_t)block * 256 + threadIdx.x;
     if (idx >= rows * groups) return;
     uint64_t const j = idx / groups, l0 = (idx - j * groups) * 8;
     v2 q[4][P];
@@ -827,7 +827,7 @@ __global__ __launch_bounds__(256) void k_lowp_split_b(const float *__restrict__ 
             uint64_t const l = l0 + 2 * t + e;
             x[e] = (j < m && l < nq) ? b[j * bsj + l * bsl] : 0.f;
         }
-        if constexpr (MODE == LP_FP16X2) x = scale2(x, exps[1]);
+        if constexpr (MODE == LP_FP16X2) x = scale2(x, eb);
         L::split2(x, q[t]);
     }
 #pragma unroll
@@ -836,6 +836,14 @@ __global__ __launch_bounds__(256) void k_lowp_split_b(const float *__restrict__ 
         auto const hi = __builtin_shufflevector(q[2][p], q[3][p], 0, 1, 2, 3);
         *reinterpret_cast<v8 *>(bs + p * plane + j * ldb + l0) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(256) void k_lowp_split_b(const float *__restrict__ b, typename Lp<MODE>::op *__restrict__ bs,
+                                                      uint64_t m, uint64_t nq, uint64_t bsj, uint64_t bsl, uint64_t ldb,
+                                                      uint64_t rows, uint64_t plane, const int *__restrict__ exps)
+{
+    split_b_block<MODE>(blockIdx.x, b, bs, m, nq, bsj, bsl, ldb, rows, plane, MODE == LP_FP16X2 ? exps[1] : 0);
 }
 
 // One product: a grid of BM x 128 blocks over the pre-converted B (BM = 64
@@ -961,6 +969,401 @@ __global__ __launch_bounds__(256, lp_group_blocks_per_cu(BM)) void k_lowp_groupe
 }
 
 // ---------------------------------------------------------------------------
+// Products over two pre-converted operands ("planes"): any extents and any
+// element-aligned buffers.
+//
+// A is converted once into P planes of `op` in the layout of B's planes --
+// column n of the fold as row n, contiguous along l, zero-padded to whole
+// tiles and slices -- so the product kernel moves only whole, aligned 16-byte
+// pieces by LDS DMA, whatever w, n_q and the base pointers are.  Bound by the
+// traffic of the passes: A [255, 301, 173] x_2, m = 120, FP16X2 1670 -> 75 us
+// (one thread per element before: serial chains of n_q loads), BF16X3
+// 1597 -> 81, BF16 1449 -> 44, FP8 2440 -> 56 us; of FP16X2's 68 us in
+// kernels the scale pass takes 15 (5.3 TB/s), the conversion 27 (4.4 TB/s)
+// and the product 23.
+// ---------------------------------------------------------------------------
+
+// A -> planes, TN view: rows of A are contiguous along l, in the order of the
+// planes.  One thread per 8 consecutive l of a row: two 16-byte loads at
+// element alignment, one 16-byte store per plane.
+template <int MODE>
+__device__ __forceinline__ void planes_a_rows(unsigned block, const float *__restrict__ a, typename Lp<MODE>::op *__restrict__ as,
+                                              uint64_t ncols, uint64_t nq, uint64_t ldk, uint64_t rows, uint64_t plane,
+                                              int ea)
+{
+    using L = Lp<MODE>;
+    using v2 = typename L::v2;
+    using v8 = typename L::v8;
+    constexpr int P = L::PARTS;
+    uint64_t const groups = ldk / 8;
+    uint64_t const idx = (uint64_t)block * 256 + threadIdx.x;
+    if (idx >= rows * groups) return;
+    uint64_t const n = idx / groups, l0 = (idx - n * groups) * 8;
+    f32x4 v[2] = {zero4(), zero4()};
+    if (n < ncols) {
+        const float *row = a + n * nq;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            uint64_t const l = l0 + 4 * h;
+            if (l + 4 <= nq) {
+                f32x4 const x = ldg<f32x4u>(row + l);
+                v[h] = x;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (l + e < nq) v[h][e] = ldg<float>(row + l + e);
+            }
+        }
+    }
+    v2 q[4][P];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        f32x2 x = {v[t >> 1][2 * (t & 1)], v[t >> 1][2 * (t & 1) + 1]};
+        if constexpr (MODE == LP_FP16X2) x = scale2(x, ea);
+        L::split2(x, q[t]);
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        auto const lo = __builtin_shufflevector(q[0][p], q[1][p], 0, 1, 2, 3);
+        auto const hi = __builtin_shufflevector(q[2][p], q[3][p], 0, 1, 2, 3);
+        stg<v8>(as + p * plane + n * ldk + l0, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+}
+
+// A -> planes, NN view: column n = k * w + i runs along l with stride w.  One
+// block per 64 columns x 64 l: lane = column, so a wave instruction reads 64
+// consecutive floats of one row l (256 bytes, any alignment, across slab
+// ends), 16 rows per thread in flight; the converted columns cross LDS and
+// leave as 128-byte row segments.  The columns' places cost one division per
+// thread.
+template <int MODE>
+__device__ __forceinline__ void planes_a_cols(unsigned block, const float *__restrict__ a, typename Lp<MODE>::op *__restrict__ as,
+                                              uint64_t ncols, uint64_t nq, uint64_t w, uint64_t ldk, uint64_t plane,
+                                              int ea)
+{
+    using L = Lp<MODE>;
+    using op = typename L::op;
+    using v2 = typename L::v2;
+    using v8 = typename L::v8;
+    constexpr int P = L::PARTS;
+    constexpr int LDT = 64 + 8; // elements per column in LDS (16-byte pieces spread over the banks)
+    __shared__ __attribute__((aligned(16))) op sT[P][64 * LDT];
+    unsigned const lblocks = (unsigned)(ldk / 64);
+    uint64_t const cb = block / lblocks, l0 = (uint64_t)(block % lblocks) * 64;
+    uint64_t const n0 = cb * 64;
+    int const tid = threadIdx.x, c = tid & 63, g = tid >> 6;
+    uint64_t const n = n0 + c;
+    bool const ok = n < ncols;
+    uint64_t const k = ok ? n / w : 0;
+    const float *col = a + k * nq * w + (ok ? n - k * w : 0);
+    float v[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        uint64_t const l = l0 + 16 * g + e;
+        v[e] = (ok && l < nq) ? ldg_nt<float>(col + l * w) : 0.f;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        v2 q[4][P];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x2 x = {v[8 * h + 2 * t], v[8 * h + 2 * t + 1]};
+            if constexpr (MODE == LP_FP16X2) x = scale2(x, ea);
+            L::split2(x, q[t]);
+        }
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            auto const lo = __builtin_shufflevector(q[0][p], q[1][p], 0, 1, 2, 3);
+            auto const hi = __builtin_shufflevector(q[2][p], q[3][p], 0, 1, 2, 3);
+            *reinterpret_cast<v8 *>(&sT[p][c * LDT + 16 * g + 8 * h]) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            int const r = (tid >> 3) + 32 * i, piece = tid & 7;
+            stg<v8>(as + p * plane + (n0 + r) * ldk + l0 + 8 * piece,
+                    *reinterpret_cast<const v8 *>(&sT[p][r * LDT + 8 * piece]));
+        }
+}
+
+// Both conversions in one launch: blocks [0, blocks_a) take A, the rest B.
+template <int MODE, bool TN>
+__global__ __launch_bounds__(256) void k_planes_convert(
+    const float *__restrict__ a, typename Lp<MODE>::op *__restrict__ as, uint64_t ncols, uint64_t w, uint64_t rows_a,
+    uint64_t plane_a, const float *__restrict__ b, typename Lp<MODE>::op *__restrict__ bs, uint64_t m, uint64_t bsj,
+    uint64_t bsl, uint64_t rows_b, uint64_t plane_b, uint64_t nq, uint64_t ldk, unsigned blocks_a,
+    const int *__restrict__ exps)
+{
+    int const ea = MODE == LP_FP16X2 ? exps[0] : 0, eb = MODE == LP_FP16X2 ? exps[1] : 0;
+    if (blockIdx.x >= blocks_a)
+        split_b_block<MODE>(blockIdx.x - blocks_a, b, bs, m, nq, bsj, bsl, ldk, rows_b, plane_b, eb);
+    else if constexpr (TN)
+        planes_a_rows<MODE>(blockIdx.x, a, as, ncols, nq, ldk, rows_a, plane_a, ea);
+    else
+        planes_a_cols<MODE>(blockIdx.x, a, as, ncols, nq, w, ldk, plane_a, ea);
+}
+
+// The product: WM x WN waves, each JT x NT MFMA tiles of 16 x 16; block
+// BM = 16 JT WM rows of B by BN = 16 NT WN columns of A; stages of KS slices
+// of 32 in two LDS buffers.  Planes are padded to whole blocks and stages, so
+// nothing in the loop is guarded.  LDS layout of a slice: lds_row / lds_swz,
+// filled by LDS DMA (a wave instruction moves the 1 KB of 16 physical rows;
+// see dma_b in lowp_tile for the lane order).
+//
+// Per stage: the next stage's DMA goes into the other buffer, fragments are
+// read one MFMA group ahead, and behind the last reads come the wait for that
+// DMA and the one barrier; the stage's last MFMA group runs behind it, while
+// the next stage's first fragments are read.
+template <int MODE, int WM, int WN, int JT, int NT, int KS>
+struct PlaneTile
+{
+    static constexpr int BM = 16 * JT * WM, BN = 16 * NT * WN, WAVES = WM * WN;
+    static constexpr int P = Lp<MODE>::PARTS;
+    static constexpr int LDS_BYTES = 2 * KS * P * (BM + BN) * LP_LDK * 2;
+    // blocks per CU: by LDS, at most 2 waves per SIMD of 256 registers for the
+    // 128 x 64 wave tiles, 4 of 128 registers otherwise
+    static constexpr int by_lds = 160 * 1024 / LDS_BYTES;
+    static constexpr int by_regs = (JT * NT >= 32 || P > 1 ? 8 : 16) / WAVES;
+    static constexpr int blocks = by_lds < by_regs ? by_lds : by_regs;
+    static constexpr int waves_per_simd = blocks * WAVES / 4 > 0 ? blocks * WAVES / 4 : 1;
+};
+
+template <int MODE, int WM, int WN, int JT, int NT, int KS, bool TSTORE>
+__global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>::waves_per_simd)) void k_planes(
+    const typename Lp<MODE>::op *__restrict__ as, uint64_t plane_a, const typename Lp<MODE>::op *__restrict__ bs,
+    uint64_t plane_b, uint64_t ldk, float *__restrict__ c, uint64_t ncols, uint64_t w, uint64_t m, unsigned nj,
+    unsigned total, int c_vec, const int *__restrict__ exps)
+{
+    using L = Lp<MODE>;
+    using op = typename L::op;
+    using v8 = typename L::v8;
+    using S = PlaneTile<MODE, WM, WN, JT, NT, KS>;
+    constexpr int P = L::PARTS, BM = S::BM, BN = S::BN, WAVES = S::WAVES;
+    static_assert(NT == 4 && JT % 4 == 0, "a lane's four column and row tiles are adjacent columns and rows");
+    __shared__ __attribute__((aligned(16))) op sA0[KS][P][BN * LP_LDK], sA1[KS][P][BN * LP_LDK];
+    __shared__ __attribute__((aligned(16))) op sB0[KS][P][BM * LP_LDK], sB1[KS][P][BM * LP_LDK];
+
+    unsigned jb, nb;
+    lp_block_coords(nj, total, jb, nb);
+    uint64_t const j0 = (uint64_t)jb * BM, n0 = (uint64_t)nb * BN;
+    int const tid = threadIdx.x, lane = tid & 63;
+    int const wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int const lc = lane & 15, lg = lane >> 4;
+    int const wm = wave % WM, wn = wave / WM;
+
+    // LDS DMA through buffer descriptors of the block's rows in each plane: as
+    // a buffer load it counts against the vector-memory counter alone (the
+    // global form also holds up every LDS wait).  Byte offsets within a
+    // block's rows stay below 2^32 (n_q < 2^22).
+    // Lane's offset within a piece of 16 physical rows: logical row 4 (lane / 4)
+    // past the piece's first, chunk (lane % 4) ^ swizzle.
+    uint32_t const ldk2 = (uint32_t)ldk * 2u;
+    uint32_t const lane_off = 4u * (uint32_t)(lane >> 2) * ldk2 + 16u * (uint32_t)((lane & 3) ^ lds_swz(lane >> 2));
+    // (the block's place comes out of a division in vector registers; a
+    // descriptor is scalar)
+    auto rows = [&](const op *base, uint32_t bytes) {
+        uint64_t const u = reinterpret_cast<uint64_t>(base);
+        uint64_t const lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u);
+        uint64_t const hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32));
+        return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(hi << 32 | lo), 0, bytes, 0x00027000);
+    };
+    __amdgpu_buffer_rsrc_t ra[P], rb[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        ra[p] = rows(as + p * plane_a + n0 * ldk, BN * ldk2);
+        rb[p] = rows(bs + p * plane_b + j0 * ldk, BM * ldk2);
+    }
+    auto dma = [&](uint32_t s, op (*sa)[P][BN * LP_LDK], op (*sb)[P][BM * LP_LDK]) {
+        auto piece = [&](__amdgpu_buffer_rsrc_t rs, uint32_t soff, op *dst) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (void __attribute__((address_space(3))) *)dst, 16, lane_off,
+                                                     soff, 0, 0);
+        };
+        constexpr int RA = BN / 16, RB = BM / 16; // pieces per slice and plane
+        static_assert(RA % WAVES == 0 && RB % WAVES == 0, "pieces divide over the waves");
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+                for (int i = 0; i < RA / WAVES; ++i) {
+                    uint32_t const r = (uint32_t)(wave + WAVES * i);
+                    piece(ra[p], (64u * (r >> 2) + (r & 3u)) * ldk2 + s * (64u * KS) + 64u * ks, &sa[ks][p][16 * r * LP_LDK]);
+                }
+#pragma unroll
+                for (int i = 0; i < RB / WAVES; ++i) {
+                    uint32_t const r = (uint32_t)(wave + WAVES * i);
+                    piece(rb[p], (64u * (r >> 2) + (r & 3u)) * ldk2 + s * (64u * KS) + 64u * ks, &sb[ks][p][16 * r * LP_LDK]);
+                }
+            }
+    };
+
+    f32x4 acc[JT][NT];
+#pragma unroll
+    for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[jt][nt] = zero4();
+
+    v8 fa[2][P][NT], fb[2][P];
+    int const arow = 16 * NT * wn + lc, brow = 16 * JT * wm + lc;
+    auto read_a = [&](int set, op (*sa)[P][BN * LP_LDK], int ks) {
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                fa[set][p][nt] = *reinterpret_cast<const v8 *>(&sa[ks][p][lds_at(arow + 16 * nt, lg)]);
+    };
+    auto read_b = [&](int set, op (*sb)[P][BM * LP_LDK], int ks, int jt) {
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            fb[set][p] = *reinterpret_cast<const v8 *>(&sb[ks][p][lds_at(brow + 16 * jt, lg)]);
+    };
+    auto products = [&](int sa, int sb, int jt) {
+        auto step = [&](int pb, int pa) {
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[jt][nt] = L::mfma(fb[sb][pb], fa[sa][pa][nt], acc[jt][nt]);
+        };
+        if constexpr (P == 3) {
+            step(1, 1);
+            step(0, 2);
+            step(2, 0);
+            step(0, 1);
+            step(1, 0);
+        } else if constexpr (P == 2) {
+            step(0, 1);
+            step(1, 0);
+        }
+        step(0, 0);
+    };
+    uint32_t const ns = (uint32_t)(ldk / (32 * KS));
+    // Fragments of slice ks of a stage in buffer BUF sit in set ks % 2 (KS
+    // even) or BUF; the last MFMA group of a stage runs behind the barrier,
+    // while the next stage's first fragments are read.
+    auto stage = [&](auto buf_tag, uint32_t s, op (*sa)[P][BN * LP_LDK], op (*sb)[P][BM * LP_LDK],
+                     op (*na)[P][BN * LP_LDK], op (*nb_)[P][BM * LP_LDK]) {
+        constexpr int BUF = decltype(buf_tag)::value;
+        constexpr int S0 = KS % 2 == 0 ? 0 : BUF; // set of the stage's first slice; the other holds the carry
+        if (s + 1 < ns) dma(s + 1, na, nb_);
+        read_a(S0, sa, 0);
+        read_b(0, sb, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        products(S0 ^ 1, 1, JT - 1); // carried over (zeros ahead of the first stage)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            int const set = KS % 2 == 0 ? ks & 1 : BUF;
+#pragma unroll
+            for (int jt = 0; jt < JT; ++jt) {
+                if (ks + 1 == KS && jt + 1 == JT) break;
+                if (jt + 1 < JT) {
+                    read_b((jt + 1) & 1, sb, ks, jt + 1);
+                } else {
+                    read_a(set ^ 1, sa, ks + 1);
+                    read_b(0, sb, ks + 1, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                products(set, jt & 1, jt);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0x0070); // vmcnt(0) lgkmcnt(0): the next stage is here, this one read
+        asm volatile("s_barrier" ::: "memory");
+    };
+    static_assert(JT % 2 == 0 && (KS == 1 || KS % 2 == 0), "fragment sets alternate");
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        fb[1][p] = v8{};
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) fa[1][p][nt] = v8{};
+    }
+    dma(0, sA0, sB0);
+    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
+    asm volatile("s_barrier" ::: "memory");
+    uint32_t s = 0;
+    for (; s + 1 < ns; s += 2) {
+        stage(std::integral_constant<int, 0>(), s, sA0, sB0, sA1, sB1);
+        stage(std::integral_constant<int, 1>(), s + 1, sA1, sB1, sA0, sB0);
+    }
+    if (s < ns) {
+        stage(std::integral_constant<int, 0>(), s, sA0, sB0, sA1, sB1);
+        products(KS % 2 == 0 ? 1 : 0, 1, JT - 1);
+    } else {
+        products(1, 1, JT - 1);
+    }
+    if constexpr (MODE == LP_FP16X2) {
+        int const ce = exps[0] + exps[1];
+#pragma unroll
+        for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[jt][nt][r] = ldexpf(acc[jt][nt][r], -ce);
+    }
+
+    // A lane holds, for row tile jt and element r, row 64 (jt / 4) + 4 (4 lg + r)
+    // + jt % 4 of its wave's rows and the four adjacent columns 4 lc + nt.
+    // c_vec: the vectors of C are 16-byte aligned, else they are element-aligned.
+    uint64_t const ncol0 = n0 + 16 * NT * wn + 4 * lc;
+    uint64_t const jw = j0 + 16 * JT * wm;
+    auto store4 = [&](float *p, f32x4 o) {
+        if (c_vec) stg<f32x4>(p, o);
+        else stg<f32x4u>(p, o);
+    };
+    if constexpr (!TSTORE) {
+        if (ncol0 >= ncols) return;
+        uint64_t const k = ncol0 / w, i = ncol0 - k * w;
+        bool const whole = i + 4 <= w; // one slab (then all four columns are in range)
+        float *cb = c + k * m * w + i;
+        uint64_t off[4]; // columns of the next slabs
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            uint64_t ii = i + nt, kk = 0;
+            while (ii >= w) {
+                ii -= w;
+                ++kk;
+            }
+            off[nt] = kk * m * w + ii - i;
+        }
+#pragma unroll
+        for (int jt = 0; jt < JT; ++jt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                uint64_t const j = jw + 64 * (jt >> 2) + 4 * (4 * lg + r) + (jt & 3);
+                if (j >= m) continue;
+                if (whole) {
+                    store4(cb + j * w, f32x4{acc[jt][0][r], acc[jt][1][r], acc[jt][2][r], acc[jt][3][r]});
+                } else {
+#pragma unroll
+                    for (int nt = 0; nt < 4; ++nt)
+                        if (ncol0 + nt < ncols) stg<float>(cb + j * w + off[nt], acc[jt][nt][r]);
+                }
+            }
+    } else {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            if (ncol0 + nt >= ncols) continue;
+            float *crow = c + (ncol0 + nt) * m;
+#pragma unroll
+            for (int g = 0; g < JT / 4; ++g)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    uint64_t const j = jw + 64 * g + 4 * (4 * lg + r);
+                    if (j + 4 <= m) {
+                        store4(crow + j, f32x4{acc[4 * g][nt][r], acc[4 * g + 1][nt][r], acc[4 * g + 2][nt][r],
+                                               acc[4 * g + 3][nt][r]});
+                    } else {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            if (j + t < m) stg<float>(crow + j + t, acc[4 * g + t][nt][r]);
+                    }
+                }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // FP8 e4m3fn with per-slice E8M0 scales: 64 x 64 blocks, K-slices of 128.
 // ---------------------------------------------------------------------------
 constexpr float FP8_MAX = 448.f;
@@ -1021,6 +1424,8 @@ struct Fp8Rows
     int e[8]; // the slice's exponent per step
 };
 
+// ANY: any n_q and element-aligned rows.
+template <bool ANY>
 __device__ __forceinline__ void fp8_rows_load(const float *__restrict__ x, uint64_t row0, uint64_t nrows, uint64_t nq,
                                               uint64_t l0, int tid, Fp8Rows &out)
 {
@@ -1031,7 +1436,19 @@ __device__ __forceinline__ void fp8_rows_load(const float *__restrict__ x, uint6
         int const c = (wave * 8 + i) * 8 + (lane >> 3);
         uint64_t const r = row0 + (c >> 2);
         uint64_t const l = l0 + 32 * (c & 3) + 4 * (lane & 7);
-        v[i] = (r < nrows && l < nq) ? *reinterpret_cast<const f32x4 *>(x + r * nq + l) : zero4();
+        if constexpr (ANY) {
+            v[i] = zero4();
+            if (r < nrows && l + 4 <= nq) {
+                f32x4 const t = ldg<f32x4u>(x + r * nq + l);
+                v[i] = t;
+            } else if (r < nrows) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (l + e < nq) v[i][e] = ldg<float>(x + r * nq + l + e);
+            }
+        } else {
+            v[i] = (r < nrows && l < nq) ? *reinterpret_cast<const f32x4 *>(x + r * nq + l) : zero4();
+        }
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -1078,6 +1495,7 @@ __global__ __launch_bounds__(256) void k_fp8_split_b(const float *__restrict__ b
 // of the fold as row n, padded to `rows` rows and ldq bytes), once per
 // product.  TN view: rows of A are contiguous along l; one 64 x 128 tile per
 // block, read 2 rows x 512 bytes per wave instruction (fp8_rows_load).
+template <bool ANY>
 __global__ __launch_bounds__(256) void k_fp8_split_a_rows(const float *__restrict__ a, unsigned char *__restrict__ qa,
                                                           unsigned char *__restrict__ sa, uint64_t ncols, uint64_t nq,
                                                           uint64_t ldq, uint64_t lblocks)
@@ -1086,7 +1504,7 @@ __global__ __launch_bounds__(256) void k_fp8_split_a_rows(const float *__restric
     uint64_t const row0 = rb * 64;
     int const tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     Fp8Rows r;
-    fp8_rows_load(a, row0, ncols, nq, l0, tid, r);
+    fp8_rows_load<ANY>(a, row0, ncols, nq, l0, tid, r);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         int const cix = (wave * 8 + i) * 8 + (lane >> 3);
@@ -1102,7 +1520,9 @@ __global__ __launch_bounds__(256) void k_fp8_split_a_rows(const float *__restric
 // columns share a slab and a 16-byte vector): the tile is read row by row in
 // 16-byte vectors (16 lanes per 256-byte row), transposed through LDS, and
 // quantized and written as in the TN view (eight lanes per 32-wide slice,
-// 2 columns x 128 bytes per wave instruction).
+// 2 columns x 128 bytes per wave instruction).  ANY (any w, element-aligned
+// A): a lane reads one column, 64 consecutive floats per wave instruction.
+template <bool ANY>
 __global__ __launch_bounds__(256) void k_fp8_split_a_cols(const float *__restrict__ a, unsigned char *__restrict__ qa,
                                                           unsigned char *__restrict__ sa, uint64_t ncols, uint64_t nq,
                                                           uint64_t w, uint64_t ldq, uint64_t lblocks)
@@ -1112,23 +1532,41 @@ __global__ __launch_bounds__(256) void k_fp8_split_a_cols(const float *__restric
     uint64_t const cb = blockIdx.x / lblocks, l0 = (blockIdx.x - cb * lblocks) * 128;
     uint64_t const n0 = cb * 64;
     int const tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // load: thread tid covers columns n0 + 4 (tid % 16) .. + 3 of rows l0 + tid / 16 + 16 i
-    int const cg = tid & 15;
-    uint64_t const n = n0 + 4 * cg;
-    bool const ok = n < ncols;
-    uint64_t const k = ok ? n / w : 0;
-    uint64_t const base = ok ? k * nq * w + (n - k * w) : 0;
-    f32x4 v[8];
+    if constexpr (ANY) {
+        int const col = lane;
+        uint64_t const n = n0 + col;
+        bool const ok = n < ncols;
+        uint64_t const k = ok ? n / w : 0;
+        const float *p = a + k * nq * w + (ok ? n - k * w : 0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        uint64_t const l = l0 + (tid >> 4) + 16 * i;
-        v[i] = (ok && l < nq) ? *reinterpret_cast<const f32x4 *>(a + base + l * w) : zero4();
-    }
+        for (int i = 0; i < 8; ++i) {
+            f32x4 v;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        int const lr = (tid >> 4) + 16 * i;
+            for (int e = 0; e < 4; ++e) {
+                uint64_t const l = l0 + 32 * wave + 4 * i + e;
+                v[e] = (ok && l < nq) ? ldg<float>(p + l * w) : 0.f;
+            }
+            *reinterpret_cast<f32x4 *>(&sT[col * LDT + 32 * wave + 4 * i]) = v;
+        }
+    } else {
+        // load: thread tid covers columns n0 + 4 (tid % 16) .. + 3 of rows l0 + tid / 16 + 16 i
+        int const cg = tid & 15;
+        uint64_t const n = n0 + 4 * cg;
+        bool const ok = n < ncols;
+        uint64_t const k = ok ? n / w : 0;
+        uint64_t const base = ok ? k * nq * w + (n - k * w) : 0;
+        f32x4 v[8];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sT[(4 * cg + e) * LDT + lr] = v[i][e];
+        for (int i = 0; i < 8; ++i) {
+            uint64_t const l = l0 + (tid >> 4) + 16 * i;
+            v[i] = (ok && l < nq) ? *reinterpret_cast<const f32x4 *>(a + base + l * w) : zero4();
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            int const lr = (tid >> 4) + 16 * i;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sT[(4 * cg + e) * LDT + lr] = v[i][e];
+        }
     }
     __syncthreads();
 #pragma unroll
@@ -1431,14 +1869,134 @@ ttm_status_t launch_lp(const Fold &f, const float *a, const float *b, float *c, 
     return TTM_SUCCESS;
 }
 
+// ---- products over planes -----------------------------------------------------
+// Block shape: 64 x 128 (two waves) for at most 64 rows of B, else 128 x 128,
+// or 256 x 256 (eight waves, one block per CU) where at least one block per
+// compute unit of them remains.
+enum PlaneShape : int
+{
+    PLANES_64 = 0,
+    PLANES_128 = 1,
+    PLANES_256 = 2
+};
+PlaneShape plane_shape(const Fold &f, int parts)
+{
+    uint64_t const ncols = f.outer * f.w;
+    if (f.m <= 64) return PLANES_64;
+    uint64_t const big = ((f.m + 255) / 256) * ((ncols + 255) / 256);
+    if (parts < 3 && f.m > 128 && big >= (uint64_t)device_cus()) return PLANES_256;
+    return PLANES_128;
+}
+struct PlaneGeom
+{
+    uint64_t bm, bn, ldk, rows_a, rows_b, plane_a, plane_b;
+    size_t bytes; // of both operands' planes
+};
+PlaneGeom plane_geom(const Fold &f, int parts)
+{
+    PlaneShape const sh = plane_shape(f, parts);
+    PlaneGeom g;
+    g.bm = sh == PLANES_64 ? 64 : sh == PLANES_128 ? 128 : 256;
+    g.bn = sh == PLANES_256 ? 256 : 128;
+    uint64_t const kq = parts == 1 ? 64 : 32; // contraction indices per stage
+    g.ldk = (f.nq + kq - 1) / kq * kq;
+    if (f.w != 1) g.ldk = (g.ldk + 63) / 64 * 64; // the NN conversion writes 64 x 64 tiles
+    uint64_t const ncols = f.outer * f.w;
+    g.rows_a = (ncols + g.bn - 1) / g.bn * g.bn;
+    g.rows_b = (f.m + g.bm - 1) / g.bm * g.bm;
+    g.plane_a = g.rows_a * g.ldk;
+    g.plane_b = g.rows_b * g.ldk;
+    g.bytes = (size_t)parts * (g.plane_a + g.plane_b) * 2;
+    return g;
+}
+int mode_parts(ttm_precision_t prec) { return prec == TTM_PREC_BF16X3 ? 3 : prec == TTM_PREC_FP16X2 ? 2 : 1; }
+
+template <int MODE, int WM, int WN, int JT, int NT, int KS>
+void launch_planes_shape(const Fold &f, const PlaneGeom &g, const typename Lp<MODE>::op *as,
+                         const typename Lp<MODE>::op *bs, float *c, const int *exps, hipStream_t s)
+{
+    using S = PlaneTile<MODE, WM, WN, JT, NT, KS>;
+    unsigned const nj = (unsigned)(g.rows_b / S::BM);
+    unsigned const total = nj * (unsigned)(g.rows_a / S::BN);
+    bool const ts = f.w == 1;
+    int const c_vec = (reinterpret_cast<uintptr_t>(c) & 15u) == 0 && (ts ? f.m : f.w) % 4 == 0;
+    uint64_t const ncols = f.outer * f.w;
+    if (ts)
+        hipLaunchKernelGGL((k_planes<MODE, WM, WN, JT, NT, KS, true>), dim3(total), dim3(64 * WM * WN), 0, s, as,
+                           g.plane_a, bs, g.plane_b, g.ldk, c, ncols, f.w, f.m, nj, total, c_vec, exps);
+    else
+        hipLaunchKernelGGL((k_planes<MODE, WM, WN, JT, NT, KS, false>), dim3(total), dim3(64 * WM * WN), 0, s, as,
+                           g.plane_a, bs, g.plane_b, g.ldk, c, ncols, f.w, f.m, nj, total, c_vec, exps);
+}
+
+template <int MODE>
+ttm_status_t launch_planes(const Fold &f, const float *a, const float *b, float *c, hipStream_t s)
+{
+    using op = typename Lp<MODE>::op;
+    constexpr int P = Lp<MODE>::PARTS;
+    constexpr bool SCALED = MODE == LP_FP16X2;
+    PlaneGeom const g = plane_geom(f, P);
+    uint64_t const ncols = f.outer * f.w;
+    size_t const planes_bytes = (g.bytes + 255) / 256 * 256;
+    ScalePass const sp = SCALED ? scale_pass(f, true) : ScalePass();
+    void *ws = nullptr;
+    if (ttm_status_t const st = ws_acquire(planes_bytes + (SCALED ? sp.bytes() : 0), s, &ws,
+                                           "workspace for the converted operands");
+        st != TTM_SUCCESS)
+        return st;
+    op *const as = static_cast<op *>(ws);
+    op *const bs = as + P * g.plane_a;
+    int const *exps = nullptr;
+    if constexpr (SCALED) exps = launch_scale_pass(f, a, b, sp, static_cast<char *>(ws) + planes_bytes, s);
+    unsigned const blocks_a =
+        (unsigned)(f.w == 1 ? (g.plane_a / 8 + 255) / 256 : g.rows_a / 64 * (g.ldk / 64));
+    unsigned const blocks_b = (unsigned)((g.plane_b / 8 + 255) / 256);
+    auto const convert = f.w == 1 ? k_planes_convert<MODE, true> : k_planes_convert<MODE, false>;
+    hipLaunchKernelGGL(convert, dim3(blocks_a + blocks_b), dim3(256), 0, s, a, as, ncols, f.w, g.rows_a, g.plane_a, b,
+                       bs, f.m, f.b_stride_j(), f.b_stride_l(), g.rows_b, g.plane_b, f.nq, g.ldk, blocks_a, exps);
+    constexpr int KS = P == 1 ? 2 : 1;
+    PlaneShape const sh = plane_shape(f, P);
+    if (sh == PLANES_64) {
+        launch_planes_shape<MODE, 1, 2, 4, 4, KS>(f, g, as, bs, c, exps, s);
+    } else if (sh == PLANES_128) {
+        launch_planes_shape<MODE, 2, 2, 4, 4, KS>(f, g, as, bs, c, exps, s);
+    } else {
+        if constexpr (P < 3) launch_planes_shape<MODE, 2, 4, 8, 4, KS>(f, g, as, bs, c, exps, s);
+    }
+    hipError_t const e = hipGetLastError();
+    ws_release(ws, s);
+    if (e != hipSuccess) {
+        set_error(TTM_ERR_HIP, hipGetErrorString(e));
+        return TTM_ERR_HIP;
+    }
+    return TTM_SUCCESS;
+}
+
 // Rows of B per FP8 block: 128 where B has more than 64 rows (each block's
 // copy of A's slice then serves twice as many rows of C), else 64.
 int fp8_block_rows(const Fold &f) { return f.m > 64 ? 128 : 64; }
 
+// Workspace of the quantized operands and their scales.
+struct Fp8Bytes
+{
+    size_t qb, sb, qa, sa;
+    size_t total() const { return qb + sb + qa + sa; }
+};
+Fp8Bytes fp8_bytes(const Fold &f)
+{
+    uint64_t const bm = (uint64_t)fp8_block_rows(f);
+    uint64_t const ldq = (f.nq + 127) / 128 * 128;
+    uint64_t const rows_b = (f.m + bm - 1) / bm * bm;
+    uint64_t const rows_a = (f.outer * f.w + 63) / 64 * 64;
+    auto round256 = [](uint64_t x) { return (x + 255) / 256 * 256; };
+    return {round256(rows_b * ldq), round256(rows_b * (ldq / 32)), round256(rows_a * ldq),
+            round256(rows_a * (ldq / 32))};
+}
+
 // A and B quantized once per product (k_fp8_split_a_*, k_fp8_split_b) into
 // pooled workspace: N_A + m n_q bytes (rounded up to whole blocks and
 // slices) plus a scale byte per 32 of them; then the tiles.
-template <bool TN>
+template <bool TN, bool ANY>
 ttm_status_t launch_fp8(const Fold &f, const float *a, const float *b, float *c, hipStream_t s)
 {
     uint64_t const bm = (uint64_t)fp8_block_rows(f);
@@ -1454,9 +2012,8 @@ ttm_status_t launch_fp8(const Fold &f, const float *a, const float *b, float *c,
         set_error(TTM_ERR_ARGUMENT, "operands too large for the FP8 kernels");
         return TTM_ERR_ARGUMENT;
     }
-    auto round256 = [](uint64_t x) { return (x + 255) / 256 * 256; };
-    size_t const bytes_qb = round256(rows * ldq), bytes_sb = round256(rows * (ldq / 32));
-    size_t const bytes_qa = round256(rows_a * ldq), bytes_sa = round256(rows_a * (ldq / 32));
+    Fp8Bytes const by = fp8_bytes(f);
+    size_t const bytes_qb = by.qb, bytes_sb = by.sb, bytes_qa = by.qa, bytes_sa = by.sa;
     void *ws = nullptr;
     if (ttm_status_t const st = ws_acquire(bytes_qb + bytes_sb + bytes_qa + bytes_sa, s, &ws,
                                            "workspace for the quantized operands");
@@ -1469,10 +2026,10 @@ ttm_status_t launch_fp8(const Fold &f, const float *a, const float *b, float *c,
     hipLaunchKernelGGL(k_fp8_split_b, dim3((unsigned)split_blocks), dim3(256), 0, s, b, qb, sb, f.m, f.nq,
                        f.b_stride_j(), f.b_stride_l(), ldq, rows);
     if constexpr (TN)
-        hipLaunchKernelGGL(k_fp8_split_a_rows, dim3((unsigned)split_a_blocks), dim3(256), 0, s, a, qa, sa, ncols,
+        hipLaunchKernelGGL(k_fp8_split_a_rows<ANY>, dim3((unsigned)split_a_blocks), dim3(256), 0, s, a, qa, sa, ncols,
                            f.nq, ldq, ldq / 128);
     else
-        hipLaunchKernelGGL(k_fp8_split_a_cols, dim3((unsigned)split_a_blocks), dim3(256), 0, s, a, qa, sa, ncols,
+        hipLaunchKernelGGL(k_fp8_split_a_cols<ANY>, dim3((unsigned)split_a_blocks), dim3(256), 0, s, a, qa, sa, ncols,
                            f.nq, f.w, ldq, ldq / 128);
     if (bm == 128)
         hipLaunchKernelGGL((k_fp8<TN, 128>), dim3(total), dim3(256), 0, s, qa, sa, qb, sb, ldq, c, ncols, f.nq, f.w,
@@ -1488,6 +2045,10 @@ ttm_status_t launch_fp8(const Fold &f, const float *a, const float *b, float *c,
     }
     return TTM_SUCCESS;
 }
+
+// Largest workspace of a product over planes; beyond it the padding of a
+// degenerate shape (a column or a row against a whole tile) is the bulk.
+constexpr size_t kAnyMaxBytes = 32ull << 30;
 
 template <int MODE>
 ttm_status_t launch_lp_mode(const Fold &f, const float *a, const float *b, float *c, hipStream_t s)
@@ -1507,18 +2068,50 @@ bool lowp_supports(const Fold &f, bool aligned)
     return blocks < (1ull << 31);
 }
 
-std::string lowp_symbol(const Fold &f, ttm_precision_t prec, bool generic)
+bool lowp_any_supports(const Fold &f, ttm_precision_t prec)
+{
+    // Short contractions over few elements: one thread per element takes about
+    // 6 us + 0.4 us per contraction index (a serial chain), the conversions
+    // and the product 15-20 us ([63, K, 31] x_2, m = 33, bf16: 9.3 / 19 / 57 us
+    // at K = 9 / 33 / 129 against 21-23 us).
+    if (f.nq <= 24 && f.m * f.numel_a() <= (8u << 20)) return false;
+    // grid limits, 32-bit byte offsets within a block's rows, and a bound on
+    // what the padding to whole tiles may cost
+    if (f.nq >= (1ull << 22)) return false;
+    if (prec == TTM_PREC_FP8_E4M3)
+        return fp8_bytes(f).total() <= kAnyMaxBytes && ((f.outer * f.w + 63) / 64) * ((f.m + 63) / 64) < (1ull << 31);
+    PlaneGeom const g = plane_geom(f, mode_parts(prec));
+    // blocks of the conversions: 8 elements a thread, or 64 x 64 tiles
+    return g.bytes <= kAnyMaxBytes && (g.rows_a / g.bn) * (g.rows_b / g.bm) < (1ull << 31) &&
+           g.plane_a / 2048 + g.plane_b / 2048 + 2 < (1ull << 31);
+}
+
+bool lowp_any_fits(const Fold &f, ttm_precision_t prec)
+{
+    if (!lowp_any_supports(f, prec)) return false;
+    size_t const room = scratch_available();
+    if (prec == TTM_PREC_FP8_E4M3) return fp8_bytes(f).total() <= room;
+    size_t const scale = prec == TTM_PREC_FP16X2 ? scale_pass(f, true).bytes() : 0;
+    return plane_geom(f, mode_parts(prec)).bytes + 512 + scale <= room;
+}
+
+std::string lowp_symbol(const Fold &f, ttm_precision_t prec, bool generic, bool aligned)
 {
     char const *tn = f.w == 1 ? "true" : "false";
     char buf[96];
     if (generic) return "k_lowp_generic";
+    int const mode = prec == TTM_PREC_BF16 ? LP_BF16
+                     : prec == TTM_PREC_FP16 ? LP_FP16
+                     : prec == TTM_PREC_FP16X2 ? LP_FP16X2
+                                               : LP_BF16X3;
     if (prec == TTM_PREC_FP8_E4M3) {
         std::snprintf(buf, sizeof buf, "k_fp8<%s, %d>", tn, fp8_block_rows(f));
+    } else if (!lowp_supports(f, aligned)) {
+        static const char *const shapes[] = {"1, 2, 4, 4", "2, 2, 4, 4", "2, 4, 8, 4"};
+        int const parts = mode_parts(prec);
+        std::snprintf(buf, sizeof buf, "k_planes<%d, %s, %d, %s>", mode, shapes[plane_shape(f, parts)],
+                      parts == 1 ? 2 : 1, tn);
     } else {
-        int const mode = prec == TTM_PREC_BF16 ? LP_BF16
-                         : prec == TTM_PREC_FP16 ? LP_FP16
-                         : prec == TTM_PREC_FP16X2 ? LP_FP16X2
-                                                   : LP_BF16X3;
         std::snprintf(buf, sizeof buf, "k_lowp<%d, %s, %d>", mode, tn, lp_block_rows(f));
     }
     return buf;
@@ -1527,6 +2120,9 @@ std::string lowp_symbol(const Fold &f, ttm_precision_t prec, bool generic)
 ttm_status_t launch_lowp(const Fold &f, const float *a, const float *b, float *c, ttm_precision_t prec,
                          hipStream_t s, bool generic)
 {
+    bool const aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) |
+                           reinterpret_cast<uintptr_t>(c)) & 15u) == 0;
+    bool const tile = !generic && lowp_supports(f, aligned);
     if (generic) {
         uint64_t const total = f.numel_c();
         uint64_t blocks = (total + 255) / 256;
@@ -1544,7 +2140,15 @@ ttm_status_t launch_lowp(const Fold &f, const float *a, const float *b, float *c
                            f.m, f.b_stride_j(), f.b_stride_l(), (int)prec, exps);
         ws_release(ws, s);
     } else if (prec == TTM_PREC_FP8_E4M3) {
-        return f.w == 1 ? launch_fp8<true>(f, a, b, c, s) : launch_fp8<false>(f, a, b, c, s);
+        if (!tile) return f.w == 1 ? launch_fp8<true, true>(f, a, b, c, s) : launch_fp8<false, true>(f, a, b, c, s);
+        return f.w == 1 ? launch_fp8<true, false>(f, a, b, c, s) : launch_fp8<false, false>(f, a, b, c, s);
+    } else if (!tile) {
+        switch (prec) {
+        case TTM_PREC_BF16: return launch_planes<LP_BF16>(f, a, b, c, s);
+        case TTM_PREC_FP16: return launch_planes<LP_FP16>(f, a, b, c, s);
+        case TTM_PREC_FP16X2: return launch_planes<LP_FP16X2>(f, a, b, c, s);
+        default: return launch_planes<LP_BF16X3>(f, a, b, c, s);
+        }
     } else if (prec == TTM_PREC_BF16) {
         return launch_lp_mode<LP_BF16>(f, a, b, c, s);
     } else if (prec == TTM_PREC_FP16) {

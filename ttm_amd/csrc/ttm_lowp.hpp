@@ -16,8 +16,15 @@ namespace ttm_amd
 // either w == 1 with nq % 4 == 0 (TN view) or w % 4 == 0 (NN view).
 bool lowp_supports(const Fold &f, bool aligned);
 
-// Template instance launched for a fold and precision (as profilers print it).
-std::string lowp_symbol(const Fold &f, ttm_precision_t prec, bool generic);
+// True when the kernels over pre-converted operands can run the fold (any
+// extents, element-aligned buffers), and when their workspace also fits the
+// scratch region bound to this thread, if one is.
+bool lowp_any_supports(const Fold &f, ttm_precision_t prec);
+bool lowp_any_fits(const Fold &f, ttm_precision_t prec);
+
+// Template instance launched for a fold and precision (as profilers print it);
+// `aligned`: A, B and C 16-byte aligned.
+std::string lowp_symbol(const Fold &f, ttm_precision_t prec, bool generic, bool aligned);
 
 // `generic` selects the one-thread-per-element kernel (any shape/alignment).
 ttm_status_t launch_lowp(const Fold &f, const float *a, const float *b, float *c, ttm_precision_t prec,
