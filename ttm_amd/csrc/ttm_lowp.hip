@@ -806,16 +806,16 @@ __device__ __forceinline__ void lowp_tile(const float *__restrict__ a, const flo
 // product): plane p at bs + p * plane, row j at j * ldb, zero outside m x nq.
 // One thread per 8 consecutive l of a row.
 template <int MODE>
-__device__ __forceinline__ void split_b_block(unsigned block, const float *__restrict__ b, typename Lp<MODE>::op *__restrict__ bs,
-                                              uint64_t m, uint64_t nq, uint64_t bsj, uint64_t bsl, uint64_t ldb,
-                                              uint64_t rows, uint64_t plane, int eb)
+__global__ __launch_bounds__(256) void k_lowp_split_b(const float *__restrict__ b, typename Lp<MODE>::op *__restrict__ bs,
+                                                      uint64_t m, uint64_t nq, uint64_t bsj, uint64_t bsl, uint64_t ldb,
+                                                      uint64_t rows, uint64_t plane, const int *__restrict__ exps)
 {
     using L = Lp<MODE>;
     using v2 = typename L::v2;
     using v8 = typename L::v8;
     constexpr int P = L::PARTS;
     uint64_t const groups = ldb / 8;
-    uint64_t const idx = (uint64_t)block * 256 + threadIdx.x;
+    uint64_t const idx = (uint64_t)blockIdx.x * 256 + threadIdx.x;
     if (idx >= rows * groups) return;
     uint64_t const j = idx / groups, l0 = (idx - j * groups) * 8;
     v2 q[4][P];
@@ -827,7 +827,7 @@ __device__ __forceinline__ void split_b_block(unsigned block, const float *__res
             uint64_t const l = l0 + 2 * t + e;
             x[e] = (j < m && l < nq) ? b[j * bsj + l * bsl] : 0.f;
         }
-        if constexpr (MODE == LP_FP16X2) x = scale2(x, eb);
+        if constexpr (MODE == LP_FP16X2) x = scale2(x, exps[1]);
         L::split2(x, q[t]);
     }
 #pragma unroll
@@ -836,14 +836,6 @@ __device__ __forceinline__ void split_b_block(unsigned block, const float *__res
         auto const hi = __builtin_shufflevector(q[2][p], q[3][p], 0, 1, 2, 3);
         *reinterpret_cast<v8 *>(bs + p * plane + j * ldb + l0) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     }
-}
-
-template <int MODE>
-__global__ __launch_bounds__(256) void k_lowp_split_b(const float *__restrict__ b, typename Lp<MODE>::op *__restrict__ bs,
-                                                      uint64_t m, uint64_t nq, uint64_t bsj, uint64_t bsl, uint64_t ldb,
-                                                      uint64_t rows, uint64_t plane, const int *__restrict__ exps)
-{
-    split_b_block<MODE>(blockIdx.x, b, bs, m, nq, bsj, bsl, ldb, rows, plane, MODE == LP_FP16X2 ? exps[1] : 0);
 }
 
 // One product: a grid of BM x 128 blocks over the pre-converted B (BM = 64
@@ -976,134 +968,170 @@ __global__ __launch_bounds__(256, lp_group_blocks_per_cu(BM)) void k_lowp_groupe
 // column n of the fold as row n, contiguous along l, zero-padded to whole
 // tiles and slices -- so the product kernel moves only whole, aligned 16-byte
 // pieces by LDS DMA, whatever w, n_q and the base pointers are.  Bound by the
-// traffic of the passes: A [255, 301, 173] x_2, m = 120, FP16X2 1670 -> 75 us
+// traffic of the passes: A [255, 301, 173] x_2, m = 120, FP16X2 1670 -> 70 us
 // (one thread per element before: serial chains of n_q loads), BF16X3
-// 1597 -> 81, BF16 1449 -> 44, FP8 2440 -> 56 us; of FP16X2's 68 us in
-// kernels the scale pass takes 15 (5.3 TB/s), the conversion 27 (4.4 TB/s)
-// and the product 23.
+// 1597 -> 77, BF16 1449 -> 42, FP8 2440 -> 56 us.  Where A and C are aligned
+// the fused tiles (lowp_tile) stay: they read A once, the planes' passes move
+// 3 to 4 times its bytes (A 1024x1024x512, m = 1024: FP16X2 3.8 against
+// 3.7 ms, BF16 1.9-2.2 against 2.0-2.1 ms, m = 256: 1.0 against 0.67 ms).
 // ---------------------------------------------------------------------------
 
-// A -> planes, TN view: rows of A are contiguous along l, in the order of the
-// planes.  One thread per 8 consecutive l of a row: two 16-byte loads at
-// element alignment, one 16-byte store per plane.
+// Layout of a plane: for every group of 64 rows and slice of 32 l a block of
+// 4 KB, groups slowest, in the order the block has in LDS (physical rows of
+// lds_row, chunks swizzled by lds_swz).  A piece of 16 physical rows is 1 KB
+// of consecutive memory, so a wave's LDS DMA reads whole lines of consecutive
+// addresses (from planes of plain rows it read 16 pieces of 64 bytes whole rows
+// apart): the FP16X2 product of A 1024x1024x512 x_2, m = 1024 takes 2.59 ms
+// (1275 TFLOP/s on the matrix cores) against 2.87.
+// Element offset of the 8 elements (row, chunk) of slice sl, nsl slices a row.
+__device__ __forceinline__ uint64_t plane_at(uint64_t row, uint64_t sl, int chunk, uint64_t nsl)
+{
+    int const P = lds_row((int)(row & 63));
+    return (((row >> 6) * nsl + sl) << 11) + lds_at(P, chunk);
+}
+
+// Eight consecutive l of a row -> one 16-byte store per plane.
 template <int MODE>
-__device__ __forceinline__ void planes_a_rows(unsigned block, const float *__restrict__ a, typename Lp<MODE>::op *__restrict__ as,
-                                              uint64_t ncols, uint64_t nq, uint64_t ldk, uint64_t rows, uint64_t plane,
-                                              int ea)
+__device__ __forceinline__ void plane_store(const f32x4 (&v)[2], int e, typename Lp<MODE>::op *dst, uint64_t plane)
 {
     using L = Lp<MODE>;
     using v2 = typename L::v2;
     using v8 = typename L::v8;
     constexpr int P = L::PARTS;
-    uint64_t const groups = ldk / 8;
-    uint64_t const idx = (uint64_t)block * 256 + threadIdx.x;
-    if (idx >= rows * groups) return;
-    uint64_t const n = idx / groups, l0 = (idx - n * groups) * 8;
-    f32x4 v[2] = {zero4(), zero4()};
-    if (n < ncols) {
-        const float *row = a + n * nq;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            uint64_t const l = l0 + 4 * h;
-            if (l + 4 <= nq) {
-                f32x4 const x = ldg<f32x4u>(row + l);
-                v[h] = x;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (l + e < nq) v[h][e] = ldg<float>(row + l + e);
-            }
-        }
-    }
     v2 q[4][P];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
         f32x2 x = {v[t >> 1][2 * (t & 1)], v[t >> 1][2 * (t & 1) + 1]};
-        if constexpr (MODE == LP_FP16X2) x = scale2(x, ea);
+        if constexpr (MODE == LP_FP16X2) x = scale2(x, e);
         L::split2(x, q[t]);
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         auto const lo = __builtin_shufflevector(q[0][p], q[1][p], 0, 1, 2, 3);
         auto const hi = __builtin_shufflevector(q[2][p], q[3][p], 0, 1, 2, 3);
-        stg<v8>(as + p * plane + n * ldk + l0, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        stg<v8>(dst + p * plane, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
+}
+
+// Rows contiguous along l (A in the TN view, a row-major B; `nrows` of them, at
+// element alignment) -> planes.  One block per 64 rows and 4 slices; a wave
+// instruction reads the 128 bytes of a slice of 8 rows (16 bytes a lane, 8
+// loads in flight) and stores 512 consecutive bytes per plane.
+template <int MODE>
+__device__ __forceinline__ void planes_from_rows(uint64_t group, uint64_t sl0, const float *__restrict__ x,
+                                                 uint64_t nrows, uint64_t nq, uint64_t nsl,
+                                                 typename Lp<MODE>::op *__restrict__ out, uint64_t plane, int e)
+{
+    using L = Lp<MODE>;
+    using v2 = typename L::v2;
+    using v4 = typename L::v4;
+    constexpr int P = L::PARTS;
+    int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    f32x4 v[2][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        int const pr = 16 * wave + 8 * h + (lane >> 3); // physical row of the group
+        uint64_t const row = 64 * group + lds_row_inv(pr);
+        const float *src = x + (row < nrows ? row : 0) * nq;
+        int const chunk = (lane >> 1 & 3) ^ lds_swz(pr);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint64_t const l = 32 * (sl0 + i) + 8 * chunk + 4 * (lane & 1);
+            v[h][i] = zero4();
+            if (row < nrows && l + 4 <= nq) {
+                f32x4 const t = ldg<f32x4u>(src + l);
+                v[h][i] = t;
+            } else if (row < nrows) {
+#pragma unroll
+                for (int y = 0; y < 4; ++y)
+                    if (l + y < nq) v[h][i][y] = ldg<float>(src + l + y);
+            }
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (sl0 + i >= nsl) break;
+            f32x2 lo = {v[h][i][0], v[h][i][1]}, hi = {v[h][i][2], v[h][i][3]};
+            if constexpr (MODE == LP_FP16X2) {
+                lo = scale2(lo, e);
+                hi = scale2(hi, e);
+            }
+            v2 ql[P], qh[P];
+            L::split2(lo, ql);
+            L::split2(hi, qh);
+            auto *dst = out + ((group * nsl + sl0 + i) << 11) + (16 * wave + 8 * h) * LP_LDK + 4 * lane;
+#pragma unroll
+            for (int p = 0; p < P; ++p) stg<v4>(dst + p * plane, __builtin_shufflevector(ql[p], qh[p], 0, 1, 2, 3));
+        }
 }
 
 // A -> planes, NN view: column n = k * w + i runs along l with stride w.  One
 // block per 64 columns x 64 l: lane = column, so a wave instruction reads 64
 // consecutive floats of one row l (256 bytes, any alignment, across slab
-// ends), 16 rows per thread in flight; the converted columns cross LDS and
-// leave as 128-byte row segments.  The columns' places cost one division per
-// thread.
+// ends), 16 rows per thread in flight; the columns cross LDS as floats and
+// leave as whole pieces.  The columns' places cost one division per thread.
+// (A column-major B is the same with w = nrows = m and one slab.)
 template <int MODE>
-__device__ __forceinline__ void planes_a_cols(unsigned block, const float *__restrict__ a, typename Lp<MODE>::op *__restrict__ as,
-                                              uint64_t ncols, uint64_t nq, uint64_t w, uint64_t ldk, uint64_t plane,
-                                              int ea)
+__device__ __forceinline__ void planes_from_cols(uint64_t group, uint64_t sl0, const float *__restrict__ x,
+                                                 uint64_t ncols, uint64_t nq, uint64_t w, uint64_t nsl,
+                                                 typename Lp<MODE>::op *__restrict__ out, uint64_t plane, int e)
 {
-    using L = Lp<MODE>;
-    using op = typename L::op;
-    using v2 = typename L::v2;
-    using v8 = typename L::v8;
-    constexpr int P = L::PARTS;
-    constexpr int LDT = 64 + 8; // elements per column in LDS (16-byte pieces spread over the banks)
-    __shared__ __attribute__((aligned(16))) op sT[P][64 * LDT];
-    unsigned const lblocks = (unsigned)(ldk / 64);
-    uint64_t const cb = block / lblocks, l0 = (uint64_t)(block % lblocks) * 64;
-    uint64_t const n0 = cb * 64;
-    int const tid = threadIdx.x, c = tid & 63, g = tid >> 6;
-    uint64_t const n = n0 + c;
-    bool const ok = n < ncols;
-    uint64_t const k = ok ? n / w : 0;
-    const float *col = a + k * nq * w + (ok ? n - k * w : 0);
-    float v[16];
+    constexpr int LDT = 64 + 4; // floats per column in LDS
+    __shared__ __attribute__((aligned(16))) float sT[64 * LDT];
+    int const lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    {
+        uint64_t const n = 64 * group + lane;
+        bool const ok = n < ncols;
+        uint64_t const k = ok ? n / w : 0;
+        const float *col = x + k * nq * w + (ok ? n - k * w : 0);
+        f32x4 v[4];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        uint64_t const l = l0 + 16 * g + e;
-        v[e] = (ok && l < nq) ? ldg_nt<float>(col + l * w) : 0.f;
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        v2 q[4][P];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            f32x2 x = {v[8 * h + 2 * t], v[8 * h + 2 * t + 1]};
-            if constexpr (MODE == LP_FP16X2) x = scale2(x, ea);
-            L::split2(x, q[t]);
+        for (int y = 0; y < 16; ++y) {
+            uint64_t const l = 32 * sl0 + 16 * wave + y;
+            v[y >> 2][y & 3] = (ok && l < nq) ? ldg_nt<float>(col + l * w) : 0.f;
         }
 #pragma unroll
-        for (int p = 0; p < P; ++p) {
-            auto const lo = __builtin_shufflevector(q[0][p], q[1][p], 0, 1, 2, 3);
-            auto const hi = __builtin_shufflevector(q[2][p], q[3][p], 0, 1, 2, 3);
-            *reinterpret_cast<v8 *>(&sT[p][c * LDT + 16 * g + 8 * h]) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        }
+        for (int y = 0; y < 4; ++y) *reinterpret_cast<f32x4 *>(&sT[lane * LDT + 16 * wave + 4 * y]) = v[y];
     }
     __syncthreads();
+    int const P = 16 * wave + (lane >> 2);
+    int const chunk = (lane & 3) ^ lds_swz(P);
+    int const r = lds_row_inv(P);
 #pragma unroll
-    for (int p = 0; p < P; ++p)
+    for (int i = 0; i < 2; ++i) {
+        if (sl0 + i >= nsl) break;
+        f32x4 v[2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            int const r = (tid >> 3) + 32 * i, piece = tid & 7;
-            stg<v8>(as + p * plane + (n0 + r) * ldk + l0 + 8 * piece,
-                    *reinterpret_cast<const v8 *>(&sT[p][r * LDT + 8 * piece]));
-        }
+        for (int h = 0; h < 2; ++h)
+            v[h] = *reinterpret_cast<const f32x4 *>(&sT[r * LDT + 32 * i + 8 * chunk + 4 * h]);
+        plane_store<MODE>(v, e, out + plane_at(64 * group + r, sl0 + i, chunk, nsl), plane);
+    }
 }
 
 // Both conversions in one launch: blocks [0, blocks_a) take A, the rest B.
-template <int MODE, bool TN>
-__global__ __launch_bounds__(256) void k_planes_convert(
-    const float *__restrict__ a, typename Lp<MODE>::op *__restrict__ as, uint64_t ncols, uint64_t w, uint64_t rows_a,
-    uint64_t plane_a, const float *__restrict__ b, typename Lp<MODE>::op *__restrict__ bs, uint64_t m, uint64_t bsj,
-    uint64_t bsl, uint64_t rows_b, uint64_t plane_b, uint64_t nq, uint64_t ldk, unsigned blocks_a,
-    const int *__restrict__ exps)
+// An operand's blocks run over its groups of 64 rows, 4 (rows) or 2 (columns)
+// slices each, slices fastest.
+template <int MODE>
+__global__ __launch_bounds__(256) void k_planes_convert(const float *__restrict__ a, typename Lp<MODE>::op *__restrict__ as,
+                                                        uint64_t ncols, uint64_t w, uint64_t plane_a,
+                                                        const float *__restrict__ b, typename Lp<MODE>::op *__restrict__ bs,
+                                                        uint64_t m, int b_rows, uint64_t plane_b, uint64_t nq, unsigned nsl,
+                                                        unsigned blocks_a, const int *__restrict__ exps)
 {
-    int const ea = MODE == LP_FP16X2 ? exps[0] : 0, eb = MODE == LP_FP16X2 ? exps[1] : 0;
-    if (blockIdx.x >= blocks_a)
-        split_b_block<MODE>(blockIdx.x - blocks_a, b, bs, m, nq, bsj, bsl, ldk, rows_b, plane_b, eb);
-    else if constexpr (TN)
-        planes_a_rows<MODE>(blockIdx.x, a, as, ncols, nq, ldk, rows_a, plane_a, ea);
-    else
-        planes_a_cols<MODE>(blockIdx.x, a, as, ncols, nq, w, ldk, plane_a, ea);
+    bool const is_a = blockIdx.x < blocks_a;
+    unsigned const block = is_a ? blockIdx.x : blockIdx.x - blocks_a;
+    int const e = MODE == LP_FP16X2 ? exps[is_a ? 0 : 1] : 0;
+    bool const rows = is_a ? w == 1 : b_rows != 0;
+    unsigned const step = rows ? 4 : 2, per = (nsl + step - 1) / step;
+    uint64_t const group = block / per;
+    uint64_t const sl0 = (uint64_t)(block % per) * step;
+    const float *x = is_a ? a : b;
+    auto *out = is_a ? as : bs;
+    uint64_t const n = is_a ? ncols : m, plane = is_a ? plane_a : plane_b;
+    if (rows) planes_from_rows<MODE>(group, sl0, x, n, nq, nsl, out, plane, e);
+    else planes_from_cols<MODE>(group, sl0, x, n, nq, is_a ? w : m, nsl, out, plane, e);
 }
 
 // The product: WM x WN waves, each JT x NT MFMA tiles of 16 x 16; block
@@ -1117,12 +1145,12 @@ __global__ __launch_bounds__(256) void k_planes_convert(
 // read one MFMA group ahead, and behind the last reads come the wait for that
 // DMA and the one barrier; the stage's last MFMA group runs behind it, while
 // the next stage's first fragments are read.
-template <int MODE, int WM, int WN, int JT, int NT, int KS>
+template <int MODE, int WM, int WN, int JT, int NT, int KS, int NS>
 struct PlaneTile
 {
     static constexpr int BM = 16 * JT * WM, BN = 16 * NT * WN, WAVES = WM * WN;
     static constexpr int P = Lp<MODE>::PARTS;
-    static constexpr int LDS_BYTES = 2 * KS * P * (BM + BN) * LP_LDK * 2;
+    static constexpr int LDS_BYTES = NS * KS * P * (BM + BN) * LP_LDK * 2;
     // blocks per CU: by LDS, at most 2 waves per SIMD of 256 registers for the
     // 128 x 64 wave tiles, 4 of 128 registers otherwise
     static constexpr int by_lds = 160 * 1024 / LDS_BYTES;
@@ -1131,8 +1159,8 @@ struct PlaneTile
     static constexpr int waves_per_simd = blocks * WAVES / 4 > 0 ? blocks * WAVES / 4 : 1;
 };
 
-template <int MODE, int WM, int WN, int JT, int NT, int KS, bool TSTORE>
-__global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>::waves_per_simd)) void k_planes(
+template <int MODE, int WM, int WN, int JT, int NT, int KS, int NS, bool TSTORE>
+__global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS, NS>::waves_per_simd)) void k_planes(
     const typename Lp<MODE>::op *__restrict__ as, uint64_t plane_a, const typename Lp<MODE>::op *__restrict__ bs,
     uint64_t plane_b, uint64_t ldk, float *__restrict__ c, uint64_t ncols, uint64_t w, uint64_t m, unsigned nj,
     unsigned total, int c_vec, const int *__restrict__ exps)
@@ -1140,11 +1168,30 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
     using L = Lp<MODE>;
     using op = typename L::op;
     using v8 = typename L::v8;
-    using S = PlaneTile<MODE, WM, WN, JT, NT, KS>;
+    using S = PlaneTile<MODE, WM, WN, JT, NT, KS, NS>;
     constexpr int P = L::PARTS, BM = S::BM, BN = S::BN, WAVES = S::WAVES;
     static_assert(NT == 4 && JT % 4 == 0, "a lane's four column and row tiles are adjacent columns and rows");
-    __shared__ __attribute__((aligned(16))) op sA0[KS][P][BN * LP_LDK], sA1[KS][P][BN * LP_LDK];
-    __shared__ __attribute__((aligned(16))) op sB0[KS][P][BM * LP_LDK], sB1[KS][P][BM * LP_LDK];
+    // (arrays of their own, so that the compiler tells a stage's reads from
+    // the other stages' DMA; those past NS are unreferenced, and so not
+    // allocated)
+    __shared__ __attribute__((aligned(16))) op sA0[KS][P][BN * LP_LDK], sA1[KS][P][BN * LP_LDK], sA2[KS][P][BN * LP_LDK],
+        sA3[KS][P][BN * LP_LDK];
+    __shared__ __attribute__((aligned(16))) op sB0[KS][P][BM * LP_LDK], sB1[KS][P][BM * LP_LDK], sB2[KS][P][BM * LP_LDK],
+        sB3[KS][P][BM * LP_LDK];
+    auto buf_a = [&](auto tag) {
+        constexpr int i = decltype(tag)::value % NS;
+        if constexpr (i == 0) return sA0;
+        else if constexpr (i == 1) return sA1;
+        else if constexpr (i == 2) return sA2;
+        else return sA3;
+    };
+    auto buf_b = [&](auto tag) {
+        constexpr int i = decltype(tag)::value % NS;
+        if constexpr (i == 0) return sB0;
+        else if constexpr (i == 1) return sB1;
+        else if constexpr (i == 2) return sB2;
+        else return sB3;
+    };
 
     unsigned jb, nb;
     lp_block_coords(nj, total, jb, nb);
@@ -1158,10 +1205,8 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
     // a buffer load it counts against the vector-memory counter alone (the
     // global form also holds up every LDS wait).  Byte offsets within a
     // block's rows stay below 2^32 (n_q < 2^22).
-    // Lane's offset within a piece of 16 physical rows: logical row 4 (lane / 4)
-    // past the piece's first, chunk (lane % 4) ^ swizzle.
-    uint32_t const ldk2 = (uint32_t)ldk * 2u;
-    uint32_t const lane_off = 4u * (uint32_t)(lane >> 2) * ldk2 + 16u * (uint32_t)((lane & 3) ^ lds_swz(lane >> 2));
+    uint32_t const nsl = (uint32_t)(ldk / 32);
+    uint32_t const lane_off = 16u * (uint32_t)lane;
     // (the block's place comes out of a division in vector registers; a
     // descriptor is scalar)
     auto rows = [&](const op *base, uint32_t bytes) {
@@ -1173,8 +1218,8 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
     __amdgpu_buffer_rsrc_t ra[P], rb[P];
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-        ra[p] = rows(as + p * plane_a + n0 * ldk, BN * ldk2);
-        rb[p] = rows(bs + p * plane_b + j0 * ldk, BM * ldk2);
+        ra[p] = rows(as + p * plane_a + n0 * ldk, BN * 64u * nsl);
+        rb[p] = rows(bs + p * plane_b + j0 * ldk, BM * 64u * nsl);
     }
     auto dma = [&](uint32_t s, op (*sa)[P][BN * LP_LDK], op (*sb)[P][BM * LP_LDK]) {
         auto piece = [&](__amdgpu_buffer_rsrc_t rs, uint32_t soff, op *dst) {
@@ -1183,6 +1228,8 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
         };
         constexpr int RA = BN / 16, RB = BM / 16; // pieces per slice and plane
         static_assert(RA % WAVES == 0 && RB % WAVES == 0, "pieces divide over the waves");
+        // piece r of slice sl: group r / 4, its physical rows 16 (r % 4) .. + 15
+        auto at = [&](uint32_t r, uint32_t sl) { return ((r >> 2) * nsl + sl) * 4096u + (r & 3u) * 1024u; };
 #pragma unroll
         for (int p = 0; p < P; ++p)
 #pragma unroll
@@ -1190,12 +1237,12 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
 #pragma unroll
                 for (int i = 0; i < RA / WAVES; ++i) {
                     uint32_t const r = (uint32_t)(wave + WAVES * i);
-                    piece(ra[p], (64u * (r >> 2) + (r & 3u)) * ldk2 + s * (64u * KS) + 64u * ks, &sa[ks][p][16 * r * LP_LDK]);
+                    piece(ra[p], at(r, s * KS + ks), &sa[ks][p][16 * r * LP_LDK]);
                 }
 #pragma unroll
                 for (int i = 0; i < RB / WAVES; ++i) {
                     uint32_t const r = (uint32_t)(wave + WAVES * i);
-                    piece(rb[p], (64u * (r >> 2) + (r & 3u)) * ldk2 + s * (64u * KS) + 64u * ks, &sb[ks][p][16 * r * LP_LDK]);
+                    piece(rb[p], at(r, s * KS + ks), &sb[ks][p][16 * r * LP_LDK]);
                 }
             }
     };
@@ -1206,7 +1253,7 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[jt][nt] = zero4();
 
-    v8 fa[2][P][NT], fb[2][P];
+    v8 fa[2][P][NT], fb[4][P];
     int const arow = 16 * NT * wn + lc, brow = 16 * JT * wm + lc;
     auto read_a = [&](int set, op (*sa)[P][BN * LP_LDK], int ks) {
 #pragma unroll
@@ -1220,10 +1267,14 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
         for (int p = 0; p < P; ++p)
             fb[set][p] = *reinterpret_cast<const v8 *>(&sb[ks][p][lds_at(brow + 16 * jt, lg)]);
     };
+    // NN stores want a lane's results along n (D[j][n], operand order B, A), TN
+    // stores along j (D[n][j], operand order A, B).
     auto products = [&](int sa, int sb, int jt) {
         auto step = [&](int pb, int pa) {
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[jt][nt] = L::mfma(fb[sb][pb], fa[sa][pa][nt], acc[jt][nt]);
+            for (int nt = 0; nt < NT; ++nt)
+                acc[jt][nt] = TSTORE ? L::mfma(fa[sa][pa][nt], fb[sb][pb], acc[jt][nt])
+                                     : L::mfma(fb[sb][pb], fa[sa][pa][nt], acc[jt][nt]);
         };
         if constexpr (P == 3) {
             step(1, 1);
@@ -1238,59 +1289,87 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
         step(0, 0);
     };
     uint32_t const ns = (uint32_t)(ldk / (32 * KS));
-    // Fragments of slice ks of a stage in buffer BUF sit in set ks % 2 (KS
-    // even) or BUF; the last MFMA group of a stage runs behind the barrier,
-    // while the next stage's first fragments are read.
-    auto stage = [&](auto buf_tag, uint32_t s, op (*sa)[P][BN * LP_LDK], op (*sb)[P][BM * LP_LDK],
-                     op (*na)[P][BN * LP_LDK], op (*nb_)[P][BM * LP_LDK]) {
-        constexpr int BUF = decltype(buf_tag)::value;
-        constexpr int S0 = KS % 2 == 0 ? 0 : BUF; // set of the stage's first slice; the other holds the carry
-        if (s + 1 < ns) dma(s + 1, na, nb_);
+    // Stage s (in buffer I = s mod NS): its first slice's fragments sit in set
+    // S0, the next one's in the other.  The barrier before it freed the buffer
+    // of stage s - 1, which takes stage s + NS - 1.
+    constexpr int PIECES = P * KS * (BM + BN) / 16 / WAVES; // DMA instructions of a wave per stage
+    auto stage = [&](auto tag, uint32_t s) __attribute__((always_inline)) {
+        constexpr int I = decltype(tag)::value;
+        constexpr int S0 = KS % 2 == 0 ? 0 : I % 2;
+        auto *const sa = buf_a(tag);
+        auto *const sb = buf_b(tag);
+        using Freed = std::integral_constant<int, I + NS - 1>;
+        bool const more = s + NS - 1 < ns;
+        if (more) dma(s + NS - 1, buf_a(Freed()), buf_b(Freed()));
+        // group g (row tile g mod JT of slice g / JT) has its B fragment in slot
+        // g mod 4, read two groups ahead; the last two run in the next stage
+        // (zeros ahead of the first one)
+        constexpr int G = KS * JT;
         read_a(S0, sa, 0);
         read_b(0, sb, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        products(S0 ^ 1, 1, JT - 1); // carried over (zeros ahead of the first stage)
+        products(S0 ^ 1, 2, JT - 2);
+        __builtin_amdgcn_sched_barrier(0);
+        read_b(1, sb, 0, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        products(S0 ^ 1, 3, JT - 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            int const set = KS % 2 == 0 ? ks & 1 : BUF;
-#pragma unroll
-            for (int jt = 0; jt < JT; ++jt) {
-                if (ks + 1 == KS && jt + 1 == JT) break;
-                if (jt + 1 < JT) {
-                    read_b((jt + 1) & 1, sb, ks, jt + 1);
-                } else {
-                    read_a(set ^ 1, sa, ks + 1);
-                    read_b(0, sb, ks + 1, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                products(set, jt & 1, jt);
-                __builtin_amdgcn_sched_barrier(0);
-            }
+        for (int g = 0; g + 2 < G; ++g) {
+            int const ahead = g + 2;
+            if (ahead % JT == 0) read_a(S0 ^ (ahead / JT & 1), sa, ahead / JT);
+            read_b(ahead & 3, sb, ahead / JT, ahead % JT);
+            __builtin_amdgcn_sched_barrier(0);
+            products(S0 ^ (g / JT & 1), g & 3, g % JT);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_s_waitcnt(0x0070); // vmcnt(0) lgkmcnt(0): the next stage is here, this one read
+        // the next stage is here (the DMA of the NS - 2 stages after it may
+        // stay in flight), this one read
+        constexpr int FLY = (NS - 2) * PIECES;
+        static_assert(FLY < 64, "vmcnt");
+        if (more) __builtin_amdgcn_s_waitcnt((FLY & 15) | (FLY >> 4) << 14 | 0x70);
+        else __builtin_amdgcn_s_waitcnt(0x0070);
         asm volatile("s_barrier" ::: "memory");
     };
-    static_assert(JT % 2 == 0 && (KS == 1 || KS % 2 == 0), "fragment sets alternate");
+    static_assert(JT % 4 == 0 && (KS == 1 || (KS % 2 == 0 && NS != 3)) && NS >= 2 && NS <= 4, "fragment sets alternate");
 #pragma unroll
     for (int p = 0; p < P; ++p) {
-        fb[1][p] = v8{};
+        fb[2][p] = fb[3][p] = v8{};
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) fa[1][p][nt] = v8{};
     }
     dma(0, sA0, sB0);
-    __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
-    asm volatile("s_barrier" ::: "memory");
-    uint32_t s = 0;
-    for (; s + 1 < ns; s += 2) {
-        stage(std::integral_constant<int, 0>(), s, sA0, sB0, sA1, sB1);
-        stage(std::integral_constant<int, 1>(), s + 1, sA1, sB1, sA0, sB0);
-    }
-    if (s < ns) {
-        stage(std::integral_constant<int, 0>(), s, sA0, sB0, sA1, sB1);
-        products(KS % 2 == 0 ? 1 : 0, 1, JT - 1);
+    if (NS > 2 && ns > 1) dma(1, buf_a(std::integral_constant<int, 1>()), buf_b(std::integral_constant<int, 1>()));
+    if (NS > 3 && ns > 2) dma(2, buf_a(std::integral_constant<int, 2>()), buf_b(std::integral_constant<int, 2>()));
+    if (ns >= NS - 1) {
+        constexpr int FLY = (NS - 2) * PIECES;
+        __builtin_amdgcn_s_waitcnt((FLY & 15) | (FLY >> 4) << 14 | 0x0F70);
     } else {
-        products(1, 1, JT - 1);
+        __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
+    }
+    asm volatile("s_barrier" ::: "memory");
+    // one trip: every buffer, an even number of stages
+    uint32_t s = 0;
+    auto trip = [&](auto... tags) {
+        for (; s + sizeof...(tags) <= ns; s += sizeof...(tags)) (stage(tags, s + decltype(tags)::value), ...);
+        ((s + decltype(tags)::value < ns ? stage(tags, s + decltype(tags)::value) : void()), ...);
+    };
+    constexpr int TRIP = NS == 3 && KS == 1 ? 6 : NS;
+    using std::integral_constant;
+    if constexpr (TRIP == 2)
+        trip(integral_constant<int, 0>(), integral_constant<int, 1>());
+    else if constexpr (TRIP == 4)
+        trip(integral_constant<int, 0>(), integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 3>());
+    else
+        trip(integral_constant<int, 0>(), integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 3>(),
+             integral_constant<int, 4>(), integral_constant<int, 5>());
+    int const set = KS % 2 == 0 || ns % 2 == 0 ? 1 : 0;
+    if (set) {
+        products(1, 2, JT - 2);
+        products(1, 3, JT - 1);
+    } else {
+        products(0, 2, JT - 2);
+        products(0, 3, JT - 1);
     }
     if constexpr (MODE == LP_FP16X2) {
         int const ce = exps[0] + exps[1];
@@ -1302,8 +1381,11 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
                 for (int r = 0; r < 4; ++r) acc[jt][nt][r] = ldexpf(acc[jt][nt][r], -ce);
     }
 
-    // A lane holds, for row tile jt and element r, row 64 (jt / 4) + 4 (4 lg + r)
-    // + jt % 4 of its wave's rows and the four adjacent columns 4 lc + nt.
+    // Tile t of a 64-row group holds its rows 4 x + t (x < 16), so the four
+    // tiles of a group give a lane four adjacent results.  NN: columns 4 lc ..
+    // + 3 of row 64 (jt / 4) + 4 (4 lg + r) + jt % 4; TN: rows 64 g + 4 lc ..
+    // + 3 of column 4 (4 lg + r) + nt.  Either way a wave instruction stores
+    // four segments of 256 contiguous bytes.
     // c_vec: the vectors of C are 16-byte aligned, else they are element-aligned.
     uint64_t const ncol0 = n0 + 16 * NT * wn + 4 * lc;
     uint64_t const jw = j0 + 16 * JT * wm;
@@ -1341,15 +1423,17 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
                 }
             }
     } else {
+        uint64_t const nw = n0 + 16 * NT * wn;
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-            if (ncol0 + nt >= ncols) continue;
-            float *crow = c + (ncol0 + nt) * m;
+        for (int nt = 0; nt < 4; ++nt)
 #pragma unroll
-            for (int g = 0; g < JT / 4; ++g)
+            for (int r = 0; r < 4; ++r) {
+                uint64_t const n = nw + 4 * (4 * lg + r) + nt;
+                if (n >= ncols) continue;
+                float *crow = c + n * m;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    uint64_t const j = jw + 64 * g + 4 * (4 * lg + r);
+                for (int g = 0; g < JT / 4; ++g) {
+                    uint64_t const j = jw + 64 * g + 4 * lc;
                     if (j + 4 <= m) {
                         store4(crow + j, f32x4{acc[4 * g][nt][r], acc[4 * g + 1][nt][r], acc[4 * g + 2][nt][r],
                                                acc[4 * g + 3][nt][r]});
@@ -1359,7 +1443,7 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS>:
                             if (j + t < m) stg<float>(crow + j + t, acc[4 * g + t][nt][r]);
                     }
                 }
-        }
+            }
     }
 }
 
@@ -1871,8 +1955,11 @@ ttm_status_t launch_lp(const Fold &f, const float *a, const float *b, float *c, 
 
 // ---- products over planes -----------------------------------------------------
 // Block shape: 64 x 128 (two waves) for at most 64 rows of B, else 128 x 128,
-// or 256 x 256 (eight waves, one block per CU) where at least one block per
-// compute unit of them remains.
+// or where at least one 256 x 256 block per compute unit remains the largest
+// wave tiles (128 x 64): one plane 128 x 256 in three stages, two blocks per CU
+// (A [999, 1001, 203], m = 333, BF16: 0.43 ms against 0.45-0.50 with 256 x 256,
+// whose stores nothing overlaps), two planes 256 x 256 in two stages, eight
+// waves.
 enum PlaneShape : int
 {
     PLANES_64 = 0,
@@ -1896,11 +1983,10 @@ PlaneGeom plane_geom(const Fold &f, int parts)
 {
     PlaneShape const sh = plane_shape(f, parts);
     PlaneGeom g;
-    g.bm = sh == PLANES_64 ? 64 : sh == PLANES_128 ? 128 : 256;
+    g.bm = sh == PLANES_64 ? 64 : sh == PLANES_128 || parts == 1 ? 128 : 256;
     g.bn = sh == PLANES_256 ? 256 : 128;
     uint64_t const kq = parts == 1 ? 64 : 32; // contraction indices per stage
     g.ldk = (f.nq + kq - 1) / kq * kq;
-    if (f.w != 1) g.ldk = (g.ldk + 63) / 64 * 64; // the NN conversion writes 64 x 64 tiles
     uint64_t const ncols = f.outer * f.w;
     g.rows_a = (ncols + g.bn - 1) / g.bn * g.bn;
     g.rows_b = (f.m + g.bm - 1) / g.bm * g.bm;
@@ -1911,21 +1997,21 @@ PlaneGeom plane_geom(const Fold &f, int parts)
 }
 int mode_parts(ttm_precision_t prec) { return prec == TTM_PREC_BF16X3 ? 3 : prec == TTM_PREC_FP16X2 ? 2 : 1; }
 
-template <int MODE, int WM, int WN, int JT, int NT, int KS>
+template <int MODE, int WM, int WN, int JT, int NT, int KS, int NS>
 void launch_planes_shape(const Fold &f, const PlaneGeom &g, const typename Lp<MODE>::op *as,
                          const typename Lp<MODE>::op *bs, float *c, const int *exps, hipStream_t s)
 {
-    using S = PlaneTile<MODE, WM, WN, JT, NT, KS>;
+    using S = PlaneTile<MODE, WM, WN, JT, NT, KS, NS>;
     unsigned const nj = (unsigned)(g.rows_b / S::BM);
     unsigned const total = nj * (unsigned)(g.rows_a / S::BN);
     bool const ts = f.w == 1;
     int const c_vec = (reinterpret_cast<uintptr_t>(c) & 15u) == 0 && (ts ? f.m : f.w) % 4 == 0;
     uint64_t const ncols = f.outer * f.w;
     if (ts)
-        hipLaunchKernelGGL((k_planes<MODE, WM, WN, JT, NT, KS, true>), dim3(total), dim3(64 * WM * WN), 0, s, as,
+        hipLaunchKernelGGL((k_planes<MODE, WM, WN, JT, NT, KS, NS, true>), dim3(total), dim3(64 * WM * WN), 0, s, as,
                            g.plane_a, bs, g.plane_b, g.ldk, c, ncols, f.w, f.m, nj, total, c_vec, exps);
     else
-        hipLaunchKernelGGL((k_planes<MODE, WM, WN, JT, NT, KS, false>), dim3(total), dim3(64 * WM * WN), 0, s, as,
+        hipLaunchKernelGGL((k_planes<MODE, WM, WN, JT, NT, KS, NS, false>), dim3(total), dim3(64 * WM * WN), 0, s, as,
                            g.plane_a, bs, g.plane_b, g.ldk, c, ncols, f.w, f.m, nj, total, c_vec, exps);
 }
 
@@ -1948,20 +2034,22 @@ ttm_status_t launch_planes(const Fold &f, const float *a, const float *b, float 
     op *const bs = as + P * g.plane_a;
     int const *exps = nullptr;
     if constexpr (SCALED) exps = launch_scale_pass(f, a, b, sp, static_cast<char *>(ws) + planes_bytes, s);
-    unsigned const blocks_a =
-        (unsigned)(f.w == 1 ? (g.plane_a / 8 + 255) / 256 : g.rows_a / 64 * (g.ldk / 64));
-    unsigned const blocks_b = (unsigned)((g.plane_b / 8 + 255) / 256);
-    auto const convert = f.w == 1 ? k_planes_convert<MODE, true> : k_planes_convert<MODE, false>;
-    hipLaunchKernelGGL(convert, dim3(blocks_a + blocks_b), dim3(256), 0, s, a, as, ncols, f.w, g.rows_a, g.plane_a, b,
-                       bs, f.m, f.b_stride_j(), f.b_stride_l(), g.rows_b, g.plane_b, f.nq, g.ldk, blocks_a, exps);
+    unsigned const nsl = (unsigned)(g.ldk / 32);
+    auto blocks = [&](uint64_t rows, bool along) {
+        return (unsigned)(rows / 64) * ((nsl + (along ? 3 : 1)) / (along ? 4 : 2));
+    };
+    unsigned const blocks_a = blocks(g.rows_a, f.w == 1), blocks_b = blocks(g.rows_b, !f.b_colmajor);
+    hipLaunchKernelGGL(k_planes_convert<MODE>, dim3(blocks_a + blocks_b), dim3(256), 0, s, a, as, ncols, f.w, g.plane_a,
+                       b, bs, f.m, f.b_colmajor ? 0 : 1, g.plane_b, f.nq, nsl, blocks_a, exps);
     constexpr int KS = P == 1 ? 2 : 1;
     PlaneShape const sh = plane_shape(f, P);
     if (sh == PLANES_64) {
-        launch_planes_shape<MODE, 1, 2, 4, 4, KS>(f, g, as, bs, c, exps, s);
+        launch_planes_shape<MODE, 1, 2, 4, 4, KS, 2>(f, g, as, bs, c, exps, s);
     } else if (sh == PLANES_128) {
-        launch_planes_shape<MODE, 2, 2, 4, 4, KS>(f, g, as, bs, c, exps, s);
+        launch_planes_shape<MODE, 2, 2, 4, 4, KS, 2>(f, g, as, bs, c, exps, s);
     } else {
-        if constexpr (P < 3) launch_planes_shape<MODE, 2, 4, 8, 4, KS>(f, g, as, bs, c, exps, s);
+        if constexpr (P == 2) launch_planes_shape<MODE, 2, 4, 8, 4, KS, 2>(f, g, as, bs, c, exps, s);
+        else if constexpr (P == 1) launch_planes_shape<MODE, 1, 4, 8, 4, 1, 3>(f, g, as, bs, c, exps, s);
     }
     hipError_t const e = hipGetLastError();
     ws_release(ws, s);
@@ -2109,8 +2197,7 @@ std::string lowp_symbol(const Fold &f, ttm_precision_t prec, bool generic, bool 
     } else if (!lowp_supports(f, aligned)) {
         static const char *const shapes[] = {"1, 2, 4, 4", "2, 2, 4, 4", "2, 4, 8, 4"};
         int const parts = mode_parts(prec);
-        std::snprintf(buf, sizeof buf, "k_planes<%d, %s, %d, %s>", mode, shapes[plane_shape(f, parts)],
-                      parts == 1 ? 2 : 1, tn);
+        std::snprintf(buf, sizeof buf, "k_planes<%d, %s, %s>", mode, shapes[plane_shape(f, parts)], tn);
     } else {
         std::snprintf(buf, sizeof buf, "k_lowp<%d, %s, %d>", mode, tn, lp_block_rows(f));
     }
