@@ -64,6 +64,27 @@ def test_ragged_slice_takes_its_elements(cfg):
             assert kept == want and 0 <= start and start + vec <= m * nq
 
 
+@pytest.mark.parametrize("cfg", sorted({c[1:5] for c in gemm_configs() if c[6]}), ids=lambda c: "-".join(map(str, c)))
+def test_tn_stores_cover_a_block_once(cfg):
+    """The C[n][j] epilogue with swapped operands: every element of a BM x BN
+    block is stored by exactly one lane, whole vectors inside their rows."""
+    vec, JT, NT, WM = cfg
+    BM, BN = WM * 16 * JT, (4 // WM) * 16 * NT
+    for m, ncols in ((BM, BN), (BM - 1, BN - 3), (1, 1)):
+        seen = np.zeros((BN, BM), dtype=int)
+        for tid in range(256):
+            lane, wave = tid & 63, tid >> 6
+            lc, lr, wm, wn = lane & 15, lane >> 4, wave % WM, wave // WM
+            jr = wm * 16 * JT + JT * lc
+            for nt, r in itertools.product(range(NT), range(4)):
+                k = wn * 16 * NT + NT * (4 * lr + r if vec == 4 else 4 * r + lr) + nt
+                if k >= ncols:
+                    continue
+                n = JT if JT % vec == 0 and jr + JT <= m else max(0, min(JT, m - jr))
+                seen[k, jr:jr + n] += 1
+        assert np.all(seen[:ncols, :m] == 1) and seen.sum() == ncols * m
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype,nqs", [(np.float32, (95, 96, 97, 112, 127, 192, 193, 225)),
                                        (np.float64, (383, 384, 385, 399, 416, 433))])

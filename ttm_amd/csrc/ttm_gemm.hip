@@ -22,8 +22,8 @@
 // tile jt holds the rows {JT*x + jt : x < 16} and tile nt the columns
 // {NT*y + nt : y < 16}, so the JT (NT) fragment values a lane needs for one
 // k are adjacent in LDS and arrive with one vector read; and a lane's NT
-// results of one row are adjacent columns (NN: one 16-byte store) and its JT
-// results of one column adjacent rows (TN: one 16-byte store).
+// results of one row are adjacent columns (NN: one 16-byte store) or, with
+// the operands swapped, its JT results of one column adjacent rows (TN).
 //
 // MFMA lane conventions (16x16x4, lane = 16*lr + lc): srcA holds
 // Afrag[lc][lr], srcB holds Bfrag[lr][lc], accumulator element r holds
@@ -571,6 +571,10 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     int const a_off = wn * 16 * NT + NT * lc; // this lane's columns within the At tile
     int const b_off = wm * 16 * JT + JT * lc; // this lane's rows within the B tile
 
+    // Operand order: D[j][n] (a lane's results run along n) or, for the C[n][j]
+    // stores, D[n][j] (along j); the sums are the same bits either way.
+    auto mma = [](Acc &d, T bj, T an) { d = TSTORE ? Gt::mfma(an, bj, d) : Gt::mfma(bj, an, d); };
+
     uint64_t const nslices = (nq + BK - 1) / BK;
     // The products of one slice from LDS buffer buf.
     auto multiply = [&](int buf) {
@@ -583,7 +587,7 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
 #pragma unroll
             for (int jt = 0; jt < JT; ++jt)
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc[jt][nt] = Gt::mfma(fa[jt], fb[nt], acc[jt][nt]);
+                for (int nt = 0; nt < NT; ++nt) mma(acc[jt][nt], fa[jt], fb[nt]);
         }
     };
     using I0 = std::integral_constant<int, 0>;
@@ -662,7 +666,7 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
 #pragma unroll
         for (int jt = jt0; jt < jt1; ++jt)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[jt][nt] = Gt::mfma(fa[set][jt], fb[set][nt], acc[jt][nt]);
+            for (int nt = 0; nt < NT; ++nt) mma(acc[jt][nt], fa[set][jt], fb[set][nt]);
     };
     // Slice s (in LDS buffer BUF, its first fragments in set 0).  LOAD: load
     // slice s + 1 + PF into the registers that the store of slice s + 1 frees;
@@ -818,33 +822,38 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                 }
             }
     } else {
-        // one column (row k of C), JT adjacent rows j
+        // Element r of tile nt is column NT * acc_row(lr, r) + nt of the wave's,
+        // and lane lc holds its JT adjacent rows JT * lc ..: a wave instruction
+        // stores four rows of C, up to 16 JT consecutive elements of each (with
+        // the operands the other way round it stored 64 pieces of 16 bytes, 64
+        // bytes apart: the order-5 tensor 32x24x40x16x48 with q fastest, m = 64,
+        // float32 130 -> 76 us, A [300, 1000, 500] x_1, m = 101, 485 -> 360 us).
+        uint64_t const jr = j0 + wm * 16 * JT + JT * lc;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            uint64_t const k = ncol0 + nt;
-            if (k >= ncols) continue;
-            T *crow = c + k * m;
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                uint64_t const jr = j0 + wm * 16 * JT + JT * Gt::acc_row(lr, r);
+                uint64_t const k = n0 + wn * 16 * NT + NT * Gt::acc_row(lr, r) + nt;
+                if (k >= ncols) continue;
+                T *crow = c + k * m + jr;
                 if constexpr (JT % VEC == 0) {
-                    if (c_vec && jr + JT <= m) {
+                    if (jr + JT <= m) {
 #pragma unroll
                         for (int jt = 0; jt < JT; jt += VEC) {
                             V o;
 #pragma unroll
                             for (int x = 0; x < VEC; ++x) o[x] = acc[jt + x][nt][r];
-                            if (nt_c) stg_nt<V>(crow + jr + jt, o);
-                            else stg<V>(crow + jr + jt, o);
+                            if (!c_vec) stg<typename Gt::vec_u>(crow + jt, o);
+                            else if (nt_c) stg_nt<V>(crow + jt, o);
+                            else stg<V>(crow + jt, o);
                         }
                         continue;
                     }
                 }
 #pragma unroll
                 for (int jt = 0; jt < JT; ++jt)
-                    if (jr + jt < m) stg<T>(crow + jr + jt, acc[jt][nt][r]);
+                    if (jr + jt < m) stg<T>(crow + jt, acc[jt][nt][r]);
             }
-        }
     }
 }
 

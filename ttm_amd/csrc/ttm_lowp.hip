@@ -510,7 +510,8 @@ __device__ __forceinline__ void lowp_tile(const float *__restrict__ a, const flo
             // back to back)
             auto step = [&](int pb, int pa) {
 #pragma unroll
-                for (int nt = 0; nt < NTL; ++nt) acc[jt][nt] = L::mfma(fb[pb], fa[pa][nt], acc[jt][nt]);
+                for (int nt = 0; nt < NTL; ++nt)
+                    acc[jt][nt] = TSTORE ? L::mfma(fa[pa][nt], fb[pb], acc[jt][nt]) : L::mfma(fb[pb], fa[pa][nt], acc[jt][nt]);
             };
             if constexpr (P == 3) {
                 step(1, 1);
@@ -757,48 +758,35 @@ __device__ __forceinline__ void lowp_tile(const float *__restrict__ a, const flo
                         if (ncol0 + nt < ncols) stg<float>(cb + j * w + nt, acc[jt][nt][r]);
                 }
             }
-    } else if constexpr (COLSPLIT) {
-        // C[n][j]: MFMA tile nt of wave w reads physical A rows 32 w + 16 nt + lc,
-        // i.e. column 64 (w / 2) + 4 lc + 2 (w % 2) + nt; its row tile jt reads
-        // physical B rows 16 jt + lc, so accumulator element r of tile jt is
-        // row 4 (4 lg + r) + jt: the four tiles give four consecutive rows
-#pragma unroll
-        for (int nt = 0; nt < NTL; ++nt) {
-            uint64_t const k = n0 + 64 * (wave >> 1) + 4 * lc + 2 * (wave & 1) + nt;
-            if (k >= ncols) continue;
-            float *crow = c + k * m;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                uint64_t const jr = j0 + 4 * (4 * lg + r);
-                if ((m & 3) == 0 && jr + 4 <= m) {
-                    f32x4 o = {acc[0][nt][r], acc[1][nt][r], acc[2][nt][r], acc[3][nt][r]};
-                    stg<f32x4>(crow + jr, o);
-                } else {
-#pragma unroll
-                    for (int jt = 0; jt < 4; ++jt)
-                        if (jr + jt < m) stg<float>(crow + jr + jt, acc[jt][nt][r]);
-                }
-            }
-        }
     } else {
+        // C[n][j], operands swapped (D[n][j]): element r of tile nt is A row x =
+        // 4 lg + r of the tile, i.e. column 4 x + nt of the wave's 64 (COLSPLIT:
+        // tile nt of wave w reads physical rows 32 w + 16 nt + x, column
+        // 64 (w / 2) + 4 x + 2 (w % 2) + nt), and lane lc holds rows 4 lc .. + 3
+        // of the wave's 64: a wave instruction stores four rows of C, 256
+        // consecutive bytes of each (with the operands the other way round 64
+        // pieces of 16 bytes: A 1024x1024x512, q fastest, BF16 m = 800 2.14 ->
+        // 1.98 ms, FP16X2 m = 1024 3.92 -> 3.62 ms, BF16X3 5.44 -> 5.23 ms).
+        static_assert(JTL == 4, "four adjacent rows");
+        uint64_t const jr = j0 + (COLSPLIT ? 0 : wm * 64) + 4 * lc;
+        uint64_t const nw = n0 + (COLSPLIT ? 64 * (wave >> 1) + 2 * (wave & 1) : 64 * wn);
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) {
-            uint64_t const k = ncol0 + nt;
-            if (k >= ncols) continue;
-            float *crow = c + k * m;
+        for (int nt = 0; nt < NTL; ++nt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                uint64_t const jr = j0 + wm * 64 + 4 * (4 * lg + r);
-                if ((m & 3) == 0 && jr + 4 <= m) {
+                uint64_t const k = nw + 4 * (4 * lg + r) + nt;
+                if (k >= ncols) continue;
+                float *crow = c + k * m;
+                if (jr + 4 <= m) {
                     f32x4 o = {acc[0][nt][r], acc[1][nt][r], acc[2][nt][r], acc[3][nt][r]};
-                    stg<f32x4>(crow + jr, o);
+                    if ((m & 3) == 0) stg<f32x4>(crow + jr, o);
+                    else stg<f32x4u>(crow + jr, o);
                 } else {
 #pragma unroll
                     for (int jt = 0; jt < 4; ++jt)
                         if (jr + jt < m) stg<float>(crow + jr + jt, acc[jt][nt][r]);
                 }
             }
-        }
     }
 }
 
