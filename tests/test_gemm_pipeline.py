@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 import refcases as rc
-from test_tile_bounds_cpu import gemm_configs
+from test_tile_bounds_cpu import Bounds, gemm_configs, gemm_problems, gemm_tile_accesses
 
 
 def _shift_mask(v, d, nvalid, zero=None):
@@ -83,6 +83,57 @@ def test_tn_stores_cover_a_block_once(cfg):
                 n = JT if JT % vec == 0 and jr + JT <= m else max(0, min(JT, m - jr))
                 seen[k, jr:jr + n] += 1
         assert np.all(seen[:ncols, :m] == 1) and seen.sum() == ncols * m
+
+
+@pytest.mark.parametrize("vec,NT,WM", [(4, 4, 1), (4, 4, 2), (2, 2, 1), (2, 4, 2)])
+@pytest.mark.parametrize("view", ["TN", "NN", "PAD"])
+def test_48_and_96_row_tiles_in_bounds(vec, NT, WM, view):
+    JT, BK = 3, 16
+    tn, pad = view == "TN", view == "PAD"
+    BM, BN = WM * 16 * JT, (4 // WM) * 16 * NT
+    for outer, nq, w, m in gemm_problems(vec, tn, BM, BN, BK, pad):
+        wp = 1 if tn else (w + vec - 1) // vec * vec
+        ncols = outer if tn else outer * wp
+        nj, nn = (m + BM - 1) // BM, (ncols + BN - 1) // BN
+        a_vec = (nq % vec == 0) if tn else (w % vec == 0 and not pad)
+        c_vec = (m % vec == 0) if tn else (w % vec == 0 and not pad)
+        for bcol, (jb, nb) in itertools.product((True, False), {(0, 0), (nj - 1, nn - 1)}):
+            chk = Bounds({"a": outer * nq * w, "b": m * nq, "c": outer * m * w})
+            gemm_tile_accesses(chk, vec, JT, NT, WM, BK, "TN" if tn else "NN", bcol, pad, ncols=ncols, nq=nq, ld=nq,
+                               w=w, wp=wp, m=m, j0=jb * BM, n0=nb * BN, flags=int(a_vec) | 2 * int(c_vec) | 8, a_off=0,
+                               b_off=0, c_off=0, a_len=0 if tn else (ncols // wp) * nq * w)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,ms", [(np.float32, (33, 47, 48, 65, 95, 96, 190, 288)), (np.float64, (33, 48, 90, 480))])
+def test_48_and_96_row_tiles_vs_fp64(gpu, oracle, dtype, ms):
+    import torch
+    import ttm_amd
+    tdt = torch.float32 if dtype == np.float32 else torch.float64
+    rng = np.random.default_rng(72)
+    for m, (na, pia, q) in itertools.product(ms, (([40, 300], [1, 2], 1), ([401, 260], [1, 2], 1), ([260, 41], [1, 2], 2),
+                                                  ([131, 400, 2], [1, 2, 3], 2))):
+        nq = na[q - 1]
+        wa = rc.dense_strides(na, pia)
+        nc = list(na)
+        nc[q - 1] = m
+        wc = rc.dense_strides(nc, pia)
+        a = rng.uniform(-1, 1, int(np.prod(na))).astype(dtype)
+        b = rng.uniform(-1, 1, m * nq).astype(dtype)
+        label = f"{np.dtype(dtype).name} {na} q={q} m={m}"
+        print(label, flush=True)
+        n = int(np.prod(nc))
+        C = torch.full((n + 4096,), float("nan"), dtype=tdt, device=gpu)
+        ttm_amd.force_kernel("gemm")
+        ttm_amd.ttm_raw(q, len(na), torch.from_numpy(a).to(gpu), na, wa, pia, torch.from_numpy(b).to(gpu), [m, nq], [2, 1],
+                        C[:n], nc, wc)
+        torch.cuda.synchronize()
+        sym = ttm_amd.last_kernel()[0]
+        assert ", 3, 4, " in sym or ", 3, 2, " in sym, (label, sym)
+        c = C.cpu().numpy()
+        assert np.all(np.isnan(c[n:])), label
+        err = rc.normwise_error(c[:n], oracle.ttm_brute_f64(q, a, na, wa, b, m, False, nc, wc), a, b)
+        assert err <= 4 * nq * rc.eps(dtype), (label, sym, err)
 
 
 @pytest.mark.gpu

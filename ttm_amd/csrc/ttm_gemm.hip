@@ -52,6 +52,7 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 // global_load_dwordx4).
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef float f32x3u __attribute__((ext_vector_type(3), aligned(4)));
 
 template <class T>
 struct G;
@@ -301,8 +302,10 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     // wave (little matrix work per slice to hide a load behind: the loads of
     // slice s + 2 are issued while slice s is multiplied) whose slice is at
     // most five vectors per thread, or the 16-row TN tile of one product; one
-    // otherwise (larger sets would spill in the grouped kernels).
-    constexpr int PF = (JT <= 2 && (A_PER + B_PER <= 5 || (VIEW == VIEW_TN && JT == 1))) ? 2 : 1;
+    // otherwise (larger sets would spill in the grouped kernels).  The 48-row
+    // pipelined tiles take two as well (A 1024x1024x512, m = 48: float32 546 ->
+    // 532 us NN, float64 1024 -> 990 us TN); at 64 rows it changed nothing.
+    constexpr int PF = (PIPE && WAVES_M == 1 && JT == 3) ? 2 : (JT <= 2 && (A_PER + B_PER <= 5 || (VIEW == VIEW_TN && JT == 1))) ? 2 : 1;
     V ra[PF][A_PER], rb[PF][B_PER];
     // Guarded slices: shift d and count nvalid of each vector (d | nvalid << 8),
     // applied when the slice is stored so that no load is waited for early.
@@ -850,6 +853,19 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                         continue;
                     }
                 }
+                if constexpr (JT == 3 && sizeof(T) == 4) {
+                    if (jr + 3 <= m) {
+                        stg<f32x3u>(crow, f32x3u{acc[0][nt][r], acc[1][nt][r], acc[2][nt][r]});
+                        continue;
+                    }
+                }
+                if constexpr (JT == 3 && sizeof(T) == 8) {
+                    if (jr + 3 <= m) {
+                        stg<f64x2u>(crow, f64x2u{acc[0][nt][r], acc[1][nt][r]});
+                        stg<T>(crow + 2, acc[2][nt][r]);
+                        continue;
+                    }
+                }
 #pragma unroll
                 for (int jt = 0; jt < JT; ++jt)
                     if (jr + jt < m) stg<T>(crow + jt, acc[jt][nt][r]);
@@ -1004,10 +1020,23 @@ Config pick_config(const Fold &f, bool is_double)
     // wave per SIMD), the 32-row one 75 KB (two); with 128 columns 50 / 42 KB
     // and 167 / 146 registers, three blocks per CU
     if (is_double && f.m > 16 && f.m <= 32) return {2, 2, 1, 16};
+    // 33..48 rows: three row tiles instead of four, a quarter less matrix work
+    // (A 1024x1024x512, m = 48: float32 NN 636 -> 550 us, TN 720 -> 605 us,
+    // float64 1.15 -> 1.03 ms)
+    if (is_double && f.m > 32 && f.m <= 48) return {3, 2, 1, 16};
     if (is_double && f.m > 16 && f.m <= 64) return {4, 2, 1, 16};
     if (f.m <= 16) return {1, 4, 1, 16};
     if (f.m <= 32) return {2, 4, 1, 16};
+    if (f.m <= 48) return {3, 4, 1, 16};
     if (f.m <= 64) return {4, 4, 1, 16};
+    // 96-row blocks where they save enough padded rows and the last one is at
+    // least half full: m <= 96, 145..192, 257..288, ... (A 1024x1024x128, float32: m = 96 282 -> 240 us, m = 190
+    // 525 -> 444, m = 280 760 -> 640; float64 m = 96 507 -> 403 us); with a
+    // sixteenth saved the 128-row blocks' fewer loads weigh more in float32
+    // (m = 960: 1.91 against 2.01 ms), less in float64 (m = 480: 1.90 against
+    // 1.81 ms)
+    uint64_t const rows96 = (f.m + 95) / 96 * 96, rows128 = (f.m + 127) / 128 * 128;
+    if (rows96 * (is_double ? 17 : 18) < rows128 * 16 && rows96 - f.m < 48) return {3, 4, 2, 16};
     return {4, 4, 2, 16};
 }
 
@@ -1125,9 +1154,15 @@ void launch_layout(const Fold &f, const Geom &g, const Split &sp, unsigned flags
                 }
             }
             if (cfg.jt == 2) launch_cfg<T, 2, 2, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
+            else if (cfg.jt == 3) launch_cfg<T, 3, 2, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
             else launch_cfg<T, 4, 2, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
             return;
         }
+    }
+    if (cfg.jt == 3) {
+        if (cfg.waves_m == 2) launch_cfg<T, 3, 4, 2, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
+        else if constexpr (sizeof(T) == 4) launch_cfg<T, 3, 4, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
+        return;
     }
     if (cfg.jt == 1) launch_cfg<T, 1, 4, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
     else if (cfg.jt == 2) launch_cfg<T, 2, 4, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
