@@ -138,6 +138,25 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_product_entries = {}
+
+
+def product_entry(is_double: bool, precision: int):
+    """The device product entry as a prototype that takes the metadata arrays
+    by address (seven of them can share one ctypes array: building and
+    converting them one by one is most of a small call's host time)."""
+    L = lib()
+    key = (is_double, precision != 0)
+    entry = _product_entries.get(key)
+    if entry is None or entry[0] is not L:
+        u, ex = ctypes.c_uint, precision != 0 and not is_double
+        fn = L["ttm_dttm" if is_double else "ttm_sttm_ex" if ex else "ttm_sttm"]  # a new function object
+        fn.restype = ctypes.c_int
+        fn.argtypes = [u, u, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp] + ([ctypes.c_int] if ex else []) + [_vp]
+        entry = _product_entries[key] = (L, fn)
+    return entry[1]
+
+
 def check(status: int) -> None:
     if status != 0:
         raise TTMError(status, lib().ttm_last_error().decode())

@@ -57,6 +57,9 @@ def ttm(q, A, B, precision=None):
     pib = [2, 1]                  # row-major B
     Bc = B.contiguous() if torch is not None and isinstance(B, torch.Tensor) else np.ascontiguousarray(B)
     nb = list(B.shape)
+    if torch is not None and isinstance(A, torch.Tensor) and A.is_cuda and isinstance(B, torch.Tensor) \
+            and B.device == A.device:
+        return api.device_product(int(q), p, A, na, wa, pia, Bc, nb, pib, precision, None)
     nc = list(na)
     nc[q - 1] = nb[0]
     C = api.empty_like_layout(A, nc, pia)
