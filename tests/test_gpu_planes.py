@@ -54,6 +54,15 @@ def test_odd_extents_and_offsets_match_their_emulation(gpu, prec):
             assert sym.startswith(want), (na, q, m, sym)
 
 
+@pytest.mark.parametrize("prec", ["bf16", "fp16", "fp16x2", "bf16x3"])
+def test_few_aligned_blocks_match_their_emulation(gpu, prec):
+    """Aligned products of few blocks and long contractions: the planes' kernels
+    for one and two planes, the fused tiles for three."""
+    for na, pia, q, m in (([256, 300], [1, 2], 1, 65), ([1000, 129], [1, 2], 1, 256), ([132, 260], [1, 2], 2, 130)):
+        sym = _run(gpu, na, pia, q, m, m == 256, prec, 0)
+        assert sym.startswith("k_lowp<" if prec == "bf16x3" else "k_planes<"), (na, q, m, sym)
+
+
 @pytest.mark.parametrize("prec", ["bf16", "fp16x2"])
 def test_chip_filling_blocks_match_their_emulation(gpu, prec):
     for na, pia, q, m in BIG:

@@ -732,7 +732,7 @@ const char *kernel_name(Kernel k)
     return (i >= 0 && i < static_cast<int>(Kernel::count)) ? k_kernel_names[i] : "none";
 }
 
-std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision_t prec, bool aligned)
+std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision_t prec, bool aligned, int lowp)
 {
     std::string const t = is_double ? "double" : "float";
     std::string const jt = std::to_string(pick_jt(f.m));
@@ -753,8 +753,9 @@ std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision
     }
     case Kernel::gemm: return gemm_symbol(f, is_double, aligned);
     case Kernel::skinny: return skinny_symbol(f, is_double);
-    case Kernel::lowp: return lowp_symbol(f, prec, false, aligned);
-    case Kernel::lowp_generic: return lowp_symbol(f, prec, true, aligned);
+    case Kernel::lowp:
+        return lowp_symbol(f, prec, lowp >= 0 ? static_cast<LowpRoute>(lowp) : lowp_route(f, prec, aligned));
+    case Kernel::lowp_generic: return lowp_symbol(f, prec, LowpRoute::generic);
     default: return "";
     }
 }
@@ -771,7 +772,7 @@ Kernel choose_kernel(const Fold &f, bool is_double, ttm_precision_t prec, bool a
 {
     if (prec != TTM_PREC_DEFAULT) {
         if (is_double || prec > TTM_PREC_FP16X2) return Kernel::none;
-        bool const lp_ok = lowp_supports(f, aligned) || lowp_any_supports(f, prec);
+        bool const lp_ok = lowp_route(f, prec, aligned) != LowpRoute::generic;
         if (force == Kernel::generic || force == Kernel::lowp_generic || !lp_ok) return Kernel::lowp_generic;
         return Kernel::lowp;
     }
@@ -845,17 +846,22 @@ ttm_status_t launch_f32(const Fold &f, const float *a, const float *b, float *c,
     }
     bool const ac_aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(c)) & 15u) == 0;
     if (k == Kernel::lowp || k == Kernel::lowp_generic) {
-        bool generic = k == Kernel::lowp_generic;
+        LowpRoute route = k == Kernel::lowp_generic ? LowpRoute::generic : lowp_route(f, prec, aligned);
         // without room for the converted operands, or while the stream is
-        // captured (no allocation there): one thread per element
-        bool const any = !generic && !lowp_supports(f, aligned);
-        if (any && (!lowp_any_fits(f, prec) || (!scratch_bound() && stream_capturing(stream)))) generic = true;
-        ttm_status_t st = launch_lowp(f, a, b, c, prec, stream, generic);
-        if (any && !generic && st == TTM_ERR_ALLOC) {
-            generic = true;
-            st = launch_lowp(f, a, b, c, prec, stream, true);
+        // captured (no allocation of that size there): the other kernels
+        LowpRoute const other = lowp_supports(f, aligned) ? LowpRoute::tile : LowpRoute::generic;
+        if (route == LowpRoute::planes &&
+            (!lowp_planes_fit(f, prec) || (!scratch_bound() && stream_capturing(stream))))
+            route = other;
+        ttm_status_t st = launch_lowp(f, a, b, c, prec, stream, route);
+        if (route == LowpRoute::planes && st == TTM_ERR_ALLOC) {
+            route = other;
+            st = launch_lowp(f, a, b, c, prec, stream, route);
         }
-        if (info) *info = LaunchInfo{generic ? Kernel::lowp_generic : Kernel::lowp, 1, aligned};
+        if (info) {
+            *info = LaunchInfo{route == LowpRoute::generic ? Kernel::lowp_generic : Kernel::lowp, 1, aligned};
+            info->lowp = static_cast<int>(route);
+        }
         return st;
     }
     if (want_splits == 0) want_splits = tuned_splits(k, f, false);

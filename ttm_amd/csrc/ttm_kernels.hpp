@@ -41,8 +41,10 @@ Kernel kernel_from_name(const char *name);
 Kernel choose_kernel(const Fold &f, bool is_double, ttm_precision_t prec, bool aligned, Kernel force);
 
 // Template instance of the family's kernel for a fold (as profilers print it);
-// `aligned`: A, B and C 16-byte aligned (selects the NN tile without padding).
-std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision_t prec, bool aligned = true);
+// `aligned`: A, B and C 16-byte aligned (selects the NN tile without padding);
+// lowp: the LowpRoute that ran (-1: the one the planner picks).
+std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision_t prec, bool aligned = true,
+                          int lowp = -1);
 
 // Contraction splits a launch of family k runs with: `want` (0: the cached
 // tuning of the fold's class, else the family's own choice), clamped by the
@@ -55,6 +57,7 @@ struct LaunchInfo
     Kernel kernel = Kernel::none;
     unsigned splits = 1;
     bool aligned = true;
+    int lowp = -1; // LowpRoute of a reduced-precision product
 };
 
 // Launch the product on `stream`; returns TTM_SUCCESS or TTM_ERR_HIP.

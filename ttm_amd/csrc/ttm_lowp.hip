@@ -2144,45 +2144,70 @@ bool lowp_supports(const Fold &f, bool aligned)
     return blocks < (1ull << 31);
 }
 
-bool lowp_any_supports(const Fold &f, ttm_precision_t prec)
+namespace
 {
-    // Short contractions over few elements: one thread per element takes about
-    // 6 us + 0.4 us per contraction index (a serial chain), the conversions
-    // and the product 15-20 us ([63, K, 31] x_2, m = 33, bf16: 9.3 / 19 / 57 us
-    // at K = 9 / 33 / 129 against 21-23 us).
-    if (f.nq <= 24 && f.m * f.numel_a() <= (8u << 20)) return false;
-    // grid limits, 32-bit byte offsets within a block's rows, and a bound on
-    // what the padding to whole tiles may cost
+// The planes' kernels can run the fold (grid limits, 32-bit byte offsets within
+// a block's rows, and a bound on what the padding to whole tiles may cost).
+bool planes_support(const Fold &f, ttm_precision_t prec)
+{
     if (f.nq >= (1ull << 22)) return false;
     if (prec == TTM_PREC_FP8_E4M3)
         return fp8_bytes(f).total() <= kAnyMaxBytes && ((f.outer * f.w + 63) / 64) * ((f.m + 63) / 64) < (1ull << 31);
     PlaneGeom const g = plane_geom(f, mode_parts(prec));
-    // blocks of the conversions: 8 elements a thread, or 64 x 64 tiles
+    // blocks of the conversions: at least 2048 elements each
     return g.bytes <= kAnyMaxBytes && (g.rows_a / g.bn) * (g.rows_b / g.bm) < (1ull << 31) &&
            g.plane_a / 2048 + g.plane_b / 2048 + 2 < (1ull << 31);
 }
 
-bool lowp_any_fits(const Fold &f, ttm_precision_t prec)
+// Products the fused tiles could run but the planes' kernels run faster: more
+// than 64 rows of B, long contractions and at most one 128 x 128 block for
+// every CU (two planes: every second CU).  A block then walks its slices
+// alone on its CU, and the planes' loop, whose stages arrive by DMA while the
+// last one is multiplied, beats the fused one by more than the conversion
+// costs: A [2272, 4120] x_1, m = 240 (66 blocks) BF16 77 -> 46 us, FP16X2 115
+// -> 96; A [1024, 16384] x_1, m = 256 (256 blocks) BF16 48 -> 44 but FP16X2 75
+// -> 88; 640 blocks BF16 50 -> 58.  Three planes (BF16X3) gain nothing.
+bool planes_faster(const Fold &f, ttm_precision_t prec)
 {
-    if (!lowp_any_supports(f, prec)) return false;
+    if (prec == TTM_PREC_FP8_E4M3 || prec == TTM_PREC_BF16X3 || f.m <= 64 || f.nq < 256) return false;
+    uint64_t const blocks = ((f.m + 127) / 128) * ((f.outer * f.w + 127) / 128);
+    return blocks * (unsigned)mode_parts(prec) <= (uint64_t)device_cus();
+}
+} // namespace
+
+LowpRoute lowp_route(const Fold &f, ttm_precision_t prec, bool aligned)
+{
+    bool const tile = lowp_supports(f, aligned);
+    if (tile && !planes_faster(f, prec)) return LowpRoute::tile;
+    // Short contractions over few elements: one thread per element takes about
+    // 6 us + 0.4 us per contraction index (a serial chain), the conversions
+    // and the product 15-20 us ([63, K, 31] x_2, m = 33, bf16: 9.3 / 19 / 57 us
+    // at K = 9 / 33 / 129 against 21-23 us).
+    if (!tile && f.nq <= 24 && f.m * f.numel_a() <= (8u << 20)) return LowpRoute::generic;
+    if (planes_support(f, prec)) return LowpRoute::planes;
+    return tile ? LowpRoute::tile : LowpRoute::generic;
+}
+
+bool lowp_planes_fit(const Fold &f, ttm_precision_t prec)
+{
     size_t const room = scratch_available();
     if (prec == TTM_PREC_FP8_E4M3) return fp8_bytes(f).total() <= room;
     size_t const scale = prec == TTM_PREC_FP16X2 ? scale_pass(f, true).bytes() : 0;
     return plane_geom(f, mode_parts(prec)).bytes + 512 + scale <= room;
 }
 
-std::string lowp_symbol(const Fold &f, ttm_precision_t prec, bool generic, bool aligned)
+std::string lowp_symbol(const Fold &f, ttm_precision_t prec, LowpRoute route)
 {
     char const *tn = f.w == 1 ? "true" : "false";
     char buf[96];
-    if (generic) return "k_lowp_generic";
+    if (route == LowpRoute::generic) return "k_lowp_generic";
     int const mode = prec == TTM_PREC_BF16 ? LP_BF16
                      : prec == TTM_PREC_FP16 ? LP_FP16
                      : prec == TTM_PREC_FP16X2 ? LP_FP16X2
                                                : LP_BF16X3;
     if (prec == TTM_PREC_FP8_E4M3) {
         std::snprintf(buf, sizeof buf, "k_fp8<%s, %d>", tn, fp8_block_rows(f));
-    } else if (!lowp_supports(f, aligned)) {
+    } else if (route == LowpRoute::planes) {
         static const char *const shapes[] = {"1, 2, 4, 4", "2, 2, 4, 4", "2, 4, 8, 4"};
         int const parts = mode_parts(prec);
         std::snprintf(buf, sizeof buf, "k_planes<%d, %s, %s>", mode, shapes[plane_shape(f, parts)], tn);
@@ -2193,11 +2218,9 @@ std::string lowp_symbol(const Fold &f, ttm_precision_t prec, bool generic, bool 
 }
 
 ttm_status_t launch_lowp(const Fold &f, const float *a, const float *b, float *c, ttm_precision_t prec,
-                         hipStream_t s, bool generic)
+                         hipStream_t s, LowpRoute route)
 {
-    bool const aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) |
-                           reinterpret_cast<uintptr_t>(c)) & 15u) == 0;
-    bool const tile = !generic && lowp_supports(f, aligned);
+    bool const generic = route == LowpRoute::generic, tile = route == LowpRoute::tile;
     if (generic) {
         uint64_t const total = f.numel_c();
         uint64_t blocks = (total + 255) / 256;

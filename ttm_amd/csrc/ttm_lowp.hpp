@@ -16,19 +16,25 @@ namespace ttm_amd
 // either w == 1 with nq % 4 == 0 (TN view) or w % 4 == 0 (NN view).
 bool lowp_supports(const Fold &f, bool aligned);
 
-// True when the kernels over pre-converted operands can run the fold (any
-// extents, element-aligned buffers), and when their workspace also fits the
-// scratch region bound to this thread, if one is.
-bool lowp_any_supports(const Fold &f, ttm_precision_t prec);
-bool lowp_any_fits(const Fold &f, ttm_precision_t prec);
+// Kernels of a reduced-precision product: one thread per element (any shape
+// and alignment), the fused tiles (lowp_supports), or the kernels over
+// pre-converted operands (any extents, element-aligned buffers).
+enum class LowpRoute : int
+{
+    generic = 0,
+    tile,
+    planes
+};
+// Choice for a fold (`aligned`: A, B and C 16-byte aligned), and whether the
+// planes' workspace fits the scratch region bound to this thread, if one is.
+LowpRoute lowp_route(const Fold &f, ttm_precision_t prec, bool aligned);
+bool lowp_planes_fit(const Fold &f, ttm_precision_t prec);
 
-// Template instance launched for a fold and precision (as profilers print it);
-// `aligned`: A, B and C 16-byte aligned.
-std::string lowp_symbol(const Fold &f, ttm_precision_t prec, bool generic, bool aligned);
+// Template instance launched for a fold and precision (as profilers print it).
+std::string lowp_symbol(const Fold &f, ttm_precision_t prec, LowpRoute route);
 
-// `generic` selects the one-thread-per-element kernel (any shape/alignment).
 ttm_status_t launch_lowp(const Fold &f, const float *a, const float *b, float *c, ttm_precision_t prec,
-                         hipStream_t s, bool generic);
+                         hipStream_t s, LowpRoute route);
 
 // Grouped BF16X3 or FP16X2 launches of TT products (stages of multi-TTM
 // chains) in bm x 128 tiles, bm = 128 or 64 (products of at most 64 rows);
