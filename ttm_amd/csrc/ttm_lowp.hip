@@ -1658,15 +1658,23 @@ __global__ __launch_bounds__(256) void k_fp8_split_a_cols(const float *__restric
 }
 
 // The product over the quantized operands: BM rows of B x 64 columns of A
-// per block, slices of 128; both tiles are byte copies into LDS.
+// per block, slices of 128; both tiles are byte copies into LDS.  The operand
+// whose index is contiguous in C has its 64-row groups in the order of lds_row,
+// so that four MFMA tiles give a lane four adjacent results: NN (columns n; the
+// four waves split the rows) or TN (rows j, operands swapped; the waves split
+// the columns, two by two where there are 128 rows).  A wave instruction stores
+// four segments of 256 consecutive bytes, where single floats went out 64 bytes
+// a row (NN) or 16 apart (TN): A 1024x1024x512, m = 1024, q fastest 2.31 -> 1.77
+// ms, q = 2 1.90 -> 1.80 ms.
 template <bool TN, int BM>
 __global__ __launch_bounds__(256) void k_fp8(const unsigned char *__restrict__ qa, const unsigned char *__restrict__ sa,
                                              const unsigned char *__restrict__ qb, const unsigned char *__restrict__ sb,
                                              uint64_t ldq, float *__restrict__ c, uint64_t ncols, uint64_t nq,
-                                             uint64_t w, uint64_t m, unsigned nj, unsigned total)
+                                             uint64_t w, uint64_t m, unsigned nj, unsigned total, int c_vec)
 {
     constexpr int BN = 64, BK = 128;
-    constexpr int JT = BM / 32; // 16-row MFMA tiles per wave along j (2 x 2 waves)
+    constexpr int JT = TN ? 4 : BM / 64; // 16-row MFMA tiles per wave along j
+    constexpr int NT = TN ? BM / 64 : 4; // and along n
     constexpr int LDK = BK + 16; // bytes per row
     __shared__ __attribute__((aligned(16))) unsigned char sA[BN * LDK];
     __shared__ __attribute__((aligned(16))) unsigned char sB[BM * LDK];
@@ -1680,13 +1688,16 @@ __global__ __launch_bounds__(256) void k_fp8(const unsigned char *__restrict__ q
     int const tid = threadIdx.x;
     int const lane = tid & 63, wave = tid >> 6;
     int const lc = lane & 15, lg = lane >> 4;
-    int const wm = wave & 1, wn = wave >> 1;
+    // first row of B and column of A of the wave
+    int const wj = TN ? (BM == 128 ? 64 * (wave & 1) : 0) : wave * (BM / 4);
+    int const wc = TN ? (BM == 128 ? 32 * (wave >> 1) : 16 * wave) : 0;
+    auto place = [](int row, bool grouped) { return grouped ? lds_row(row) : row; };
 
-    f32x4 acc[JT][2];
+    f32x4 acc[JT][NT];
 #pragma unroll
     for (int x = 0; x < JT; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] = zero4();
+        for (int y = 0; y < NT; ++y) acc[x][y] = zero4();
 
     // A: the pre-quantized slice, 64 rows (columns n) x 128 bytes, and its
     // 64 x 4 scales, laid out as B's.  B: BM rows x 128 bytes (16-byte piece
@@ -1722,38 +1733,47 @@ __global__ __launch_bounds__(256) void k_fp8(const unsigned char *__restrict__ q
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             int const p = tid + 256 * i;
-            *reinterpret_cast<i32x4 *>(&sA[(p >> 3) * LDK + 16 * (p & 7)]) = pa[i];
+            *reinterpret_cast<i32x4 *>(&sA[place(p >> 3, !TN) * LDK + 16 * (p & 7)]) = pa[i];
         }
-        sAs[tid] = ea;
+        sAs[place(tid >> 2, !TN) * 4 + (tid & 3)] = ea;
 #pragma unroll
         for (int i = 0; i < BM / 32; ++i) {
             int const p = tid + 256 * i;
-            *reinterpret_cast<i32x4 *>(&sB[(p >> 3) * LDK + 16 * (p & 7)]) = pb[i];
+            *reinterpret_cast<i32x4 *>(&sB[place(p >> 3, TN) * LDK + 16 * (p & 7)]) = pb[i];
         }
 #pragma unroll
-        for (int i = 0; i < BM / 64; ++i) sBs[tid + 256 * i] = eb[i];
+        for (int i = 0; i < BM / 64; ++i) {
+            int const t = tid + 256 * i;
+            sBs[place(t >> 2, TN) * 4 + (t & 3)] = eb[i];
+        }
         __syncthreads();
         if (l0 + BK < nq) load(l0 + BK);
         // Fragments: the lane's 32 bytes are k = 16*lg + [0,16) and
         // k = 64 + 16*lg + [0,16); its scale covers k = 32*lg + [0,32).
-        int sbv[JT], sav[2];
+        auto fragment = [&](const unsigned char *s, int row) {
+            i32x4 const lo = *reinterpret_cast<const i32x4 *>(&s[row * LDK + 16 * lg]);
+            i32x4 const hi = *reinterpret_cast<const i32x4 *>(&s[row * LDK + 64 + 16 * lg]);
+            return i32x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+        };
+        int sbv[JT], sav[NT];
+        i32x8 fa[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            int const rn = wc + nt * 16 + lc;
+            fa[nt] = fragment(sA, rn);
+            sav[nt] = sAs[rn * 4 + lg];
+        }
 #pragma unroll
         for (int jt = 0; jt < JT; ++jt) {
-            int const rj = wm * (BM / 2) + jt * 16 + lc;
-            i32x4 lo = *reinterpret_cast<const i32x4 *>(&sB[rj * LDK + 16 * lg]);
-            i32x4 hi = *reinterpret_cast<const i32x4 *>(&sB[rj * LDK + 64 + 16 * lg]);
-            i32x8 fb = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+            int const rj = wj + jt * 16 + lc;
+            i32x8 const fb = fragment(sB, rj);
             sbv[jt] = sBs[rj * 4 + lg];
 #pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                int const rn = wn * 32 + nt * 16 + lc;
-                i32x4 alo = *reinterpret_cast<const i32x4 *>(&sA[rn * LDK + 16 * lg]);
-                i32x4 ahi = *reinterpret_cast<const i32x4 *>(&sA[rn * LDK + 64 + 16 * lg]);
-                i32x8 fa = {alo[0], alo[1], alo[2], alo[3], ahi[0], ahi[1], ahi[2], ahi[3]};
-                sav[nt] = sAs[rn * 4 + lg];
-                acc[jt][nt] =
-                    __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb, fa, acc[jt][nt], 0, 0, 0, sbv[jt], 0, sav[nt]);
-            }
+            for (int nt = 0; nt < NT; ++nt)
+                acc[jt][nt] = TN ? __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fa[nt], fb, acc[jt][nt], 0, 0, 0,
+                                                                                    sav[nt], 0, sbv[jt])
+                                 : __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb, fa[nt], acc[jt][nt], 0, 0, 0,
+                                                                                    sbv[jt], 0, sav[nt]);
         }
         // All fragments of the slice have been read before the next slice is
         // stored.  Keep the scale registers allocated until then, so that no
@@ -1762,29 +1782,61 @@ __global__ __launch_bounds__(256) void k_fp8(const unsigned char *__restrict__ q
         __syncthreads();
 #pragma unroll
         for (int jt = 0; jt < JT; ++jt) asm volatile("" ::"v"(sbv[jt]));
-        asm volatile("" ::"v"(sav[0]), "v"(sav[1]));
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) asm volatile("" ::"v"(sav[nt]));
     }
 
+    // c_vec: the vectors of C are 16-byte aligned, else they are element-aligned
+    auto store4 = [&](float *p, f32x4 o) {
+        if (c_vec) stg<f32x4>(p, o);
+        else stg<f32x4u>(p, o);
+    };
+    if constexpr (!TN) {
+        uint64_t const col = n0 + 4 * lc;
+        if (col >= ncols) return;
+        uint64_t k = col / w, i = col - k * w;
+        bool const whole = i + 4 <= w; // one slab (then all four columns are in range)
+        float *cb = c + k * m * w + i;
+        uint64_t off[4];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
-        uint64_t const col = n0 + wn * 32 + nt * 16 + lc;
-        if (col >= ncols) continue;
-        float *cbase;
-        uint64_t stride;
-        if constexpr (!TN) {
-            uint64_t const k = col / w;
-            cbase = c + k * m * w + (col - k * w);
-            stride = w;
-        } else {
-            cbase = c + col * m;
-            stride = 1;
+        for (int nt = 0; nt < 4; ++nt) {
+            uint64_t ii = i + nt, kk = 0;
+            while (ii >= w) {
+                ii -= w;
+                ++kk;
+            }
+            off[nt] = kk * m * w + ii - i;
         }
 #pragma unroll
         for (int jt = 0; jt < JT; ++jt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                uint64_t const jj = j0 + wm * (BM / 2) + jt * 16 + 4 * lg + r;
-                if (jj < m) cbase[jj * stride] = acc[jt][nt][r];
+                uint64_t const jj = j0 + wj + jt * 16 + 4 * lg + r;
+                if (jj >= m) continue;
+                if (whole) {
+                    store4(cb + jj * w, f32x4{acc[jt][0][r], acc[jt][1][r], acc[jt][2][r], acc[jt][3][r]});
+                } else {
+#pragma unroll
+                    for (int nt = 0; nt < 4; ++nt)
+                        if (col + nt < ncols) stg<float>(cb + jj * w + off[nt], acc[jt][nt][r]);
+                }
+            }
+    } else {
+        uint64_t const jj = j0 + wj + 4 * lc;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                uint64_t const col = n0 + wc + nt * 16 + 4 * lg + r;
+                if (col >= ncols) continue;
+                float *crow = c + col * m + jj;
+                if (jj + 4 <= m) {
+                    store4(crow, f32x4{acc[0][nt][r], acc[1][nt][r], acc[2][nt][r], acc[3][nt][r]});
+                } else {
+#pragma unroll
+                    for (int jt = 0; jt < 4; ++jt)
+                        if (jj + jt < m) stg<float>(crow + jt, acc[jt][nt][r]);
+                }
             }
     }
 }
@@ -2107,12 +2159,13 @@ ttm_status_t launch_fp8(const Fold &f, const float *a, const float *b, float *c,
     else
         hipLaunchKernelGGL(k_fp8_split_a_cols<ANY>, dim3((unsigned)split_a_blocks), dim3(256), 0, s, a, qa, sa, ncols,
                            f.nq, f.w, ldq, ldq / 128);
+    int const c_vec = (reinterpret_cast<uintptr_t>(c) & 15u) == 0 && (TN ? f.m : f.w) % 4 == 0;
     if (bm == 128)
         hipLaunchKernelGGL((k_fp8<TN, 128>), dim3(total), dim3(256), 0, s, qa, sa, qb, sb, ldq, c, ncols, f.nq, f.w,
-                           f.m, nj, total);
+                           f.m, nj, total, c_vec);
     else
         hipLaunchKernelGGL((k_fp8<TN, 64>), dim3(total), dim3(256), 0, s, qa, sa, qb, sb, ldq, c, ncols, f.nq, f.w,
-                           f.m, nj, total);
+                           f.m, nj, total, c_vec);
     hipError_t const e = hipGetLastError();
     ws_release(ws, s);
     if (e != hipSuccess) {
