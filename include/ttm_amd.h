@@ -119,6 +119,8 @@ ttm_status_t ttm_sttm_ex(unsigned q, unsigned p,
  * allocates nothing.  A product whose scratch would exceed the array is
  * rejected with TTM_ERR_ALLOC before any launch (ttm_last_error() gives the
  * bytes needed); contraction splits are limited so that their partials fit.
+ * Reduced-precision products that would convert A into padded planes first run
+ * on the kernels that need none when the planes do not fit.
  * Every call on one GPU shares that GPU's array: calls that overlap on one
  * GPU (other threads, other streams) race and must be serialised by the
  * caller. */
@@ -312,7 +314,8 @@ unsigned ttm_plan_splits(unsigned q, unsigned p, int is_double, const size_t *na
  * this thread ran ("" before any), and its contraction splits (0 before any). */
 const char *ttm_last_kernel(void);
 unsigned ttm_last_splits(void);
-/* Device memory held by the current device's workspace pool (bytes). */
+/* Device memory held by the current device's workspace pool (bytes); at most
+ * 8 GiB of freed workspace stay in it across a synchronization. */
 size_t ttm_workspace_bytes(void);
 /* Library version string. */
 const char *ttm_version(void);

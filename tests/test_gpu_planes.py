@@ -68,3 +68,18 @@ def test_chip_filling_blocks_match_their_emulation(gpu, prec):
     for na, pia, q, m in BIG:
         sym = _run(gpu, na, pia, q, m, False, prec, 1)
         assert sym.startswith("k_planes<"), sym
+
+
+def test_large_workspace_goes_back_to_the_device(gpu):
+    """Planes of more than 8 GiB (three of 2.0e9 elements): after a
+    synchronization the pool keeps at most 8 GiB of them."""
+    import torch
+    import ttm_amd
+    from ttm_amd import _lib
+    A = torch.zeros(801, 1201, 2003, device=gpu)
+    B = torch.ones(3, 1201, device=gpu)
+    C = ttm_amd.ttm(2, A, B, precision="bf16x3")
+    assert ttm_amd.last_kernel()[0].startswith("k_planes<")
+    torch.cuda.synchronize()
+    assert _lib.workspace_bytes() <= 8 << 30
+    assert not C.any()

@@ -20,6 +20,13 @@ thread_local size_t t_cap = 0;
 thread_local size_t t_used = 0;
 } // namespace
 
+// Freed workspace a pool keeps for later calls; what it holds beyond that goes
+// back to the device at the next synchronization.  Far above the workspaces of
+// ordinary products (planes of A 1024x1024x512 in BF16X3: 3.2 GB), a small
+// part of the device memory; the planes of one product may take up to 32 GiB,
+// whose allocation is small against the passes over them.
+constexpr uint64_t kPoolKeepBytes = 8ull << 30;
+
 hipMemPool_t workspace_pool()
 {
     int dev = 0;
@@ -36,7 +43,7 @@ hipMemPool_t workspace_pool()
         props.location.id = dev;
         hipMemPool_t pool = nullptr;
         if (hipMemPoolCreate(&pool, &props) != hipSuccess) return nullptr;
-        uint64_t keep = UINT64_MAX;
+        uint64_t keep = kPoolKeepBytes;
         if (hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) {
             (void)hipMemPoolDestroy(pool);
             return nullptr;
