@@ -1021,8 +1021,8 @@ Config pick_config(const Fold &f, bool is_double)
     // and 167 / 146 registers, three blocks per CU
     if (is_double && f.m > 16 && f.m <= 32) return {2, 2, 1, 16};
     // 33..48 rows: three row tiles instead of four, a quarter less matrix work
-    // (A 1024x1024x512, m = 48: float32 NN 636 -> 550 us, TN 720 -> 605 us,
-    // float64 1.15 -> 1.03 ms)
+    // (A 1024x1024x512, m = 48: float32 TN 614 -> 495 us in repeated calls; after
+    // a cache flush NN 636 -> 493 us, TN 720 -> 604 us, float64 1.15 -> 1.03 ms)
     if (is_double && f.m > 32 && f.m <= 48) return {3, 2, 1, 16};
     if (is_double && f.m > 16 && f.m <= 64) return {4, 2, 1, 16};
     if (f.m <= 16) return {1, 4, 1, 16};

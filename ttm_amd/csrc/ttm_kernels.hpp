@@ -19,8 +19,8 @@ enum class Kernel : int
     nn_stream,  // MFMA 16x16x4, w % vec == 0: streams A slabs along the contiguous block
     tn_stream,  // MFMA 16x16x4, w == 1: rows of A contiguous along the contraction mode
     gemm,       // LDS-staged MFMA blocks (ttm_gemm.hip), NN (w % vec == 0) or TN (w == 1) view
-    lowp,       // reduced-precision MFMA blocks (ttm_lowp.hip): bf16, fp16, bf16x3, fp8
-    lowp_generic, // reduced precision, one thread per element (any shape / alignment)
+    lowp,       // reduced-precision MFMA blocks (ttm_lowp.hip): bf16, fp16, fp16x2, bf16x3, fp8
+    lowp_generic, // reduced precision, one thread per element: short contractions, no room for planes
     skinny,     // vector-ALU stream of B (ttm_skinny.hip): w == 1 with at most eight columns
     count
 };
