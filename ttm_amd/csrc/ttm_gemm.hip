@@ -1111,16 +1111,48 @@ Split split_for(const Fold &f, bool is_double, const Geom &g, unsigned want)
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Blocks whose contraction (of one split) has at least this many indices take
-// the pipelined loop; its start and its last slices cost more than the plain
-// loop's.  Measured against the plain loop on [n, K, n] x_2 with n = 512:
-// float32 128-row blocks 1.04x at K = 96 and 0.97x at 64; 32- and 48-row
-// blocks 1.03x at 256 and 0.98x at 128; float64 128-row blocks 1.03x at 512,
-// 0.99-1.02x at 256 and 0.92x at 128 (256 registers, some spilled outside
-// the loop), 16- and 50-row blocks 1.07x at 515 and 0.99x at 255.
-bool gemm_pipelined(const Config &cfg, bool is_double, uint64_t len)
+// Whether a product's blocks run the pipelined loop.
+//
+// Its start and its last slices cost more than the plain loop's, so the
+// contraction (of one split) must be long.  Pipelined against plain, [w, K, n]
+// x_2 and [K, n] x_1, B in either order, 25 to 3000 blocks:
+//   float32 128 rows: K = 96 0.89-1.00, K = 64 0.96-1.09
+//           32 and 64 rows: K = 192 0.87-1.04, K = 128 0.92-1.06
+//           48 rows: K = 384 0.93-1.07, K = 256 0.94-1.13; 96 rows: K = 384
+//           0.95-1.06, K = 128 0.98-1.15: the whole grids of 900 and 3000
+//           blocks lose, most others gain (mean over 1000 random products of
+//           200 to 400000 columns with K between the threshold and 384: 48
+//           rows 0.92-0.96, 96 rows 0.89-0.94)
+//   float64 128 rows (256 registers, some spilled outside the loop): K = 384
+//           0.91-0.98, K = 256 0.92-1.03, K = 128 1.05-1.28
+//           16 to 96 rows: K = 384 0.81-1.05, K = 256 0.82-1.07
+//
+// Only interior blocks run it.  Where most blocks are guarded (rows past m of
+// a column-major B that no vector ends at, slab ends inside most blocks) a
+// block waits for each slice's loads in turn, and the pipelined kernels, with
+// more registers, have two blocks on a CU where the plain ones have three or
+// four: what counts is in how many rounds the grid runs.  B column-major,
+// K = 400, NN view: up to two blocks per CU 0.97-1.02, beyond 1.01-1.54
+// (float32, 17 to 95 rows, 3000 blocks: 1.06-1.38), except that both kernels
+// take two rounds for more than three and at most four blocks per CU, where
+// the float64 tiles of one row of waves and the 64-row float32 one gain
+// (0.78-0.97).  In the TN view guarded blocks lose for more than two and at
+// most three blocks per CU (0.96-1.25, float32 96 rows 1.43; elsewhere
+// 0.59-1.00), and so do blocks of 17..32 rows anywhere, bound by their loads
+// (K = 192..640, float32: 1.04-1.29, elsewhere 0.81-1.11).
+bool gemm_pipelined(const Fold &f, bool is_double, const Geom &g, const Split &sp)
 {
-    return len >= (is_double ? 384u : cfg.waves_m == 2 ? 96u : 192u);
+    Config const &cfg = g.cfg;
+    uint64_t const vec = is_double ? 2 : 4;
+    if (sp.kc < (is_double ? 384u : cfg.waves_m == 2 ? 96u : 192u)) return false;
+    uint64_t const blocks = (uint64_t)g.nj * g.nn * sp.splits, cus = (uint64_t)device_cus();
+    bool const one_round = blocks > 2 * cus && blocks <= 3 * cus; // for the plain kernels only
+    bool const two_rounds = blocks > 3 * cus && blocks <= 4 * cus; // for both
+    bool const guarded = (f.b_colmajor && f.m % vec != 0 && g.nj <= 2) ||
+                         (g.pad && f.w % vec != 0 && g.wp < 2 * (uint64_t)g.bn());
+    if (guarded && f.b_colmajor)
+        return g.tn ? !one_round : two_rounds && cfg.waves_m == 1 && (is_double || cfg.jt == 4);
+    return !(cfg.jt == 2 && one_round);
 }
 
 template <class T, int JT, int NT, int WM, int BK, bool TN, bool BCOL>
@@ -1134,7 +1166,7 @@ void launch_cfg(const Fold &f, const Geom &g, const Split &sp, unsigned flags, c
                            dim3(total, sp.splits), dim3(256), 0, s, a, b, c, g.ncols, f.nq, f.w, g.wp, f.m, g.nj,
                            total, sp.kc, c_split, flags);
     };
-    bool const pipe = gemm_pipelined(g.cfg, sizeof(T) == 8, sp.kc);
+    bool const pipe = gemm_pipelined(f, sizeof(T) == 8, g, sp);
     using Y = std::true_type;
     using N = std::false_type;
     if (!TN && g.pad) {
@@ -1184,14 +1216,15 @@ void launch_layout(const Fold &f, const Geom &g, const Split &sp, unsigned flags
 
 std::string gemm_symbol(const Fold &f, bool is_double, bool aligned)
 {
-    Config const cfg = pick_config(f, is_double);
     uint64_t const vec = is_double ? 2 : 4;
-    bool const pad = f.w != 1 && (!aligned || f.w % vec != 0);
+    Geom g = geom(f, is_double);
+    g.pad = !g.tn && (!aligned || f.w % vec != 0);
+    Config const &cfg = g.cfg;
     char buf[128];
     std::snprintf(buf, sizeof buf, "k_gemm<%s, %s, %d, %d, %d, %d, %s, %s, %s>", is_double ? "double" : "float",
-                  gemm_pipelined(cfg, is_double, split_for(f, is_double, geom(f, is_double), 0).kc) ? "true" : "false",
+                  gemm_pipelined(f, is_double, g, split_for(f, is_double, g, 0)) ? "true" : "false",
                   cfg.jt, cfg.nt, cfg.waves_m, cfg.bk, f.w == 1 ? "true" : "false", f.b_colmajor ? "true" : "false",
-                  pad ? "true" : "false");
+                  g.pad ? "true" : "false");
     return buf;
 }
 
