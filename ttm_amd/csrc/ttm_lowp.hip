@@ -29,6 +29,7 @@
 #include "ttm_lowp.hpp"
 #include "ttm_workspace.hpp"
 
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <mutex>
@@ -2212,6 +2213,55 @@ bool planes_support(const Fold &f, ttm_precision_t prec)
            g.plane_a / 2048 + g.plane_b / 2048 + 2 < (1ull << 31);
 }
 
+// Products the fused tiles cannot run: one thread per element against the
+// planes, by what each takes (microseconds; 10 000 products of 10^4 to 4 10^8
+// elements of A, n_q = 1 to 4001, m = 1 to 200, both views; the faster one was
+// taken to 1 % on average, a slower one by more than a tenth in 1 of 100).
+//
+// One thread per element: a serial chain of n_q steps, or about a microsecond
+// per 10^6 products (FP8, whose slices are read twice, two); with few rows of B
+// in the TN view the lanes of a wave read rows of A that lie apart, a line of
+// 128 bytes for each element once the rows are long.  The planes: three
+// launches, then the padded elements written, read and multiplied against 64
+// rows of B, and the stages one after the other.  With few rows
+// writing and reading A's padded planes alone takes 2 to 20 times what the
+// product takes (one thread per element against planes: BF16 [317, 33, 38237]
+// x_2, m = 1 0.52 / 1.05 ms, [5, 2 10^7] x_1, m = 2 0.30 / 1.75 ms, [3, 10^7]
+// x_1, m = 4 0.21 / 0.85 ms; but BF16X3 [711, 301, 140] x_2, m = 8 349 / 102 us).
+bool generic_faster(const Fold &f, ttm_precision_t prec)
+{
+    bool const fp8 = prec == TTM_PREC_FP8_E4M3, tn = f.w == 1;
+    // contractions from 25 on with as many rows as a block: the planes are at
+    // most 6 us behind, in the smallest products
+    if (f.m >= 63 && f.nq >= 25) return false;
+    double const m = (double)f.m, nq = (double)f.nq;
+    // FP8, FP16X2, BF16X3, one plane; NN and TN view
+    int const row = fp8 ? 0 : prec == TTM_PREC_FP16X2 ? 1 : prec == TTM_PREC_BF16X3 ? 2 : 3;
+    static constexpr double step[4][2] = {{.40, .20}, {.45, .28}, {.40, .20}, {.35, .20}};  // us per index of the chain
+    static constexpr double plane[4][2] = {{1.0, 0.9}, {1.6, 2.6}, {1.8, 3.2}, {0.9, 1.4}}; // us per 10^6 padded elements
+    static constexpr double stage[4] = {.005, .012, .029, .007};                            // us per index of the stages
+    static constexpr double products[4] = {1, 3, 6, 1};
+    double const line = std::min(1.0, nq / 32);
+    double const macs = m * (double)f.numel_a() * 1e-6;
+    double const work = macs * (fp8 ? (tn ? 1.4 : 2.0) : 1.0) * (0.9 + 2.2 / nq + (tn ? 9 * line * line / (m * m) : 0));
+    double const chain = step[row][tn] * nq;
+    double const generic = 6 + std::max(chain, work) + 0.5 * std::min(chain, work);
+    double rows_a, rows_b, ld;
+    if (fp8) {
+        rows_a = (double)((f.outer * f.w + 63) / 64 * 64);
+        rows_b = (double)((f.m + 63) / 64 * 64);
+        ld = (double)((f.nq + 127) / 128 * 128);
+    } else {
+        PlaneGeom const g = plane_geom(f, mode_parts(prec));
+        rows_a = (double)g.rows_a;
+        rows_b = (double)g.rows_b;
+        ld = (double)g.ldk;
+    }
+    double const planes = 16 + stage[row] * ld + rows_a * ld * 1e-6 * (plane[row][tn] + .002 * rows_b * products[row]) +
+                          0.6e-6 * (double)f.numel_c();
+    return generic < planes;
+}
+
 // Products the fused tiles could run but the planes' kernels run faster: more
 // than 64 rows of B, long contractions and at most one 128 x 128 block for
 // every CU (two planes: every second CU).  A block then walks its slices
@@ -2232,11 +2282,7 @@ LowpRoute lowp_route(const Fold &f, ttm_precision_t prec, bool aligned)
 {
     bool const tile = lowp_supports(f, aligned);
     if (tile && !planes_faster(f, prec)) return LowpRoute::tile;
-    // Short contractions over few elements: one thread per element takes about
-    // 6 us + 0.4 us per contraction index (a serial chain), the conversions
-    // and the product 15-20 us ([63, K, 31] x_2, m = 33, bf16: 9.3 / 19 / 57 us
-    // at K = 9 / 33 / 129 against 21-23 us).
-    if (!tile && f.nq <= 24 && f.m * f.numel_a() <= (8u << 20)) return LowpRoute::generic;
+    if (!tile && generic_faster(f, prec)) return LowpRoute::generic;
     if (planes_support(f, prec)) return LowpRoute::planes;
     return tile ? LowpRoute::tile : LowpRoute::generic;
 }
