@@ -1,6 +1,8 @@
 """Which kernels a reduced-precision product takes (ttm_lowp.hip, lowp_route):
 the fused tiles where its rows are whole vectors, otherwise one thread per
-element or the converted planes, by the estimate of generic_faster."""
+element or the converted planes, by the estimate of generic_faster; and the
+planes in place of the tiles for few column blocks (256 compute units, the
+planner's assumption without a device)."""
 import pytest
 
 from ttm_amd._lib import PRECISION_NAMES
@@ -30,4 +32,25 @@ ODD = [
 
 @pytest.mark.parametrize("na,q,m,prec,want", ODD)
 def test_odd_extents(ttmlib, na, q, m, prec, want):
+    assert _kernel(ttmlib, na, q, m, prec) == want
+
+
+# aligned, more than 64 rows of B and a long contraction: up to half a 128-column
+# block per compute unit (two planes: a quarter), fewer for narrow slabs
+FEW = [
+    ([512, 128 * 128], 1, 100, "bf16", "k_planes"), ([512, 128 * 129], 1, 100, "bf16", "k_lowp"),
+    ([512, 128 * 64], 1, 100, "fp16x2", "k_planes"), ([512, 128 * 65], 1, 100, "fp16x2", "k_lowp"),
+    ([16, 512, 8 * 128], 2, 100, "fp16", "k_planes"), ([16, 512, 8 * 129], 2, 100, "fp16", "k_lowp"),
+    ([8, 512, 16 * 96], 2, 100, "bf16", "k_planes"), ([8, 512, 16 * 97], 2, 100, "bf16", "k_lowp"),
+    ([4, 512, 32 * 64], 2, 100, "bf16", "k_planes"), ([4, 512, 32 * 65], 2, 100, "bf16", "k_lowp"),
+    ([4, 512, 32 * 32], 2, 100, "fp16x2", "k_planes"), ([4, 512, 32 * 33], 2, 100, "fp16x2", "k_lowp"),
+    # at most one block per compute unit, rows and columns together
+    ([512, 128 * 64], 1, 512, "bf16", "k_planes"), ([512, 128 * 65], 1, 512, "bf16", "k_lowp"),
+    ([512, 128 * 64], 1, 64, "bf16", "k_lowp"), ([252, 128 * 64], 1, 100, "bf16", "k_lowp"),
+    ([512, 128 * 64], 1, 100, "bf16x3", "k_lowp"),
+]
+
+
+@pytest.mark.parametrize("na,q,m,prec,want", FEW)
+def test_few_aligned_blocks(ttmlib, na, q, m, prec, want):
     assert _kernel(ttmlib, na, q, m, prec) == want

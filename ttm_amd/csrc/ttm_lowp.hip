@@ -2263,18 +2263,27 @@ bool generic_faster(const Fold &f, ttm_precision_t prec)
 }
 
 // Products the fused tiles could run but the planes' kernels run faster: more
-// than 64 rows of B, long contractions and at most one 128 x 128 block for
-// every CU (two planes: every second CU).  A block then walks its slices
-// alone on its CU, and the planes' loop, whose stages arrive by DMA while the
-// last one is multiplied, beats the fused one by more than the conversion
-// costs: A [2272, 4120] x_1, m = 240 (66 blocks) BF16 77 -> 46 us, FP16X2 115
-// -> 96; A [1024, 16384] x_1, m = 256 (256 blocks) BF16 48 -> 44 but FP16X2 75
-// -> 88; 640 blocks BF16 50 -> 58.  Three planes (BF16X3) gain nothing.
+// than 64 rows of B, long contractions and few blocks.  A block of the tiles
+// then walks its slices alone on its CU, and the planes' loop, whose stages
+// arrive by DMA while the last one is multiplied, beats it by more than the
+// conversion costs, which grows with the column blocks (128 columns).  4000
+// products of n_q = 256 to 20000 and m = 65 to 2000, planes against tiles, one
+// plane (two): 16-31 column blocks 0.52-0.56 (0.69-0.75), 64-79 0.66-0.77
+// (0.87-0.92), 112-127 0.80-0.88 (0.95-1.09), 160-191 1.02-1.13, 224 and more
+// 1.10-1.36.  The conversion of narrow slabs reads pieces of 4 w bytes: w = 8
+// and 12 64-79 0.78-0.83, 112-127 1.04-1.08 (two planes 40-47 0.90-0.94, 48 and
+// more 0.89-1.20); w = 4 48-63 0.89, 80-95 1.17, 160-191 1.75 (32-39 0.86, 48-63
+// 1.11).  A [2272, 4120] x_1, m = 240 BF16 77 -> 45 us, FP16X2 115 -> 92; A
+// [4, 8192, 6741] x_2, m = 96 (211) FP16 283 against 696.  At most one 128 x 128
+// block for every CU (two planes: every second one) as before.  Three planes
+// (BF16X3) gain nothing.
 bool planes_faster(const Fold &f, ttm_precision_t prec)
 {
     if (prec == TTM_PREC_FP8_E4M3 || prec == TTM_PREC_BF16X3 || f.m <= 64 || f.nq < 256) return false;
-    uint64_t const blocks = ((f.m + 127) / 128) * ((f.outer * f.w + 127) / 128);
-    return blocks * (unsigned)mode_parts(prec) <= (uint64_t)device_cus();
+    uint64_t const cus = (uint64_t)device_cus(), parts = (uint64_t)mode_parts(prec);
+    uint64_t const columns = (f.outer * f.w + 127) / 128;
+    uint64_t const narrow = f.w == 1 || f.w >= 16 ? 4 : f.w >= 8 ? 3 : 2; // quarters
+    return ((f.m + 127) / 128) * columns * parts <= cus && columns * parts * 8 <= cus * narrow;
 }
 } // namespace
 
