@@ -7,6 +7,7 @@ convenience that infers the layout of A from its strides.
 from __future__ import annotations
 
 import ctypes
+import operator
 
 import numpy as np
 
@@ -322,7 +323,9 @@ def ttm(q, A, B, *, layout=None, b_layout="row", precision=None, out=None, strea
     nb = list(B.shape)
     pib = [1, 2] if colmajor else [2, 1]
     if out is None and len(pia) == p and sorted(pia) == list(range(1, p + 1)) and _is_torch(A) and A.is_cuda:
-        return device_product(int(q), p, A, na, wa, [int(r) for r in pia], Bc, nb, pib, precision, stream)
+        # whole numbers only, as the indices they are below (2.5 is not mode 2)
+        return device_product(operator.index(q), p, A, na, wa, [operator.index(r) for r in pia], Bc, nb, pib, precision,
+                              stream)
     nc = list(na)
     nc[q - 1] = nb[0]
     C = out if out is not None else empty_like_layout(A, nc, pia)

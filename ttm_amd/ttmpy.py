@@ -15,6 +15,8 @@ Arrays of other dtypes are converted to float64, as pybind11's array_t does.
 """
 from __future__ import annotations
 
+import operator
+
 import numpy as np
 
 from . import api
@@ -59,7 +61,7 @@ def ttm(q, A, B, precision=None):
     nb = list(B.shape)
     if torch is not None and isinstance(A, torch.Tensor) and A.is_cuda and isinstance(B, torch.Tensor) \
             and B.device == A.device:
-        return api.device_product(int(q), p, A, na, wa, pia, Bc, nb, pib, precision, None)
+        return api.device_product(operator.index(q), p, A, na, wa, pia, Bc, nb, pib, precision, None)
     nc = list(na)
     nc[q - 1] = nb[0]
     C = api.empty_like_layout(A, nc, pia)
