@@ -820,14 +820,22 @@ unsigned launch_splits(Kernel k, const Fold &f, bool is_double, unsigned want)
 
 namespace
 {
-bool stream_capturing(hipStream_t s)
+// Room for `bytes` of workspace in the call's scratch region or, outside one,
+// in a graph that captures the stream: its allocation is made when the graph
+// is launched, where a failure can no longer choose another kernel, so the
+// device must have that much free now.  (An eager call tries the pool.)
+bool workspace_room(size_t bytes, hipStream_t s)
 {
+    if (bytes > scratch_available()) return false;
+    if (scratch_bound()) return true;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    size_t free_bytes = 0, total = 0;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess ||
+        (st != hipStreamCaptureStatusNone && hipMemGetInfo(&free_bytes, &total) != hipSuccess)) {
         (void)hipGetLastError();
-        return true;
+        return false;
     }
-    return st != hipStreamCaptureStatusNone;
+    return st == hipStreamCaptureStatusNone || bytes <= free_bytes;
 }
 } // namespace
 
@@ -847,12 +855,9 @@ ttm_status_t launch_f32(const Fold &f, const float *a, const float *b, float *c,
     bool const ac_aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(c)) & 15u) == 0;
     if (k == Kernel::lowp || k == Kernel::lowp_generic) {
         LowpRoute route = k == Kernel::lowp_generic ? LowpRoute::generic : lowp_route(f, prec, aligned);
-        // without room for the converted operands, or while the stream is
-        // captured (no allocation of that size there): the other kernels
+        // without room for the converted operands: the other kernels
         LowpRoute const other = lowp_supports(f, aligned) ? LowpRoute::tile : LowpRoute::generic;
-        if (route == LowpRoute::planes &&
-            (!lowp_planes_fit(f, prec) || (!scratch_bound() && stream_capturing(stream))))
-            route = other;
+        if (route == LowpRoute::planes && !workspace_room(lowp_planes_bytes(f, prec), stream)) route = other;
         ttm_status_t st = launch_lowp(f, a, b, c, prec, stream, route);
         if (route == LowpRoute::planes && st == TTM_ERR_ALLOC) {
             route = other;

@@ -2296,12 +2296,11 @@ LowpRoute lowp_route(const Fold &f, ttm_precision_t prec, bool aligned)
     return tile ? LowpRoute::tile : LowpRoute::generic;
 }
 
-bool lowp_planes_fit(const Fold &f, ttm_precision_t prec)
+size_t lowp_planes_bytes(const Fold &f, ttm_precision_t prec)
 {
-    size_t const room = scratch_available();
-    if (prec == TTM_PREC_FP8_E4M3) return fp8_bytes(f).total() <= room;
+    if (prec == TTM_PREC_FP8_E4M3) return fp8_bytes(f).total();
     size_t const scale = prec == TTM_PREC_FP16X2 ? scale_pass(f, true).bytes() : 0;
-    return plane_geom(f, mode_parts(prec)).bytes + 512 + scale <= room;
+    return plane_geom(f, mode_parts(prec)).bytes + 512 + scale;
 }
 
 std::string lowp_symbol(const Fold &f, ttm_precision_t prec, LowpRoute route)

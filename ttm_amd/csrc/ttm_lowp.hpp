@@ -25,10 +25,10 @@ enum class LowpRoute : int
     tile,
     planes
 };
-// Choice for a fold (`aligned`: A, B and C 16-byte aligned), and whether the
-// planes' workspace fits the scratch region bound to this thread, if one is.
+// Choice for a fold (`aligned`: A, B and C 16-byte aligned), and the workspace
+// of the planes (rounded up).
 LowpRoute lowp_route(const Fold &f, ttm_precision_t prec, bool aligned);
-bool lowp_planes_fit(const Fold &f, ttm_precision_t prec);
+size_t lowp_planes_bytes(const Fold &f, ttm_precision_t prec);
 
 // Template instance launched for a fold and precision (as profilers print it).
 std::string lowp_symbol(const Fold &f, ttm_precision_t prec, LowpRoute route);
