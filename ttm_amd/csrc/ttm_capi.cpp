@@ -482,8 +482,7 @@ unsigned ttm_plan_splits(unsigned q, unsigned p, int is_double, const size_t *na
 const char *ttm_last_kernel(void)
 {
     if (!t_last.valid) return "";
-    t_last_symbol = kernel_symbol(t_last.info.kernel, t_last.fold, t_last.is_double, t_last.prec, t_last.info.aligned,
-                                  t_last.info.lowp);
+    t_last_symbol = kernel_symbol(t_last.info.kernel, t_last.fold, t_last.is_double, t_last.prec, &t_last.info);
     return t_last_symbol.c_str();
 }
 

@@ -1056,7 +1056,9 @@ struct Geom
 {
     Config cfg;
     bool tn = false;
-    bool pad = false; // NN view that needs the PAD tile (set by the launcher from w and the pointers)
+    // set by the launcher: an NN view that needs the PAD tile (from w and the
+    // pointers), and the pipelined loop
+    bool pad = false, pipe = false;
     uint64_t wp = 1, ncols = 0;
     unsigned nj = 0, nn = 0;
     int bm() const { return cfg.waves_m * 16 * cfg.jt; }
@@ -1166,13 +1168,12 @@ void launch_cfg(const Fold &f, const Geom &g, const Split &sp, unsigned flags, c
                            dim3(total, sp.splits), dim3(256), 0, s, a, b, c, g.ncols, f.nq, f.w, g.wp, f.m, g.nj,
                            total, sp.kc, c_split, flags);
     };
-    bool const pipe = gemm_pipelined(f, sizeof(T) == 8, g, sp);
     using Y = std::true_type;
     using N = std::false_type;
     if (!TN && g.pad) {
-        if constexpr (!TN) pipe ? run(Y(), Y()) : run(Y(), N());
+        if constexpr (!TN) g.pipe ? run(Y(), Y()) : run(Y(), N());
     } else {
-        pipe ? run(N(), Y()) : run(N(), N());
+        g.pipe ? run(N(), Y()) : run(N(), N());
     }
 }
 
@@ -1214,17 +1215,20 @@ void launch_layout(const Fold &f, const Geom &g, const Split &sp, unsigned flags
 
 } // namespace
 
-std::string gemm_symbol(const Fold &f, bool is_double, bool aligned)
+GemmVariant gemm_variant(const Fold &f, bool is_double, bool aligned, unsigned splits)
 {
-    uint64_t const vec = is_double ? 2 : 4;
     Geom g = geom(f, is_double);
-    g.pad = !g.tn && (!aligned || f.w % vec != 0);
-    Config const &cfg = g.cfg;
+    g.pad = !g.tn && (!aligned || f.w % (is_double ? 2 : 4) != 0);
+    return {g.pad, gemm_pipelined(f, is_double, g, split_for(f, is_double, g, splits))};
+}
+
+std::string gemm_symbol(const Fold &f, bool is_double, GemmVariant variant)
+{
+    Config const cfg = pick_config(f, is_double);
     char buf[128];
     std::snprintf(buf, sizeof buf, "k_gemm<%s, %s, %d, %d, %d, %d, %s, %s, %s>", is_double ? "double" : "float",
-                  gemm_pipelined(f, is_double, g, split_for(f, is_double, g, 0)) ? "true" : "false",
-                  cfg.jt, cfg.nt, cfg.waves_m, cfg.bk, f.w == 1 ? "true" : "false", f.b_colmajor ? "true" : "false",
-                  g.pad ? "true" : "false");
+                  variant.pipe ? "true" : "false", cfg.jt, cfg.nt, cfg.waves_m, cfg.bk, f.w == 1 ? "true" : "false",
+                  f.b_colmajor ? "true" : "false", variant.pad ? "true" : "false");
     return buf;
 }
 
@@ -1249,7 +1253,8 @@ bool gemm_underfilled(const Fold &f, bool is_double)
 }
 
 template <class T>
-ttm_status_t launch_gemm(const Fold &f, const T *a, const T *b, T *c, hipStream_t s, unsigned want_splits)
+ttm_status_t launch_gemm(const Fold &f, const T *a, const T *b, T *c, hipStream_t s, unsigned want_splits,
+                         GemmVariant *ran)
 {
     constexpr uint64_t VEC = 16 / sizeof(T);
     Geom g = geom(f, sizeof(T) == 8);
@@ -1270,6 +1275,8 @@ ttm_status_t launch_gemm(const Fold &f, const T *a, const T *b, T *c, hipStream_
     if (aligned16(b)) flags |= TILE_B_VEC;
     if (g.nj == 1) flags |= TILE_STREAM | (sp.splits > 1 ? TILE_KEEP_C : 0u);
     g.pad = !g.tn && !((flags & TILE_A_VEC) && (flags & TILE_C_VEC));
+    g.pipe = gemm_pipelined(f, sizeof(T) == 8, g, sp);
+    if (ran) *ran = {g.pad, g.pipe};
     if (g.tn) {
         if (f.b_colmajor) launch_layout<T, true, true>(f, g, sp, flags, a, b, out, s);
         else launch_layout<T, true, false>(f, g, sp, flags, a, b, out, s);
@@ -1314,9 +1321,10 @@ void launch_sum_splits(const T *partials, uint64_t n, unsigned splits, T *c, hip
 template void launch_sum_splits<float>(const float *, uint64_t, unsigned, float *, hipStream_t);
 template void launch_sum_splits<double>(const double *, uint64_t, unsigned, double *, hipStream_t);
 
-template ttm_status_t launch_gemm<float>(const Fold &, const float *, const float *, float *, hipStream_t, unsigned);
+template ttm_status_t launch_gemm<float>(const Fold &, const float *, const float *, float *, hipStream_t, unsigned,
+                                         GemmVariant *);
 template ttm_status_t launch_gemm<double>(const Fold &, const double *, const double *, double *, hipStream_t,
-                                          unsigned);
+                                          unsigned, GemmVariant *);
 
 // ---- grouped launches -------------------------------------------------------
 // A chain stage over a mode without a factor: the layout rotation that the

@@ -16,9 +16,16 @@ namespace ttm_amd
 // buffers; false only beyond its grid limits).
 bool gemm_supports(const Fold &f, bool is_double);
 
-// Template instance the gemm launcher runs for a fold (as profilers print it);
-// `aligned`: A and C 16-byte aligned.
-std::string gemm_symbol(const Fold &f, bool is_double, bool aligned = true);
+// What a launch decides beyond the fold: padded slabs (buffers), the pipelined
+// loop (contraction splits).
+struct GemmVariant
+{
+    bool pad = false, pipe = false;
+};
+// The variant for a number of splits; `aligned`: A and C 16-byte aligned.
+GemmVariant gemm_variant(const Fold &f, bool is_double, bool aligned, unsigned splits);
+// Template instance of a launch (as profilers print it).
+std::string gemm_symbol(const Fold &f, bool is_double, GemmVariant variant);
 
 // Contraction split of a product: `splits` ranges of kc indices.
 struct Split
@@ -39,8 +46,10 @@ template <class T>
 void launch_sum_splits(const T *partials, uint64_t n, unsigned splits, T *c, hipStream_t s);
 
 // want_splits as for gemm_split.  Partials come from the call's workspace.
+// *ran: the variant launched.
 template <class T>
-ttm_status_t launch_gemm(const Fold &f, const T *a, const T *b, T *c, hipStream_t s, unsigned want_splits = 0);
+ttm_status_t launch_gemm(const Fold &f, const T *a, const T *b, T *c, hipStream_t s, unsigned want_splits = 0,
+                         GemmVariant *ran = nullptr);
 
 // ---- grouped (persistent, many products per launch) ------------------------
 

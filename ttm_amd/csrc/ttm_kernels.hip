@@ -668,7 +668,8 @@ void launch_stream(const Fold &f, const T *a, const T *b, T *c, hipStream_t s, b
 }
 
 template <class T>
-ttm_status_t launch_plain(const Fold &f, const T *a, const T *b, T *c, hipStream_t s, Kernel kern, unsigned splits)
+ttm_status_t launch_plain(const Fold &f, const T *a, const T *b, T *c, hipStream_t s, Kernel kern, unsigned splits,
+                          LaunchInfo *info)
 {
     uint64_t const bsj = f.b_stride_j(), bsl = f.b_stride_l();
     constexpr int VEC = Traits<T>::VEC;
@@ -708,7 +709,7 @@ ttm_status_t launch_plain(const Fold &f, const T *a, const T *b, T *c, hipStream
         ws_release(ws, s);
         break;
     }
-    case Kernel::gemm: return launch_gemm<T>(f, a, b, c, s, splits);
+    case Kernel::gemm: return launch_gemm<T>(f, a, b, c, s, splits, info ? &info->gemm : nullptr);
     case Kernel::skinny: return launch_skinny<T>(f, a, b, c, s, splits);
     default: set_error(TTM_ERR_ARGUMENT, "no kernel for this problem"); return TTM_ERR_ARGUMENT;
     }
@@ -732,7 +733,7 @@ const char *kernel_name(Kernel k)
     return (i >= 0 && i < static_cast<int>(Kernel::count)) ? k_kernel_names[i] : "none";
 }
 
-std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision_t prec, bool aligned, int lowp)
+std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision_t prec, const LaunchInfo *ran)
 {
     std::string const t = is_double ? "double" : "float";
     std::string const jt = std::to_string(pick_jt(f.m));
@@ -751,10 +752,11 @@ std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision
                std::to_string(stream_depth(j, tn)) + ", " +
                (stream_bvec(f, is_double ? 2 : 4, tn) ? "true" : "false") + ">";
     }
-    case Kernel::gemm: return gemm_symbol(f, is_double, aligned);
+    case Kernel::gemm:
+        return gemm_symbol(f, is_double,
+                           ran ? ran->gemm : gemm_variant(f, is_double, true, launch_splits(k, f, is_double, 0)));
     case Kernel::skinny: return skinny_symbol(f, is_double);
-    case Kernel::lowp:
-        return lowp_symbol(f, prec, lowp >= 0 ? static_cast<LowpRoute>(lowp) : lowp_route(f, prec, aligned));
+    case Kernel::lowp: return lowp_symbol(f, prec, ran ? ran->lowp : lowp_route(f, prec, true));
     case Kernel::lowp_generic: return lowp_symbol(f, prec, LowpRoute::generic);
     default: return "";
     }
@@ -852,7 +854,6 @@ ttm_status_t launch_f32(const Fold &f, const float *a, const float *b, float *c,
         set_error(TTM_ERR_PRECISION);
         return TTM_ERR_PRECISION;
     }
-    bool const ac_aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(c)) & 15u) == 0;
     if (k == Kernel::lowp || k == Kernel::lowp_generic) {
         LowpRoute route = k == Kernel::lowp_generic ? LowpRoute::generic : lowp_route(f, prec, aligned);
         // without room for the converted operands: the other kernels
@@ -864,14 +865,14 @@ ttm_status_t launch_f32(const Fold &f, const float *a, const float *b, float *c,
             st = launch_lowp(f, a, b, c, prec, stream, route);
         }
         if (info) {
-            *info = LaunchInfo{route == LowpRoute::generic ? Kernel::lowp_generic : Kernel::lowp, 1, aligned};
-            info->lowp = static_cast<int>(route);
+            *info = LaunchInfo{route == LowpRoute::generic ? Kernel::lowp_generic : Kernel::lowp};
+            info->lowp = route;
         }
         return st;
     }
     if (want_splits == 0) want_splits = tuned_splits(k, f, false);
-    if (info) *info = LaunchInfo{k, launch_splits(k, f, false, want_splits), ac_aligned};
-    return launch_plain<float>(f, a, b, c, stream, k, want_splits);
+    if (info) *info = LaunchInfo{k, launch_splits(k, f, false, want_splits)};
+    return launch_plain<float>(f, a, b, c, stream, k, want_splits, info);
 }
 
 ttm_status_t launch_f64(const Fold &f, const double *a, const double *b, double *c, hipStream_t stream,
@@ -882,9 +883,8 @@ ttm_status_t launch_f64(const Fold &f, const double *a, const double *b, double 
     bool const aligned = (bits & 15u) == 0;
     Kernel const k = (bits & 7u) ? Kernel::generic : choose_kernel(f, true, TTM_PREC_DEFAULT, aligned, force);
     if (want_splits == 0) want_splits = tuned_splits(k, f, true);
-    bool const ac_aligned = ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(c)) & 15u) == 0;
-    if (info) *info = LaunchInfo{k, launch_splits(k, f, true, want_splits), ac_aligned};
-    return launch_plain<double>(f, a, b, c, stream, k, want_splits);
+    if (info) *info = LaunchInfo{k, launch_splits(k, f, true, want_splits)};
+    return launch_plain<double>(f, a, b, c, stream, k, want_splits, info);
 }
 
 } // namespace ttm_amd

@@ -7,6 +7,8 @@
 #include <string>
 
 #include "ttm_amd.h"
+#include "ttm_gemm.hpp"
+#include "ttm_lowp.hpp"
 #include "ttm_plan.hpp"
 
 namespace ttm_amd
@@ -40,11 +42,11 @@ Kernel kernel_from_name(const char *name);
 // aligned).  `force` (may be Kernel::none) overrides when applicable.
 Kernel choose_kernel(const Fold &f, bool is_double, ttm_precision_t prec, bool aligned, Kernel force);
 
-// Template instance of the family's kernel for a fold (as profilers print it);
-// `aligned`: A, B and C 16-byte aligned (selects the NN tile without padding);
-// lowp: the LowpRoute that ran (-1: the one the planner picks).
-std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision_t prec, bool aligned = true,
-                          int lowp = -1);
+// Template instance of the family's kernel for a fold (as profilers print it):
+// the one that `ran`, or the one the planner picks for 16-byte aligned buffers.
+struct LaunchInfo;
+std::string kernel_symbol(Kernel k, const Fold &f, bool is_double, ttm_precision_t prec,
+                          const LaunchInfo *ran = nullptr);
 
 // Contraction splits a launch of family k runs with: `want` (0: the cached
 // tuning of the fold's class, else the family's own choice), clamped by the
@@ -56,8 +58,8 @@ struct LaunchInfo
 {
     Kernel kernel = Kernel::none;
     unsigned splits = 1;
-    bool aligned = true;
-    int lowp = -1; // LowpRoute of a reduced-precision product
+    GemmVariant gemm;                        // of a gemm launch
+    LowpRoute lowp = LowpRoute::generic;     // of a reduced-precision one
 };
 
 // Launch the product on `stream`; returns TTM_SUCCESS or TTM_ERR_HIP.

@@ -2015,6 +2015,20 @@ PlaneShape plane_shape(const Fold &f, int parts)
     if (parts < 3 && f.m > 128 && big >= (uint64_t)device_cus()) return PLANES_256;
     return PLANES_128;
 }
+// Template arguments of k_planes for a shape.
+struct PlaneBlock
+{
+    int wm, wn, jt, nt, ks, ns;
+    constexpr int bm() const { return 16 * jt * wm; }
+    constexpr int bn() const { return 16 * nt * wn; }
+};
+constexpr PlaneBlock plane_block(PlaneShape shape, int parts)
+{
+    int const ks = parts == 1 ? 2 : 1;
+    if (shape == PLANES_64) return {1, 2, 4, 4, ks, 2};
+    if (shape == PLANES_128) return {2, 2, 4, 4, ks, 2};
+    return parts == 1 ? PlaneBlock{1, 4, 8, 4, 1, 3} : PlaneBlock{2, 4, 8, 4, ks, 2};
+}
 struct PlaneGeom
 {
     uint64_t bm, bn, ldk, rows_a, rows_b, plane_a, plane_b;
@@ -2022,10 +2036,10 @@ struct PlaneGeom
 };
 PlaneGeom plane_geom(const Fold &f, int parts)
 {
-    PlaneShape const sh = plane_shape(f, parts);
+    PlaneBlock const block = plane_block(plane_shape(f, parts), parts);
     PlaneGeom g;
-    g.bm = sh == PLANES_64 ? 64 : sh == PLANES_128 || parts == 1 ? 128 : 256;
-    g.bn = sh == PLANES_256 ? 256 : 128;
+    g.bm = (uint64_t)block.bm();
+    g.bn = (uint64_t)block.bn();
     uint64_t const kq = parts == 1 ? 64 : 32; // contraction indices per stage
     g.ldk = (f.nq + kq - 1) / kq * kq;
     uint64_t const ncols = f.outer * f.w;
@@ -2038,21 +2052,22 @@ PlaneGeom plane_geom(const Fold &f, int parts)
 }
 int mode_parts(ttm_precision_t prec) { return prec == TTM_PREC_BF16X3 ? 3 : prec == TTM_PREC_FP16X2 ? 2 : 1; }
 
-template <int MODE, int WM, int WN, int JT, int NT, int KS, int NS>
+template <int MODE, PlaneShape SHAPE>
 void launch_planes_shape(const Fold &f, const PlaneGeom &g, const typename Lp<MODE>::op *as,
                          const typename Lp<MODE>::op *bs, float *c, const int *exps, hipStream_t s)
 {
-    using S = PlaneTile<MODE, WM, WN, JT, NT, KS, NS>;
-    unsigned const nj = (unsigned)(g.rows_b / S::BM);
-    unsigned const total = nj * (unsigned)(g.rows_a / S::BN);
+    constexpr PlaneBlock B = plane_block(SHAPE, Lp<MODE>::PARTS);
+    unsigned const nj = (unsigned)(g.rows_b / B.bm());
+    unsigned const total = nj * (unsigned)(g.rows_a / B.bn());
+    dim3 const threads(64 * B.wm * B.wn);
     bool const ts = f.w == 1;
     int const c_vec = (reinterpret_cast<uintptr_t>(c) & 15u) == 0 && (ts ? f.m : f.w) % 4 == 0;
     uint64_t const ncols = f.outer * f.w;
     if (ts)
-        hipLaunchKernelGGL((k_planes<MODE, WM, WN, JT, NT, KS, NS, true>), dim3(total), dim3(64 * WM * WN), 0, s, as,
+        hipLaunchKernelGGL((k_planes<MODE, B.wm, B.wn, B.jt, B.nt, B.ks, B.ns, true>), dim3(total), threads, 0, s, as,
                            g.plane_a, bs, g.plane_b, g.ldk, c, ncols, f.w, f.m, nj, total, c_vec, exps);
     else
-        hipLaunchKernelGGL((k_planes<MODE, WM, WN, JT, NT, KS, NS, false>), dim3(total), dim3(64 * WM * WN), 0, s, as,
+        hipLaunchKernelGGL((k_planes<MODE, B.wm, B.wn, B.jt, B.nt, B.ks, B.ns, false>), dim3(total), threads, 0, s, as,
                            g.plane_a, bs, g.plane_b, g.ldk, c, ncols, f.w, f.m, nj, total, c_vec, exps);
 }
 
@@ -2082,15 +2097,13 @@ ttm_status_t launch_planes(const Fold &f, const float *a, const float *b, float 
     unsigned const blocks_a = blocks(g.rows_a, f.w == 1), blocks_b = blocks(g.rows_b, !f.b_colmajor);
     hipLaunchKernelGGL(k_planes_convert<MODE>, dim3(blocks_a + blocks_b), dim3(256), 0, s, a, as, ncols, f.w, g.plane_a,
                        b, bs, f.m, f.b_colmajor ? 0 : 1, g.plane_b, f.nq, nsl, blocks_a, exps);
-    constexpr int KS = P == 1 ? 2 : 1;
-    PlaneShape const sh = plane_shape(f, P);
-    if (sh == PLANES_64) {
-        launch_planes_shape<MODE, 1, 2, 4, 4, KS, 2>(f, g, as, bs, c, exps, s);
-    } else if (sh == PLANES_128) {
-        launch_planes_shape<MODE, 2, 2, 4, 4, KS, 2>(f, g, as, bs, c, exps, s);
+    PlaneShape const shape = plane_shape(f, P);
+    if (shape == PLANES_64) {
+        launch_planes_shape<MODE, PLANES_64>(f, g, as, bs, c, exps, s);
+    } else if (shape == PLANES_128) {
+        launch_planes_shape<MODE, PLANES_128>(f, g, as, bs, c, exps, s);
     } else {
-        if constexpr (P == 2) launch_planes_shape<MODE, 2, 4, 8, 4, KS, 2>(f, g, as, bs, c, exps, s);
-        else if constexpr (P == 1) launch_planes_shape<MODE, 1, 4, 8, 4, 1, 3>(f, g, as, bs, c, exps, s);
+        if constexpr (P < 3) launch_planes_shape<MODE, PLANES_256>(f, g, as, bs, c, exps, s);
     }
     hipError_t const e = hipGetLastError();
     ws_release(ws, s);
@@ -2315,9 +2328,10 @@ std::string lowp_symbol(const Fold &f, ttm_precision_t prec, LowpRoute route)
     if (prec == TTM_PREC_FP8_E4M3) {
         std::snprintf(buf, sizeof buf, "k_fp8<%s, %d>", tn, fp8_block_rows(f));
     } else if (route == LowpRoute::planes) {
-        static const char *const shapes[] = {"1, 2, 4, 4", "2, 2, 4, 4", "2, 4, 8, 4"};
         int const parts = mode_parts(prec);
-        std::snprintf(buf, sizeof buf, "k_planes<%d, %s, %s>", mode, shapes[plane_shape(f, parts)], tn);
+        PlaneBlock const b = plane_block(plane_shape(f, parts), parts);
+        std::snprintf(buf, sizeof buf, "k_planes<%d, %d, %d, %d, %d, %d, %d, %s>", mode, b.wm, b.wn, b.jt, b.nt, b.ks,
+                      b.ns, tn);
     } else {
         std::snprintf(buf, sizeof buf, "k_lowp<%d, %s, %d>", mode, tn, lp_block_rows(f));
     }
