@@ -243,59 +243,51 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     // Per-thread places of the vectors within the tile and the fixed part of
     // the A addresses; NN vectors are VEC padded columns of one slab, of which
     // a_nv are real (i < w).
-    struct Place
-    {
-        uint64_t a_base[A_PER];
-        bool a_ok[A_PER];
-        int a_row[A_PER], a_col[A_PER], a_nv[A_PER];
-        int b_row[B_PER], b_col[B_PER];
-        bool b_in[B_PER];
-    };
-    auto place = [&](int t) {
-        Place g;
+    uint64_t a_base[A_PER];
+    bool a_ok[A_PER];
+    int a_row[A_PER], a_col[A_PER], a_nv[A_PER];
+    int b_row[B_PER], b_col[B_PER];
+    bool b_in[B_PER];
 #pragma unroll
-        for (int e = 0; e < A_PER; ++e) {
-            int const v = t + 256 * e;
-            g.a_ok[e] = v < A_VECS;
-            g.a_nv[e] = VEC;
-            if constexpr (!TN) {
-                g.a_row[e] = v / (BN / VEC);
-                g.a_col[e] = (v % (BN / VEC)) * VEC;
-                uint64_t const n = n0 + g.a_col[e];
-                g.a_ok[e] = g.a_ok[e] && n < ncols;
-                if constexpr (PAD) {
-                    uint64_t const k = g.a_ok[e] ? n / wp : 0;
-                    uint64_t const i = g.a_ok[e] ? n - k * wp : 0;
-                    g.a_ok[e] = g.a_ok[e] && i < w;
-                    g.a_nv[e] = g.a_ok[e] ? (int)(w - i < (uint64_t)VEC ? w - i : VEC) : 0;
-                    g.a_base[e] = g.a_ok[e] ? k * ld * w + i : 0;
-                } else {
-                    uint64_t const k = g.a_ok[e] ? n / w : 0;
-                    g.a_base[e] = k * ld * w + (g.a_ok[e] ? n - k * w : 0);
-                }
+    for (int e = 0; e < A_PER; ++e) {
+        int const v = tid + 256 * e;
+        a_ok[e] = v < A_VECS;
+        a_nv[e] = VEC;
+        if constexpr (!TN) {
+            a_row[e] = v / (BN / VEC);
+            a_col[e] = (v % (BN / VEC)) * VEC;
+            uint64_t const n = n0 + a_col[e];
+            a_ok[e] = a_ok[e] && n < ncols;
+            if constexpr (PAD) {
+                uint64_t const k = a_ok[e] ? n / wp : 0;
+                uint64_t const i = a_ok[e] ? n - k * wp : 0;
+                a_ok[e] = a_ok[e] && i < w;
+                a_nv[e] = a_ok[e] ? (int)(w - i < (uint64_t)VEC ? w - i : VEC) : 0;
+                a_base[e] = a_ok[e] ? k * ld * w + i : 0;
             } else {
-                g.a_col[e] = v / (BK / VEC);         // column n within the tile
-                g.a_row[e] = (v % (BK / VEC)) * VEC; // first l within the slice
-                uint64_t const n = n0 + g.a_col[e];
-                g.a_ok[e] = g.a_ok[e] && n < ncols;
-                g.a_base[e] = g.a_ok[e] ? n * ld : 0;
+                uint64_t const k = a_ok[e] ? n / w : 0;
+                a_base[e] = k * ld * w + (a_ok[e] ? n - k * w : 0);
             }
+        } else {
+            a_col[e] = v / (BK / VEC);         // column n within the tile
+            a_row[e] = (v % (BK / VEC)) * VEC; // first l within the slice
+            uint64_t const n = n0 + a_col[e];
+            a_ok[e] = a_ok[e] && n < ncols;
+            a_base[e] = a_ok[e] ? n * ld : 0;
         }
+    }
 #pragma unroll
-        for (int e = 0; e < B_PER; ++e) {
-            int const v = t + 256 * e;
-            g.b_in[e] = v < B_VECS;
-            if constexpr (BCOL) {
-                g.b_row[e] = v / (BM / VEC);
-                g.b_col[e] = (v % (BM / VEC)) * VEC;
-            } else {
-                g.b_col[e] = v / (BK / VEC);
-                g.b_row[e] = (v % (BK / VEC)) * VEC;
-            }
+    for (int e = 0; e < B_PER; ++e) {
+        int const v = tid + 256 * e;
+        b_in[e] = v < B_VECS;
+        if constexpr (BCOL) {
+            b_row[e] = v / (BM / VEC);
+            b_col[e] = (v % (BM / VEC)) * VEC;
+        } else {
+            b_col[e] = v / (BK / VEC);
+            b_row[e] = (v % (BK / VEC)) * VEC;
         }
-        return g;
-    };
-    Place const pl = place(tid);
+    }
     bool const b_vec_ok = (flags & TILE_B_VEC) != 0 && (BCOL ? (m % VEC == 0) : (ld % VEC == 0));
 
     // Register sets of slices in flight: two for tiles of at most 32 rows per
@@ -332,23 +324,23 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
         if (!a_vec) {
             bool whole = n0 + BN <= ncols && rows_ok;
 #pragma unroll
-            for (int e = 0; e < A_PER; ++e) whole = whole && pl.a_nv[e] == VEC;
+            for (int e = 0; e < A_PER; ++e) whole = whole && a_nv[e] == VEC;
             full = __syncthreads_and(whole ? 1 : 0) != 0;
         }
     }
     uint64_t a_fix[A_PER]; // A offset of the thread's vector in slice 0
 #pragma unroll
-    for (int e = 0; e < A_PER; ++e) a_fix[e] = TN ? pl.a_base[e] + pl.a_row[e] : pl.a_base[e] + (uint64_t)pl.a_row[e] * w;
+    for (int e = 0; e < A_PER; ++e) a_fix[e] = TN ? a_base[e] + a_row[e] : a_base[e] + (uint64_t)a_row[e] * w;
     uint64_t const a_step = TN ? 1 : w; // A offset per contraction index
 
-    auto load_tiles = [&](Place const &g, uint64_t l0, auto set) {
+    auto load_tiles = [&](uint64_t l0, auto set) {
         constexpr int S = decltype(set)::value;
 #pragma unroll
         for (int e = 0; e < A_PER; ++e) {
             ra[S][e] = vzero<V>();
             ra_dm[S][e] = DM_WHOLE;
             if constexpr (!TN) {
-                uint64_t const l = l0 + g.a_row[e];
+                uint64_t const l = l0 + a_row[e];
                 if (!PAD || a_vec) {
                     // One in-range vector per thread and no branch (a conditional
                     // load leaves its register with two values, and the compiler
@@ -356,8 +348,8 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                     // row nq - 1 and columns past the last one column 0 (a_base 0).
                     // A [120, 300, 59] x_2, m = 33, B column-major, float64: 58 ->
                     // 46 us, A [109, 200, 2740], m = 256: 885 -> 687 us.
-                    ra[S][e] = load_a(a + g.a_base[e] + (l < nq ? l : nq - 1) * w);
-                    ra_dm[S][e] = g.a_ok[e] && l < nq ? DM_WHOLE : 0;
+                    ra[S][e] = load_a(a + a_base[e] + (l < nq ? l : nq - 1) * w);
+                    ra_dm[S][e] = a_ok[e] && l < nq ? DM_WHOLE : 0;
                 } else {
                     // Branch-free: the VEC elements from the vector's first
                     // (element-aligned) address; rows of a slab are
@@ -370,12 +362,12 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                     // the read then starts before `a`, still inside A, which
                     // holds at least VEC elements)
                     uint64_t const lc = l < nq ? l : nq - 1;
-                    int64_t const addr = (int64_t)(g.a_base[e] + lc * w);
+                    int64_t const addr = (int64_t)(a_base[e] + lc * w);
                     int64_t const lim = (int64_t)a_len - VEC;
                     int64_t const ac = addr < lim ? addr : lim;
                     V const v = ldg<typename Gt::vec_u>(a + ac);
                     ra[S][e] = v;
-                    ra_dm[S][e] = (int)(addr - ac) | (l < nq ? g.a_nv[e] : 0) << 8;
+                    ra_dm[S][e] = (int)(addr - ac) | (l < nq ? a_nv[e] : 0) << 8;
                 }
             } else if (nq >= (uint64_t)VEC) {
                 // One in-bounds vector per thread and no divergent branch (a
@@ -384,28 +376,28 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                 // that would run past the row end is read as the row's last
                 // VEC elements and shifted into place; elements past the row
                 // end, and rows past the last column (read as row 0), are zero.
-                uint64_t const l = l0 + g.a_row[e];
+                uint64_t const l = l0 + a_row[e];
                 uint64_t const last = nq - VEC;
                 uint64_t const lc = l < last ? l : last;
-                V const v = ldg<typename Gt::vec_u>(a + g.a_base[e] + lc);
-                int const nvalid = (!g.a_ok[e] || l >= nq) ? 0 : (int)(nq - l < (uint64_t)VEC ? nq - l : VEC);
+                V const v = ldg<typename Gt::vec_u>(a + a_base[e] + lc);
+                int const nvalid = (!a_ok[e] || l >= nq) ? 0 : (int)(nq - l < (uint64_t)VEC ? nq - l : VEC);
                 ra[S][e] = v;
                 ra_dm[S][e] = (int)(l - lc) | nvalid << 8;
             } else {
-                uint64_t const l = l0 + g.a_row[e];
-                if (g.a_ok[e] && l < nq) {
+                uint64_t const l = l0 + a_row[e];
+                if (a_ok[e] && l < nq) {
                     if (a_vec) {
                         // nq % VEC == 0: a vector is wholly in or out of range
-                        ra[S][e] = load_a(a + g.a_base[e] + l);
+                        ra[S][e] = load_a(a + a_base[e] + l);
                     } else if (l + VEC <= nq) {
                         // element-aligned vector inside the row
-                        V const v = ldg<typename Gt::vec_u>(a + g.a_base[e] + l);
+                        V const v = ldg<typename Gt::vec_u>(a + a_base[e] + l);
                         ra[S][e] = v;
                     } else {
                         // the row's last, partial vector
 #pragma unroll
                         for (int x = 0; x < VEC; ++x)
-                            if (l + x < nq) ra[S][e][x] = ldg<T>(a + g.a_base[e] + l + x);
+                            if (l + x < nq) ra[S][e][x] = ldg<T>(a + a_base[e] + l + x);
                     }
                 }
             }
@@ -414,10 +406,10 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
         for (int e = 0; e < B_PER; ++e) {
             rb[S][e] = vzero<V>();
             rb_dm[S][e] = DM_WHOLE;
-            if (!g.b_in[e]) continue;
+            if (!b_in[e]) continue;
             if constexpr (BCOL) {
-                uint64_t const l = l0 + g.b_row[e];
-                uint64_t const j = j0 + g.b_col[e];
+                uint64_t const l = l0 + b_row[e];
+                uint64_t const j = j0 + b_col[e];
                 if (l < nq) {
                     if (j + VEC <= m) {
                         // element-aligned vector inside column l (16-byte aligned when m % VEC == 0)
@@ -432,9 +424,9 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
             } else if (nq >= (uint64_t)VEC) {
                 // as the TN rows of A; rows past m read row m - 1 (their
                 // products are never stored)
-                uint64_t const j = j0 + g.b_col[e];
+                uint64_t const j = j0 + b_col[e];
                 uint64_t const jc = j < m ? j : m - 1;
-                uint64_t const l = l0 + g.b_row[e];
+                uint64_t const l = l0 + b_row[e];
                 uint64_t const last = nq - VEC;
                 uint64_t const lc = l < last ? l : last;
                 V const v = ldg<typename Gt::vec_u>(b + jc * ld + lc);
@@ -442,8 +434,8 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                 rb[S][e] = v;
                 rb_dm[S][e] = (int)(l - lc) | nvalid << 8;
             } else {
-                uint64_t const j = j0 + g.b_col[e];
-                uint64_t const l = l0 + g.b_row[e];
+                uint64_t const j = j0 + b_col[e];
+                uint64_t const l = l0 + b_row[e];
                 if (j < m) {
                     if (l + VEC <= nq) {
                         // element-aligned vector inside row j (16-byte aligned when ld % VEC == 0)
@@ -468,8 +460,8 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     uint64_t b_fix[B_PER]; // B offset of the thread's vector in slice 0
 #pragma unroll
     for (int e = 0; e < B_PER; ++e) {
-        uint64_t const jj = pl.b_in[e] ? (uint64_t)pl.b_col[e] : 0;
-        uint64_t const ll = pl.b_in[e] ? (uint64_t)pl.b_row[e] : 0;
+        uint64_t const jj = b_in[e] ? (uint64_t)b_col[e] : 0;
+        uint64_t const ll = b_in[e] ? (uint64_t)b_row[e] : 0;
         uint64_t const j = j0 + jj;
         b_fix[e] = BCOL ? (j + VEC <= m ? j : m - VEC) + ll * m : (j < m ? j : m - 1) * ld + ll;
     }
@@ -521,13 +513,13 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
         };
 #pragma unroll
         for (int e = 0; e < A_PER; ++e) {
-            uint64_t const l = l0 + pl.a_row[e];
-            if constexpr (TN) along_l(a + a_fix[e] - pl.a_row[e], l, ra[S][e], ra_dm[S][e]);
-            else across_l(a + a_fix[e] - (uint64_t)pl.a_row[e] * w, l, w, ra[S][e], ra_dm[S][e]);
+            uint64_t const l = l0 + a_row[e];
+            if constexpr (TN) along_l(a + a_fix[e] - a_row[e], l, ra[S][e], ra_dm[S][e]);
+            else across_l(a + a_fix[e] - (uint64_t)a_row[e] * w, l, w, ra[S][e], ra_dm[S][e]);
         }
 #pragma unroll
         for (int e = 0; e < B_PER; ++e) {
-            uint64_t const ll = pl.b_in[e] ? (uint64_t)pl.b_row[e] : 0;
+            uint64_t const ll = b_in[e] ? (uint64_t)b_row[e] : 0;
             if constexpr (BCOL) across_l(b + b_fix[e] - ll * m, l0 + ll, m, rb[S][e], rb_dm[S][e]);
             else along_l(b + b_fix[e] - ll, l0 + ll, rb[S][e], rb_dm[S][e]);
         }
@@ -543,7 +535,7 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     auto tn_swz = [](int l) { return NT * (((l >> 3) * 3) & 3); };
     // full_tag false: the slice came from load_tiles or load_ragged (shift and
     // mask the vectors here).
-    auto store_tiles = [&](Place const &g, int buf, auto set, auto full_tag) {
+    auto store_tiles = [&](int buf, auto set, auto full_tag) {
         constexpr int S = decltype(set)::value;
         constexpr bool GUARDED = !decltype(full_tag)::value;
 #pragma unroll
@@ -553,24 +545,24 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                 V const v = !GUARDED ? ra[S][e]
                             : PAD    ? shift_mask(ra[S][e], ra_dm[S][e] & 0xff, ra_dm[S][e] >> 8)
                                      : (ra_dm[S][e] ? ra[S][e] : vzero<V>());
-                *reinterpret_cast<V *>(&sA[buf][g.a_row[e] * LDA + g.a_col[e]]) = v;
+                *reinterpret_cast<V *>(&sA[buf][a_row[e] * LDA + a_col[e]]) = v;
             } else {
                 V const v = GUARDED ? shift_mask(ra[S][e], ra_dm[S][e] & 0xff, ra_dm[S][e] >> 8) : ra[S][e];
 #pragma unroll
                 for (int x = 0; x < VEC; ++x)
-                    sA[buf][(g.a_row[e] + x) * LDA + (g.a_col[e] ^ tn_swz(g.a_row[e] + x))] = v[x];
+                    sA[buf][(a_row[e] + x) * LDA + (a_col[e] ^ tn_swz(a_row[e] + x))] = v[x];
             }
         }
 #pragma unroll
         for (int e = 0; e < B_PER; ++e) {
-            if (B_VECS % 256 != 0 && !g.b_in[e]) continue;
+            if (B_VECS % 256 != 0 && !b_in[e]) continue;
             if constexpr (BCOL) {
                 V const v = GUARDED ? shift_mask(rb[S][e], rb_dm[S][e] & 0xff, rb_dm[S][e] >> 8) : rb[S][e];
-                *reinterpret_cast<V *>(&sB[buf][g.b_row[e] * LDB + g.b_col[e]]) = v;
+                *reinterpret_cast<V *>(&sB[buf][b_row[e] * LDB + b_col[e]]) = v;
             } else {
                 V const v = GUARDED ? shift_mask(rb[S][e], rb_dm[S][e] & 0xff, rb_dm[S][e] >> 8) : rb[S][e];
 #pragma unroll
-                for (int x = 0; x < VEC; ++x) sB[buf][(g.b_row[e] + x) * LDB + g.b_col[e]] = v[x];
+                for (int x = 0; x < VEC; ++x) sB[buf][(b_row[e] + x) * LDB + b_col[e]] = v[x];
             }
         }
     };
@@ -607,23 +599,23 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     using I1 = std::integral_constant<int, PF - 1>;
     // Slices [sb, se) of the contraction; starts and ends with all waves
     // synchronised and both LDS buffers free.
-    auto kloop = [&](Place const &g, auto full_tag, uint64_t sb, uint64_t se) {
+    auto kloop = [&](auto full_tag, uint64_t sb, uint64_t se) {
         constexpr bool FULL = decltype(full_tag)::value;
         auto load = [&](uint64_t s, auto set) {
             if constexpr (FULL) load_full(s * BK, set);
-            else load_tiles(g, s * BK, set);
+            else load_tiles(s * BK, set);
         };
         uint64_t const n = se - sb;
         if constexpr (PF == 1) {
             load(sb, I0());
-            store_tiles(g, 0, I0(), full_tag);
+            store_tiles(0, I0(), full_tag);
             __syncthreads();
             for (uint64_t s = 0; s < n; ++s) {
                 int const buf = (int)(s & 1);
                 bool const more = s + 1 < n;
                 if (more) load(sb + s + 1, I0());
                 multiply(buf);
-                if (more) store_tiles(g, buf ^ 1, I0(), full_tag);
+                if (more) store_tiles(buf ^ 1, I0(), full_tag);
                 __syncthreads();
             }
         } else {
@@ -632,17 +624,17 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
             // buffer only after the barrier that ended its slice's products.
             load(sb, I0());
             if (n > 1) load(sb + 1, I1());
-            store_tiles(g, 0, I0(), full_tag);
+            store_tiles(0, I0(), full_tag);
             __syncthreads();
             for (uint64_t s = 0; s < n; s += 2) {
                 if (s + 2 < n) load(sb + s + 2, I0());
                 multiply(0);
-                if (s + 1 < n) store_tiles(g, 1, I1(), full_tag);
+                if (s + 1 < n) store_tiles(1, I1(), full_tag);
                 __syncthreads();
                 if (s + 1 < n) {
                     if (s + 3 < n) load(sb + s + 3, I1());
                     multiply(1);
-                    if (s + 2 < n) store_tiles(g, 0, I0(), full_tag);
+                    if (s + 2 < n) store_tiles(0, I0(), full_tag);
                     __syncthreads();
                 }
             }
@@ -698,8 +690,8 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
             bool const last = kk + 1 == STEPS;
             if (!last) fragments(BUF, kk + 1, (kk + 1) & 1);
             if (kk + 2 == STEPS && more) {
-                if (TAIL && s + 1 == nwhole) store_tiles(pl, BUF ^ 1, Set(), std::false_type());
-                else store_tiles(pl, BUF ^ 1, Set(), std::true_type());
+                if (TAIL && s + 1 == nwhole) store_tiles(BUF ^ 1, Set(), std::false_type());
+                else store_tiles(BUF ^ 1, Set(), std::true_type());
             }
             if (last) {
                 uint64_t const t = s + 1 + PF;
@@ -736,7 +728,7 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
         };
         load_full(0, I0());
         if constexpr (PF == 2) load(1, I1());
-        store_tiles(pl, 0, I0(), std::true_type());
+        store_tiles(0, I0(), std::true_type());
         load(PF, I0());
         lds_barrier();
         fragments(0, 0, 0);
@@ -757,8 +749,8 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                 bool const more = s + 1 < nslices;
                 multiply(buf);
                 if (more) {
-                    if (s + 1 == nwhole) store_tiles(pl, buf ^ 1, I0(), std::false_type());
-                    else store_tiles(pl, buf ^ 1, I0(), std::true_type());
+                    if (s + 1 == nwhole) store_tiles(buf ^ 1, I0(), std::false_type());
+                    else store_tiles(buf ^ 1, I0(), std::true_type());
                     load(s + 2, I0());
                 }
                 lds_barrier();
@@ -768,15 +760,15 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     if constexpr (VIEW == VIEW_TT) {
         // grouped chain stages (contractions of 16..256): one loop per tile,
         // unguarded only when every slice is whole
-        if (full && nq % BK == 0) kloop(pl, std::true_type(), 0, nslices);
-        else kloop(pl, std::false_type(), 0, nslices);
+        if (full && nq % BK == 0) kloop(std::true_type(), 0, nslices);
+        else kloop(std::false_type(), 0, nslices);
     } else if constexpr (PIPE) {
         if (full && nwhole > 0) kloop_pipe();
-        else kloop(pl, std::false_type(), 0, nslices);
+        else kloop(std::false_type(), 0, nslices);
     } else {
         uint64_t const n = full ? nwhole : 0; // slices with unguarded loads
-        if (n > 0) kloop(pl, std::true_type(), 0, n);
-        if (n < nslices) kloop(pl, std::false_type(), n, nslices);
+        if (n > 0) kloop(std::true_type(), 0, n);
+        if (n < nslices) kloop(std::false_type(), n, nslices);
     }
 
     // ---- epilogue ---------------------------------------------------------
@@ -1207,9 +1199,15 @@ void launch_layout(const Fold &f, const Geom &g, const Split &sp, unsigned flags
         else if constexpr (sizeof(T) == 4) launch_cfg<T, 3, 4, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
         return;
     }
+    // (256 columns: float64 takes them for at most 16 rows)
+    if constexpr (sizeof(T) == 4) {
+        if (cfg.jt == 2 || (cfg.jt == 4 && cfg.waves_m == 1)) {
+            if (cfg.jt == 2) launch_cfg<T, 2, 4, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
+            else launch_cfg<T, 4, 4, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
+            return;
+        }
+    }
     if (cfg.jt == 1) launch_cfg<T, 1, 4, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
-    else if (cfg.jt == 2) launch_cfg<T, 2, 4, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
-    else if (cfg.waves_m == 1) launch_cfg<T, 4, 4, 1, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
     else launch_cfg<T, 4, 4, 2, 16, TN, BCOL>(f, g, sp, flags, a, b, c, s);
 }
 

@@ -70,20 +70,6 @@ __device__ __forceinline__ f64x4 mfma4(double a, double b, f64x4 c)
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// Four consecutive accumulator rows (r = 0..3) stored to 4 consecutive
-// elements at p (16-byte aligned).
-__device__ __forceinline__ void store_rows4(float *p, f32x4 v) { *reinterpret_cast<f32x4 *>(p) = v; }
-__device__ __forceinline__ void store_rows4(double *p, f64x4 v)
-{
-    f64x2 lo, hi;
-    lo[0] = v[0];
-    lo[1] = v[1];
-    hi[0] = v[2];
-    hi[1] = v[3];
-    reinterpret_cast<f64x2 *>(p)[0] = lo;
-    reinterpret_cast<f64x2 *>(p)[1] = hi;
-}
-
 // ---------------------------------------------------------------------------
 // generic: one thread per element of C, any shape and alignment.
 // ---------------------------------------------------------------------------

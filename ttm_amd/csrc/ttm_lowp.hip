@@ -1125,15 +1125,17 @@ __global__ __launch_bounds__(256) void k_planes_convert(const float *__restrict_
 
 // The product: WM x WN waves, each JT x NT MFMA tiles of 16 x 16; block
 // BM = 16 JT WM rows of B by BN = 16 NT WN columns of A; stages of KS slices
-// of 32 in two LDS buffers.  Planes are padded to whole blocks and stages, so
+// of 32 in NS LDS buffers (two; three for the one-plane 128 x 256 blocks, whose
+// stages are one slice).  Planes are padded to whole blocks and stages, so
 // nothing in the loop is guarded.  LDS layout of a slice: lds_row / lds_swz,
 // filled by LDS DMA (a wave instruction moves the 1 KB of 16 physical rows;
 // see dma_b in lowp_tile for the lane order).
 //
-// Per stage: the next stage's DMA goes into the other buffer, fragments are
-// read one MFMA group ahead, and behind the last reads come the wait for that
-// DMA and the one barrier; the stage's last MFMA group runs behind it, while
-// the next stage's first fragments are read.
+// Per stage: the DMA of the stage NS - 1 ahead goes into the buffer that the
+// last stage freed, fragments are read two MFMA groups ahead, and behind the
+// last reads come the wait for the next stage's DMA and the one barrier; the
+// stage's last two MFMA groups run behind it, among the next stage's first
+// reads.
 template <int MODE, int WM, int WN, int JT, int NT, int KS, int NS>
 struct PlaneTile
 {
@@ -1161,25 +1163,21 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS, 
     constexpr int P = L::PARTS, BM = S::BM, BN = S::BN, WAVES = S::WAVES;
     static_assert(NT == 4 && JT % 4 == 0, "a lane's four column and row tiles are adjacent columns and rows");
     // (arrays of their own, so that the compiler tells a stage's reads from
-    // the other stages' DMA; those past NS are unreferenced, and so not
-    // allocated)
-    __shared__ __attribute__((aligned(16))) op sA0[KS][P][BN * LP_LDK], sA1[KS][P][BN * LP_LDK], sA2[KS][P][BN * LP_LDK],
-        sA3[KS][P][BN * LP_LDK];
-    __shared__ __attribute__((aligned(16))) op sB0[KS][P][BM * LP_LDK], sB1[KS][P][BM * LP_LDK], sB2[KS][P][BM * LP_LDK],
-        sB3[KS][P][BM * LP_LDK];
+    // the other stages' DMA; the third is unreferenced, and so not allocated,
+    // for two stages)
+    __shared__ __attribute__((aligned(16))) op sA0[KS][P][BN * LP_LDK], sA1[KS][P][BN * LP_LDK], sA2[KS][P][BN * LP_LDK];
+    __shared__ __attribute__((aligned(16))) op sB0[KS][P][BM * LP_LDK], sB1[KS][P][BM * LP_LDK], sB2[KS][P][BM * LP_LDK];
     auto buf_a = [&](auto tag) {
         constexpr int i = decltype(tag)::value % NS;
         if constexpr (i == 0) return sA0;
         else if constexpr (i == 1) return sA1;
-        else if constexpr (i == 2) return sA2;
-        else return sA3;
+        else return sA2;
     };
     auto buf_b = [&](auto tag) {
         constexpr int i = decltype(tag)::value % NS;
         if constexpr (i == 0) return sB0;
         else if constexpr (i == 1) return sB1;
-        else if constexpr (i == 2) return sB2;
-        else return sB3;
+        else return sB2;
     };
 
     unsigned jb, nb;
@@ -1320,7 +1318,7 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS, 
         else __builtin_amdgcn_s_waitcnt(0x0070);
         asm volatile("s_barrier" ::: "memory");
     };
-    static_assert(JT % 4 == 0 && (KS == 1 || (KS % 2 == 0 && NS != 3)) && NS >= 2 && NS <= 4, "fragment sets alternate");
+    static_assert(JT % 4 == 0 && (NS == 2 ? KS == 1 || KS % 2 == 0 : KS == 1 && NS == 3), "fragment sets alternate");
 #pragma unroll
     for (int p = 0; p < P; ++p) {
         fb[2][p] = fb[3][p] = v8{};
@@ -1329,7 +1327,6 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS, 
     }
     dma(0, sA0, sB0);
     if (NS > 2 && ns > 1) dma(1, buf_a(std::integral_constant<int, 1>()), buf_b(std::integral_constant<int, 1>()));
-    if (NS > 3 && ns > 2) dma(2, buf_a(std::integral_constant<int, 2>()), buf_b(std::integral_constant<int, 2>()));
     if (ns >= NS - 1) {
         constexpr int FLY = (NS - 2) * PIECES;
         __builtin_amdgcn_s_waitcnt((FLY & 15) | (FLY >> 4) << 14 | 0x0F70);
@@ -1343,12 +1340,9 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS, 
         for (; s + sizeof...(tags) <= ns; s += sizeof...(tags)) (stage(tags, s + decltype(tags)::value), ...);
         ((s + decltype(tags)::value < ns ? stage(tags, s + decltype(tags)::value) : void()), ...);
     };
-    constexpr int TRIP = NS == 3 && KS == 1 ? 6 : NS;
     using std::integral_constant;
-    if constexpr (TRIP == 2)
+    if constexpr (NS == 2)
         trip(integral_constant<int, 0>(), integral_constant<int, 1>());
-    else if constexpr (TRIP == 4)
-        trip(integral_constant<int, 0>(), integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 3>());
     else
         trip(integral_constant<int, 0>(), integral_constant<int, 1>(), integral_constant<int, 2>(), integral_constant<int, 3>(),
              integral_constant<int, 4>(), integral_constant<int, 5>());
