@@ -338,7 +338,8 @@ ttm_status_t run_host(unsigned q, unsigned p, const T *a, const size_t *na, cons
     bool const a_dev = is_device_ptr(a), b_dev = is_device_ptr(b), c_dev = is_device_ptr(c);
 
     // Device copies of the host buffers come from the per-device pool, which
-    // keeps its memory: repeated calls of one size allocate nothing new.
+    // keeps up to 8 GiB: repeated calls of one size below that allocate
+    // nothing new.
     T *da = nullptr, *db = nullptr, *dc = nullptr;
     auto release = [&]() {
         if (!a_dev && da) ws_release(da, nullptr);

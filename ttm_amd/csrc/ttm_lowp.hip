@@ -27,6 +27,7 @@
 //   accumulator element r holds D[4*lg + r][lc].
 // LDS tiles are therefore stored K-contiguous: s[row][k].
 #include "ttm_lowp.hpp"
+#include "ttm_columns.hpp"
 #include "ttm_workspace.hpp"
 
 #include <algorithm>
@@ -1379,7 +1380,8 @@ __global__ __launch_bounds__(64 * WM * WN, (PlaneTile<MODE, WM, WN, JT, NT, KS, 
     if constexpr (!TSTORE) {
         if (ncol0 >= ncols) return;
         uint64_t const k = ncol0 / w, i = ncol0 - k * w;
-        bool const whole = i + 4 <= w; // one slab (then all four columns are in range)
+        // four columns of one slab, none past the range (which may end within a slab)
+        bool const whole = i + 4 <= w && ncol0 + 4 <= ncols;
         float *cb = c + k * m * w + i;
         uint64_t off[4]; // columns of the next slabs
 #pragma unroll
@@ -1790,7 +1792,8 @@ __global__ __launch_bounds__(256) void k_fp8(const unsigned char *__restrict__ q
         uint64_t const col = n0 + 4 * lc;
         if (col >= ncols) return;
         uint64_t k = col / w, i = col - k * w;
-        bool const whole = i + 4 <= w; // one slab (then all four columns are in range)
+        // four columns of one slab, none past the range (which may end within a slab)
+        bool const whole = i + 4 <= w && col + 4 <= ncols;
         float *cb = c + k * m * w + i;
         uint64_t off[4];
 #pragma unroll
@@ -2023,10 +2026,25 @@ constexpr PlaneBlock plane_block(PlaneShape shape, int parts)
     if (shape == PLANES_128) return {2, 2, 4, 4, ks, 2};
     return parts == 1 ? PlaneBlock{1, 4, 8, 4, 1, 3} : PlaneBlock{2, 4, 8, 4, ks, 2};
 }
+// Columns of one range (for_columns) of a product whose copy of A takes
+// `bytes` per column: 4 GiB, well within what the workspace pool keeps (memory
+// beyond that is mapped and cleared again after every synchronization: FP8 on
+// A 2048x2048x4608, 20 GB of quantized A at once, 22 ms a call where it is
+// kept, 476 ms where it is not), but at least `blocks` columns to fill the
+// chip, for contractions of many thousand indices.
+uint64_t range_columns(uint64_t bytes, uint64_t blocks)
+{
+    constexpr uint64_t limit = 4ull << 30;
+    return std::max<uint64_t>(limit / bytes, blocks) / 256 * 256 + 256;
+}
+
 struct PlaneGeom
 {
-    uint64_t bm, bn, ldk, rows_a, rows_b, plane_a, plane_b;
-    size_t bytes; // of both operands' planes
+    uint64_t bm, bn, ldk, rows_b, plane_b;
+    uint64_t range;           // columns of a range at most (for_columns)
+    uint64_t rows_a, plane_a; // of a range
+    uint64_t all_rows;        // of A's planes, if it were one range
+    size_t bytes, all_bytes;  // of both operands' planes: A's of a range, all of them
 };
 PlaneGeom plane_geom(const Fold &f, int parts)
 {
@@ -2037,26 +2055,28 @@ PlaneGeom plane_geom(const Fold &f, int parts)
     uint64_t const kq = parts == 1 ? 64 : 32; // contraction indices per stage
     g.ldk = (f.nq + kq - 1) / kq * kq;
     uint64_t const ncols = f.outer * f.w;
-    g.rows_a = (ncols + g.bn - 1) / g.bn * g.bn;
     g.rows_b = (f.m + g.bm - 1) / g.bm * g.bm;
-    g.plane_a = g.rows_a * g.ldk;
     g.plane_b = g.rows_b * g.ldk;
+    g.range = range_columns((uint64_t)parts * 2 * g.ldk, g.bn * (2 * (uint64_t)device_cus() * g.bm / g.rows_b));
+    g.rows_a = (widest_range(f, g.range) + g.bn - 1) / g.bn * g.bn;
+    g.plane_a = g.rows_a * g.ldk;
+    g.all_rows = (ncols + g.bn - 1) / g.bn * g.bn;
     g.bytes = (size_t)parts * (g.plane_a + g.plane_b) * 2;
+    g.all_bytes = (size_t)parts * (g.all_rows * g.ldk + g.plane_b) * 2;
     return g;
 }
 int mode_parts(ttm_precision_t prec) { return prec == TTM_PREC_BF16X3 ? 3 : prec == TTM_PREC_FP16X2 ? 2 : 1; }
 
 template <int MODE, PlaneShape SHAPE>
-void launch_planes_shape(const Fold &f, const PlaneGeom &g, const typename Lp<MODE>::op *as,
+void launch_planes_shape(const Fold &f, const PlaneGeom &g, uint64_t ncols, const typename Lp<MODE>::op *as,
                          const typename Lp<MODE>::op *bs, float *c, const int *exps, hipStream_t s)
 {
     constexpr PlaneBlock B = plane_block(SHAPE, Lp<MODE>::PARTS);
     unsigned const nj = (unsigned)(g.rows_b / B.bm());
-    unsigned const total = nj * (unsigned)(g.rows_a / B.bn());
+    unsigned const total = nj * (unsigned)((ncols + B.bn() - 1) / B.bn());
     dim3 const threads(64 * B.wm * B.wn);
     bool const ts = f.w == 1;
     int const c_vec = (reinterpret_cast<uintptr_t>(c) & 15u) == 0 && (ts ? f.m : f.w) % 4 == 0;
-    uint64_t const ncols = f.outer * f.w;
     if (ts)
         hipLaunchKernelGGL((k_planes<MODE, B.wm, B.wn, B.jt, B.nt, B.ks, B.ns, true>), dim3(total), threads, 0, s, as,
                            g.plane_a, bs, g.plane_b, g.ldk, c, ncols, f.w, f.m, nj, total, c_vec, exps);
@@ -2072,7 +2092,6 @@ ttm_status_t launch_planes(const Fold &f, const float *a, const float *b, float 
     constexpr int P = Lp<MODE>::PARTS;
     constexpr bool SCALED = MODE == LP_FP16X2;
     PlaneGeom const g = plane_geom(f, P);
-    uint64_t const ncols = f.outer * f.w;
     size_t const planes_bytes = (g.bytes + 255) / 256 * 256;
     ScalePass const sp = SCALED ? scale_pass(f, true) : ScalePass();
     void *ws = nullptr;
@@ -2088,17 +2107,22 @@ ttm_status_t launch_planes(const Fold &f, const float *a, const float *b, float 
     auto blocks = [&](uint64_t rows, bool along) {
         return (unsigned)(rows / 64) * ((nsl + (along ? 3 : 1)) / (along ? 4 : 2));
     };
-    unsigned const blocks_a = blocks(g.rows_a, f.w == 1), blocks_b = blocks(g.rows_b, !f.b_colmajor);
-    hipLaunchKernelGGL(k_planes_convert<MODE>, dim3(blocks_a + blocks_b), dim3(256), 0, s, a, as, ncols, f.w, g.plane_a,
-                       b, bs, f.m, f.b_colmajor ? 0 : 1, g.plane_b, f.nq, nsl, blocks_a, exps);
     PlaneShape const shape = plane_shape(f, P);
-    if (shape == PLANES_64) {
-        launch_planes_shape<MODE, PLANES_64>(f, g, as, bs, c, exps, s);
-    } else if (shape == PLANES_128) {
-        launch_planes_shape<MODE, PLANES_128>(f, g, as, bs, c, exps, s);
-    } else {
-        if constexpr (P < 3) launch_planes_shape<MODE, PLANES_256>(f, g, as, bs, c, exps, s);
-    }
+    bool first = true; // B's planes are converted with the first range
+    for_columns(f, g.range, [&](ColumnRange const &r) {
+        unsigned const blocks_a = blocks((r.ncols + g.bn - 1) / g.bn * g.bn, f.w == 1);
+        unsigned const blocks_b = first ? blocks(g.rows_b, !f.b_colmajor) : 0;
+        first = false;
+        hipLaunchKernelGGL(k_planes_convert<MODE>, dim3(blocks_a + blocks_b), dim3(256), 0, s, a + r.a, as, r.ncols, f.w,
+                           g.plane_a, b, bs, f.m, f.b_colmajor ? 0 : 1, g.plane_b, f.nq, nsl, blocks_a, exps);
+        if (shape == PLANES_64) {
+            launch_planes_shape<MODE, PLANES_64>(f, g, r.ncols, as, bs, c + r.c, exps, s);
+        } else if (shape == PLANES_128) {
+            launch_planes_shape<MODE, PLANES_128>(f, g, r.ncols, as, bs, c + r.c, exps, s);
+        } else {
+            if constexpr (P < 3) launch_planes_shape<MODE, PLANES_256>(f, g, r.ncols, as, bs, c + r.c, exps, s);
+        }
+    });
     hipError_t const e = hipGetLastError();
     ws_release(ws, s);
     if (e != hipSuccess) {
@@ -2112,10 +2136,12 @@ ttm_status_t launch_planes(const Fold &f, const float *a, const float *b, float 
 // copy of A's slice then serves twice as many rows of C), else 64.
 int fp8_block_rows(const Fold &f) { return f.m > 64 ? 128 : 64; }
 
-// Workspace of the quantized operands and their scales.
+// Workspace of the quantized operands and their scales: A's of a range of at
+// most `range` columns (for_columns), and of all of them.
 struct Fp8Bytes
 {
-    size_t qb, sb, qa, sa;
+    uint64_t range;
+    size_t qb, sb, qa, sa, all;
     size_t total() const { return qb + sb + qa + sa; }
 };
 Fp8Bytes fp8_bytes(const Fold &f)
@@ -2123,57 +2149,66 @@ Fp8Bytes fp8_bytes(const Fold &f)
     uint64_t const bm = (uint64_t)fp8_block_rows(f);
     uint64_t const ldq = (f.nq + 127) / 128 * 128;
     uint64_t const rows_b = (f.m + bm - 1) / bm * bm;
-    uint64_t const rows_a = (f.outer * f.w + 63) / 64 * 64;
     auto round256 = [](uint64_t x) { return (x + 255) / 256 * 256; };
-    return {round256(rows_b * ldq), round256(rows_b * (ldq / 32)), round256(rows_a * ldq),
-            round256(rows_a * (ldq / 32))};
+    auto round64 = [](uint64_t x) { return (x + 63) / 64 * 64; };
+    Fp8Bytes by;
+    by.range = range_columns(ldq + ldq / 32, 64 * (4 * (uint64_t)device_cus() * bm / rows_b));
+    uint64_t const rows_a = round64(widest_range(f, by.range)), all = round64(f.outer * f.w);
+    by.qb = round256(rows_b * ldq);
+    by.sb = round256(rows_b * (ldq / 32));
+    by.qa = round256(rows_a * ldq);
+    by.sa = round256(rows_a * (ldq / 32));
+    by.all = by.qb + by.sb + round256(all * ldq) + round256(all * (ldq / 32));
+    return by;
 }
 
 // A and B quantized once per product (k_fp8_split_a_*, k_fp8_split_b) into
 // pooled workspace: N_A + m n_q bytes (rounded up to whole blocks and
-// slices) plus a scale byte per 32 of them; then the tiles.
+// slices) plus a scale byte per 32 of them; then the tiles.  A in ranges of
+// columns of about 4 GiB.
 template <bool TN, bool ANY>
 ttm_status_t launch_fp8(const Fold &f, const float *a, const float *b, float *c, hipStream_t s)
 {
     uint64_t const bm = (uint64_t)fp8_block_rows(f);
-    uint64_t const ncols = TN ? f.outer : f.outer * f.w;
+    Fp8Bytes const by = fp8_bytes(f);
     unsigned const nj = (unsigned)((f.m + bm - 1) / bm);
-    unsigned const total = nj * (unsigned)((ncols + 63) / 64);
     uint64_t const ldq = (f.nq + 127) / 128 * 128;
     uint64_t const rows = (uint64_t)nj * bm;
-    uint64_t const rows_a = (ncols + 63) / 64 * 64;
     uint64_t const split_blocks = (rows * (ldq / 32) + 255) / 256;
-    uint64_t const split_a_blocks = (rows_a / 64) * (ldq / 128);
+    uint64_t const split_a_blocks = (widest_range(f, by.range) + 63) / 64 * (ldq / 128);
     if (split_blocks >= (1ull << 31) || split_a_blocks >= (1ull << 31)) {
         set_error(TTM_ERR_ARGUMENT, "operands too large for the FP8 kernels");
         return TTM_ERR_ARGUMENT;
     }
-    Fp8Bytes const by = fp8_bytes(f);
-    size_t const bytes_qb = by.qb, bytes_sb = by.sb, bytes_qa = by.qa, bytes_sa = by.sa;
     void *ws = nullptr;
-    if (ttm_status_t const st = ws_acquire(bytes_qb + bytes_sb + bytes_qa + bytes_sa, s, &ws,
-                                           "workspace for the quantized operands");
+    if (ttm_status_t const st = ws_acquire(by.total(), s, &ws, "workspace for the quantized operands");
         st != TTM_SUCCESS)
         return st;
     unsigned char *const qb = static_cast<unsigned char *>(ws);
-    unsigned char *const sb = qb + bytes_qb;
-    unsigned char *const qa = sb + bytes_sb;
-    unsigned char *const sa = qa + bytes_qa;
+    unsigned char *const sb = qb + by.qb;
+    unsigned char *const qa = sb + by.sb;
+    unsigned char *const sa = qa + by.qa;
     hipLaunchKernelGGL(k_fp8_split_b, dim3((unsigned)split_blocks), dim3(256), 0, s, b, qb, sb, f.m, f.nq,
                        f.b_stride_j(), f.b_stride_l(), ldq, rows);
-    if constexpr (TN)
-        hipLaunchKernelGGL(k_fp8_split_a_rows<ANY>, dim3((unsigned)split_a_blocks), dim3(256), 0, s, a, qa, sa, ncols,
-                           f.nq, ldq, ldq / 128);
-    else
-        hipLaunchKernelGGL(k_fp8_split_a_cols<ANY>, dim3((unsigned)split_a_blocks), dim3(256), 0, s, a, qa, sa, ncols,
-                           f.nq, f.w, ldq, ldq / 128);
-    int const c_vec = (reinterpret_cast<uintptr_t>(c) & 15u) == 0 && (TN ? f.m : f.w) % 4 == 0;
-    if (bm == 128)
-        hipLaunchKernelGGL((k_fp8<TN, 128>), dim3(total), dim3(256), 0, s, qa, sa, qb, sb, ldq, c, ncols, f.nq, f.w,
-                           f.m, nj, total, c_vec);
-    else
-        hipLaunchKernelGGL((k_fp8<TN, 64>), dim3(total), dim3(256), 0, s, qa, sa, qb, sb, ldq, c, ncols, f.nq, f.w,
-                           f.m, nj, total, c_vec);
+    for_columns(f, by.range, [&](ColumnRange const &r) {
+        uint64_t const blocks_n = (r.ncols + 63) / 64;
+        dim3 const split_a((unsigned)(blocks_n * (ldq / 128)));
+        if constexpr (TN)
+            hipLaunchKernelGGL(k_fp8_split_a_rows<ANY>, split_a, dim3(256), 0, s, a + r.a, qa, sa, r.ncols, f.nq, ldq,
+                               ldq / 128);
+        else
+            hipLaunchKernelGGL(k_fp8_split_a_cols<ANY>, split_a, dim3(256), 0, s, a + r.a, qa, sa, r.ncols, f.nq, f.w,
+                               ldq, ldq / 128);
+        unsigned const total = nj * (unsigned)blocks_n;
+        float *const cr = c + r.c;
+        int const c_vec = (reinterpret_cast<uintptr_t>(cr) & 15u) == 0 && (TN ? f.m : f.w) % 4 == 0;
+        if (bm == 128)
+            hipLaunchKernelGGL((k_fp8<TN, 128>), dim3(total), dim3(256), 0, s, qa, sa, qb, sb, ldq, cr, r.ncols, f.nq,
+                               f.w, f.m, nj, total, c_vec);
+        else
+            hipLaunchKernelGGL((k_fp8<TN, 64>), dim3(total), dim3(256), 0, s, qa, sa, qb, sb, ldq, cr, r.ncols, f.nq,
+                               f.w, f.m, nj, total, c_vec);
+    });
     hipError_t const e = hipGetLastError();
     ws_release(ws, s);
     if (e != hipSuccess) {
@@ -2183,8 +2218,9 @@ ttm_status_t launch_fp8(const Fold &f, const float *a, const float *b, float *c,
     return TTM_SUCCESS;
 }
 
-// Largest workspace of a product over planes; beyond it the padding of a
-// degenerate shape (a column or a row against a whole tile) is the bulk.
+// Most bytes of planes (all ranges together) that a product may write; beyond
+// it the padding of a degenerate shape (a column or a row against a whole tile)
+// is the bulk.
 constexpr size_t kAnyMaxBytes = 32ull << 30;
 
 template <int MODE>
@@ -2213,10 +2249,10 @@ bool planes_support(const Fold &f, ttm_precision_t prec)
 {
     if (f.nq >= (1ull << 22)) return false;
     if (prec == TTM_PREC_FP8_E4M3)
-        return fp8_bytes(f).total() <= kAnyMaxBytes && ((f.outer * f.w + 63) / 64) * ((f.m + 63) / 64) < (1ull << 31);
+        return fp8_bytes(f).all <= kAnyMaxBytes && ((f.outer * f.w + 63) / 64) * ((f.m + 63) / 64) < (1ull << 31);
     PlaneGeom const g = plane_geom(f, mode_parts(prec));
     // blocks of the conversions: at least 2048 elements each
-    return g.bytes <= kAnyMaxBytes && (g.rows_a / g.bn) * (g.rows_b / g.bm) < (1ull << 31) &&
+    return g.all_bytes <= kAnyMaxBytes && (g.rows_a / g.bn) * (g.rows_b / g.bm) < (1ull << 31) &&
            g.plane_a / 2048 + g.plane_b / 2048 + 2 < (1ull << 31);
 }
 
@@ -2260,7 +2296,7 @@ bool generic_faster(const Fold &f, ttm_precision_t prec)
         ld = (double)((f.nq + 127) / 128 * 128);
     } else {
         PlaneGeom const g = plane_geom(f, mode_parts(prec));
-        rows_a = (double)g.rows_a;
+        rows_a = (double)g.all_rows;
         rows_b = (double)g.rows_b;
         ld = (double)g.ldk;
     }

@@ -3,11 +3,11 @@
 //
 // By default a call takes its workspace from a per-device stream-ordered
 // memory pool that keeps its memory between calls, up to 8 GiB across a
-// synchronization (hipMallocFromPoolAsync / hipFreeAsync), so a steady stream of products allocates nothing new from
-// the driver after the first.  An allocation-free entry point instead binds a
-// fixed device region for the duration of its call (ScratchScope); requests
-// are then carved from that region and fail with TTM_ERR_ALLOC when it is too
-// small.
+// synchronization (hipMallocFromPoolAsync / hipFreeAsync), so a steady stream
+// of products allocates nothing new from the driver after the first.  An
+// allocation-free entry point instead binds a fixed device region for the
+// duration of its call (ScratchScope); requests are then carved from that
+// region and fail with TTM_ERR_ALLOC when it is too small.
 #pragma once
 
 #include <hip/hip_runtime.h>
