@@ -8,6 +8,7 @@ import pathlib
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
 
 ROOT = pathlib.Path(__file__).resolve().parents[1]
@@ -26,6 +27,39 @@ def test_ranges_cover_every_column_once():
     assert res.returncode == 0, res.stderr
     run = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert run.returncode == 0 and run.stdout.startswith("0 violations"), run.stdout + run.stderr
+
+
+@pytest.mark.parametrize("outer,w,i0,ncols", [(1, 1537, 0, 1537), (2, 1539, 1280, 259), (1, 1282, 1024, 258), (3, 5, 0, 15),
+                                              (4, 259, 0, 1036), (2, 512, 256, 256), (1, 770, 512, 258)])
+def test_nn_stores_of_a_range_cover_its_columns_once(outer, w, i0, ncols):
+    """The C[j][n] epilogue of k_planes and k_fp8 on a range (i0: its first
+    column within its slab, 0 for whole slabs): a lane's four columns go out as
+    one vector only inside one slab and inside the range, so that no element
+    of the next row or beyond C is written."""
+    m, BN = 2, 128
+    seen = np.zeros(outer * m * w, dtype=int)
+    c0 = i0  # C's element of the range's first column (slab 0)
+    for ncol0 in range(0, -(-ncols // BN) * BN, 4):
+        if ncol0 >= ncols:
+            continue
+        k, i = divmod(ncol0, w)
+        whole = i + 4 <= w and ncol0 + 4 <= ncols
+        for j in range(m):
+            base = c0 + k * m * w + i + j * w
+            for nt in range(4):
+                ii, kk = i + nt, 0
+                while ii >= w:
+                    ii, kk = ii - w, kk + 1
+                if whole:
+                    seen[base + nt] += 1
+                elif ncol0 + nt < ncols:
+                    seen[base + kk * m * w + ii - i] += 1
+    want = np.zeros_like(seen).reshape(outer, m, w)
+    if i0:
+        want[0, :, i0:i0 + ncols] = 1
+    else:
+        want[: ncols // w, :, :] = 1
+    assert np.array_equal(seen.reshape(outer, m, w), want)
 
 
 # first-order extents, q: q fastest, slabs of 33, one slab, two slabs wider than a range
