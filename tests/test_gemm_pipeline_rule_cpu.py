@@ -23,23 +23,21 @@ CASES = [
     ([512, 95, 512], 2, 128, "row", "f32", False), ([512, 96, 512], 2, 128, "row", "f32", True),
     ([512, 191, 2048], 2, 64, "row", "f32", False), ([512, 192, 2048], 2, 64, "row", "f32", True),
     ([384, 65536], 1, 64, "col", "f64", True), ([383, 65536], 1, 64, "col", "f64", False),
-    # guarded blocks of a column-major B: rows that no vector ends at, in one or two row blocks
-    ([512, 400, 512], 2, 17, "col", "f32", False), ([512, 400, 512], 2, 20, "col", "f32", True),
-    ([512, 400, 512], 2, 127, "col", "f32", False), ([512, 400, 512], 2, 129, "col", "f32", False),
-    ([512, 400, 512], 2, 299, "col", "f32", True), ([512, 400, 512], 2, 129, "row", "f32", True),
-    ([512, 400, 512], 2, 41, "col", "f64", False), ([512, 400, 512], 2, 42, "col", "f64", True),
+    # rows that no vector of a column-major B ends at
+    ([512, 400, 2048], 2, 17, "col", "f32", True), ([512, 400, 512], 2, 127, "col", "f32", True),
+    ([512, 400, 512], 2, 451, "col", "f32", True), ([512, 400, 512], 2, 41, "col", "f64", True),
     # slab ends inside most blocks
     ([131, 400, 2000], 2, 128, "col", "f32", False), ([131, 400, 2000], 2, 128, "row", "f32", True),
     ([2051, 400, 128], 2, 128, "col", "f32", True),
-    # ... except where both kernels take two rounds
-    ([128, 400, 900], 2, 41, "col", "f64", True), ([128, 400, 1025], 2, 41, "col", "f64", False),
-    ([128, 400, 768], 2, 41, "col", "f64", False), ([256, 400, 900], 2, 41, "col", "f32", False),
+    # ... but for the tiles of one row of waves where both kernels take two rounds
+    ([131, 400, 900], 2, 41, "col", "f64", True), ([131, 400, 1000], 2, 41, "col", "f64", False),
+    ([131, 400, 700], 2, 41, "col", "f64", False), ([131, 400, 1800], 2, 41, "col", "f32", False),
+    ([131, 400, 1800], 2, 63, "col", "f32", True),
     # more than two, at most three blocks per compute unit
     ([256, 400, 512], 2, 20, "row", "f32", True), ([256, 400, 513], 2, 20, "row", "f32", False),
     ([256, 400, 768], 2, 20, "row", "f32", False), ([256, 400, 769], 2, 20, "row", "f32", True),
     ([256, 400, 600], 2, 40, "row", "f32", True), ([128, 400, 600], 2, 20, "row", "f64", False),
-    ([400, 128 * 600], 1, 20, "row", "f64", False), ([400, 128 * 600], 1, 41, "col", "f64", False),
-    ([400, 128 * 500], 1, 41, "col", "f64", True), ([400, 128 * 800], 1, 41, "col", "f64", True),
+    ([400, 128 * 600], 1, 20, "row", "f64", False), ([400, 128 * 600], 1, 41, "col", "f64", True),
 ]
 
 

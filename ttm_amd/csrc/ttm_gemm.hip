@@ -313,11 +313,13 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     // (every vector of a whole slice lies inside its row or column); the TT
     // tiles of the grouped kernels keep the aligned-only rule.
     // Rows past m (the last row block of a ragged m) read row m - 1 of a
-    // row-major B, or the column's last whole vector of a column-major B
-    // (which needs m % VEC == 0, so that no vector is part in and part out
-    // of range), and their products are never stored: such blocks keep the
-    // unguarded loop.
-    bool const rows_ok = j0 + BM <= m || !BCOL || m % VEC == 0;
+    // row-major B, or the column's last whole vector of a column-major B, and
+    // their products are never stored: such blocks keep the unguarded loop.
+    // A vector of a column-major B that is part in and part out of range
+    // (m % VEC != 0) reads on into the next column; only the slice of the
+    // last column, whose vector would leave B, is guarded (`straddle`).
+    bool const straddle = BCOL && j0 + BM > m && m % VEC != 0;
+    bool const rows_ok = !straddle || m > (uint64_t)VEC;
     bool full = n0 + BN <= ncols && rows_ok &&
                 (VIEW == VIEW_TT ? (a_vec && b_vec_ok) : (TN || a_vec || !PAD));
     if constexpr (PAD) {
@@ -463,7 +465,7 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
         uint64_t const jj = b_in[e] ? (uint64_t)b_col[e] : 0;
         uint64_t const ll = b_in[e] ? (uint64_t)b_row[e] : 0;
         uint64_t const j = j0 + jj;
-        b_fix[e] = BCOL ? (j + VEC <= m ? j : m - VEC) + ll * m : (j < m ? j : m - 1) * ld + ll;
+        b_fix[e] = BCOL ? (j < m ? j : m - VEC) + ll * m : (j < m ? j : m - 1) * ld + ll;
     }
     uint64_t const b_step = BCOL ? m : 1; // B offset per contraction index
     auto load_full = [&](uint64_t l0, auto set) {
@@ -493,11 +495,14 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
             else rb[S][e] = ldg<typename Gt::vec_u>(bp);
         }
     };
-    // The ragged last slice of an interior tile (nq % BK != 0, at least one
-    // whole slice before it): the same vectors read at in-range addresses,
-    // with the shift and the count of valid elements kept for the store.
-    // Vectors along n (or j) are whole or past the last index; vectors along
-    // l are moved back to the row's last VEC elements.
+    // The last slice of an interior tile that is not whole (nq % BK != 0) or
+    // holds the last column of a straddling B, with at least one whole slice
+    // before it: the same vectors read at in-range addresses, with the shift
+    // and the count of valid elements kept for the store.  Vectors along n (or
+    // j) are whole or past the last index, but for the last column's vector
+    // across row m, which is moved back to the end of B (its elements past row
+    // m are some of B's: their rows are never stored); vectors along l are
+    // moved back to the row's last VEC elements.
     auto load_ragged = [&](uint64_t l0, auto set) {
         constexpr int S = decltype(set)::value;
         using VU = typename Gt::vec_u;
@@ -520,8 +525,14 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
 #pragma unroll
         for (int e = 0; e < B_PER; ++e) {
             uint64_t const ll = b_in[e] ? (uint64_t)b_row[e] : 0;
-            if constexpr (BCOL) across_l(b + b_fix[e] - ll * m, l0 + ll, m, rb[S][e], rb_dm[S][e]);
-            else along_l(b + b_fix[e] - ll, l0 + ll, rb[S][e], rb_dm[S][e]);
+            if constexpr (BCOL) {
+                uint64_t const l = l0 + ll, j = b_fix[e] - ll * m;
+                uint64_t const at = j + (l < nq ? l : nq - 1) * m, end = nq * m - VEC;
+                rb[S][e] = ldg<VU>(b + (at < end ? at : end));
+                rb_dm[S][e] = (at < end ? 0 : (int)(at - end)) | (l < nq ? DM_WHOLE : 0);
+            } else {
+                along_l(b + b_fix[e] - ll, l0 + ll, rb[S][e], rb_dm[S][e]);
+            }
         }
     };
 
@@ -676,7 +687,7 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     // Slice s (in LDS buffer BUF, its first fragments in set 0).  LOAD: load
     // slice s + 1 + PF into the registers that the store of slice s + 1 frees;
     // TAIL: near the end, where a slice may be the ragged one or not exist.
-    uint64_t const nwhole = nq / BK;
+    uint64_t const nwhole = straddle ? (nq - 1) / BK : nq / BK;
     auto slice = [&](auto buf_tag, auto tail_tag, uint64_t s) {
         constexpr int BUF = decltype(buf_tag)::value;
         constexpr bool TAIL = decltype(tail_tag)::value;
@@ -1121,19 +1132,20 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 //           0.91-0.98, K = 256 0.92-1.03, K = 128 1.05-1.28
 //           16 to 96 rows: K = 384 0.81-1.05, K = 256 0.82-1.07
 //
-// Only interior blocks run it.  Where most blocks are guarded (rows past m of
-// a column-major B that no vector ends at, slab ends inside most blocks) a
-// block waits for each slice's loads in turn, and the pipelined kernels, with
-// more registers, have two blocks on a CU where the plain ones have three or
-// four: what counts is in how many rounds the grid runs.  B column-major,
-// K = 400, NN view: up to two blocks per CU 0.97-1.02, beyond 1.01-1.54
-// (float32, 17 to 95 rows, 3000 blocks: 1.06-1.38), except that both kernels
-// take two rounds for more than three and at most four blocks per CU, where
-// the float64 tiles of one row of waves and the 64-row float32 one gain
-// (0.78-0.97).  In the TN view guarded blocks lose for more than two and at
-// most three blocks per CU (0.96-1.25, float32 96 rows 1.43; elsewhere
-// 0.59-1.00), and so do blocks of 17..32 rows anywhere, bound by their loads
-// (K = 192..640, float32: 1.04-1.29, elsewhere 0.81-1.11).
+// Only interior blocks run it, and the pipelined kernels, with more registers,
+// have two blocks on a CU where the plain ones have three or four: what counts
+// beside the loop is in how many rounds the grid runs.
+//   - Slab ends inside most blocks: those blocks wait for each slice's loads in
+//     turn.  B column-major, K = 400: up to two blocks per CU 0.97-1.02, beyond
+//     1.01-1.54 (float32, 17 to 95 rows, 3000 blocks: 1.06-1.38), except that
+//     both kernels take two rounds for more than three and at most four blocks
+//     per CU, where the float64 tiles of one row of waves and the 64-row
+//     float32 one gain (0.78-0.97).
+//   - Blocks of 17..32 rows are bound by their loads, which three blocks hide
+//     as well as the pipelining does: where the plain kernel runs in one round
+//     and the pipelined one in two (K = 200 to 4000, 2.1 to 3 blocks per CU)
+//     float32 0.98-1.08, read at element alignment 1.02-1.30, TN view
+//     0.94-1.22, float64 0.96-1.26.
 bool gemm_pipelined(const Fold &f, bool is_double, const Geom &g, const Split &sp)
 {
     Config const &cfg = g.cfg;
@@ -1142,10 +1154,9 @@ bool gemm_pipelined(const Fold &f, bool is_double, const Geom &g, const Split &s
     uint64_t const blocks = (uint64_t)g.nj * g.nn * sp.splits, cus = (uint64_t)device_cus();
     bool const one_round = blocks > 2 * cus && blocks <= 3 * cus; // for the plain kernels only
     bool const two_rounds = blocks > 3 * cus && blocks <= 4 * cus; // for both
-    bool const guarded = (f.b_colmajor && f.m % vec != 0 && g.nj <= 2) ||
-                         (g.pad && f.w % vec != 0 && g.wp < 2 * (uint64_t)g.bn());
-    if (guarded && f.b_colmajor)
-        return g.tn ? !one_round : two_rounds && cfg.waves_m == 1 && (is_double || cfg.jt == 4);
+    // slab ends inside most blocks
+    bool const guarded = g.pad && f.w % vec != 0 && g.wp < 2 * (uint64_t)g.bn();
+    if (guarded && f.b_colmajor) return two_rounds && cfg.waves_m == 1 && (is_double || cfg.jt == 4);
     return !(cfg.jt == 2 && one_round);
 }
 
