@@ -330,10 +330,17 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
             full = __syncthreads_and(whole ? 1 : 0) != 0;
         }
     }
-    uint64_t a_fix[A_PER]; // A offset of the thread's vector in slice 0
+    // A offset of the thread's vector e in slice 0.  NN: the vectors lie in one
+    // column, A_ROWS rows apart, so only the first one's is kept (the rest of
+    // the offset is uniform: the float64 128 x 128 pipelined tile has no
+    // registers to spare).
+    constexpr uint64_t A_ROWS = 256 / (BN / VEC);
+    uint64_t a_first[TN ? A_PER : 1];
 #pragma unroll
-    for (int e = 0; e < A_PER; ++e) a_fix[e] = TN ? a_base[e] + a_row[e] : a_base[e] + (uint64_t)a_row[e] * w;
-    uint64_t const a_step = TN ? 1 : w; // A offset per contraction index
+    for (int e = 0; e < (TN ? A_PER : 1); ++e) a_first[e] = TN ? a_base[e] + a_row[e] : a_base[e] + (uint64_t)a_row[e] * w;
+    auto a_at = [&](int e, uint64_t l0) { // element offset of vector e in the slice at l0
+        return TN ? a_first[TN ? e : 0] + l0 : a_first[0] + (l0 + A_ROWS * e) * w;
+    };
 
     auto load_tiles = [&](uint64_t l0, auto set) {
         constexpr int S = decltype(set)::value;
@@ -476,17 +483,17 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
                 if (!a_vec) {
                     // element-aligned whole vectors
                     using VU = typename Gt::vec_u;
-                    ra[S][e] = nt_a ? (V)ldg_nt<VU>(a + a_fix[e] + l0 * a_step) : (V)ldg<VU>(a + a_fix[e] + l0 * a_step);
+                    ra[S][e] = nt_a ? (V)ldg_nt<VU>(a + a_at(e, l0)) : (V)ldg<VU>(a + a_at(e, l0));
                     continue;
                 }
             }
             if constexpr (TN && VIEW != VIEW_TT) {
                 if (!a_vec) {
-                    ra[S][e] = ldg<typename Gt::vec_u>(a + a_fix[e] + l0 * a_step);
+                    ra[S][e] = ldg<typename Gt::vec_u>(a + a_at(e, l0));
                     continue;
                 }
             }
-            ra[S][e] = load_a(a + a_fix[e] + l0 * a_step);
+            ra[S][e] = load_a(a + a_at(e, l0));
         }
 #pragma unroll
         for (int e = 0; e < B_PER; ++e) {
@@ -519,8 +526,8 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
 #pragma unroll
         for (int e = 0; e < A_PER; ++e) {
             uint64_t const l = l0 + a_row[e];
-            if constexpr (TN) along_l(a + a_fix[e] - a_row[e], l, ra[S][e], ra_dm[S][e]);
-            else across_l(a + a_fix[e] - (uint64_t)a_row[e] * w, l, w, ra[S][e], ra_dm[S][e]);
+            if constexpr (TN) along_l(a + a_first[e] - a_row[e], l, ra[S][e], ra_dm[S][e]);
+            else across_l(a + a_first[0] - (uint64_t)a_row[0] * w, l, w, ra[S][e], ra_dm[S][e]);
         }
 #pragma unroll
         for (int e = 0; e < B_PER; ++e) {
