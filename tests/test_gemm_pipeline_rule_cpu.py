@@ -37,7 +37,9 @@ CASES = [
     ([256, 400, 512], 2, 20, "row", "f32", True), ([256, 400, 513], 2, 20, "row", "f32", False),
     ([256, 400, 768], 2, 20, "row", "f32", False), ([256, 400, 769], 2, 20, "row", "f32", True),
     ([256, 400, 600], 2, 40, "row", "f32", True), ([128, 400, 600], 2, 20, "row", "f64", False),
-    ([400, 128 * 600], 1, 20, "row", "f64", False), ([400, 128 * 600], 1, 41, "col", "f64", True),
+    ([400, 128 * 600], 1, 20, "row", "f64", False), ([400, 128 * 600 - 1], 1, 20, "row", "f64", True),
+    ([200, 256 * 600], 1, 32, "col", "f32", False), ([200, 256 * 600 + 1], 1, 32, "col", "f32", True),
+    ([400, 128 * 600], 1, 41, "col", "f64", True),
 ]
 
 

@@ -1152,7 +1152,11 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 //     as well as the pipelining does: where the plain kernel runs in one round
 //     and the pipelined one in two (K = 200 to 4000, 2.1 to 3 blocks per CU)
 //     float32 0.98-1.08, read at element alignment 1.02-1.30, TN view
-//     0.94-1.22, float64 0.96-1.26.
+//     0.94-1.22, float64 0.96-1.26.  In the TN view a last block of fewer
+//     columns, alone with its guarded slices, is what the grid waits for, and
+//     the plain loop is the slower one there: [K, n] x_1 with n no multiple of
+//     the block's columns, K = 200 to 4000: float32 0.78-0.98, float64
+//     0.67-0.94 ([1000, 66000] m = 17: 221 against 158 us).
 bool gemm_pipelined(const Fold &f, bool is_double, const Geom &g, const Split &sp)
 {
     Config const &cfg = g.cfg;
@@ -1164,7 +1168,7 @@ bool gemm_pipelined(const Fold &f, bool is_double, const Geom &g, const Split &s
     // slab ends inside most blocks
     bool const guarded = g.pad && f.w % vec != 0 && g.wp < 2 * (uint64_t)g.bn();
     if (guarded && f.b_colmajor) return two_rounds && cfg.waves_m == 1 && (is_double || cfg.jt == 4);
-    return !(cfg.jt == 2 && one_round);
+    return !(cfg.jt == 2 && one_round && !(g.tn && g.ncols % (uint64_t)g.bn() != 0));
 }
 
 template <class T, int JT, int NT, int WM, int BK, bool TN, bool BCOL>
