@@ -295,8 +295,9 @@ __device__ __forceinline__ void gemm_tile(const T *__restrict__ a, const T *__re
     // slice s + 2 are issued while slice s is multiplied) whose slice is at
     // most five vectors per thread, or the 16-row TN tile of one product; one
     // otherwise (larger sets would spill in the grouped kernels).  The 48-row
-    // pipelined tiles take two as well (A 1024x1024x512, m = 48: float32 546 ->
-    // 532 us NN, float64 1024 -> 990 us TN); at 64 rows it changed nothing.
+    // pipelined tiles take two as well (A 1024x1024x512, m = 48, after a cache
+    // flush, one -> two: TN view float32 489 -> 467 us, float64 947 -> 922 us, NN
+    // view 469 -> 469 and 822 -> 836 us); at 64 rows it changed nothing.
     constexpr int PF = (PIPE && WAVES_M == 1 && JT == 3) ? 2 : (JT <= 2 && (A_PER + B_PER <= 5 || (VIEW == VIEW_TN && JT == 1))) ? 2 : 1;
     V ra[PF][A_PER], rb[PF][B_PER];
     // Guarded slices: shift d and count nvalid of each vector (d | nvalid << 8),
@@ -1041,8 +1042,9 @@ Config pick_config(const Fold &f, bool is_double)
     // and 167 / 146 registers, three blocks per CU
     if (is_double && f.m > 16 && f.m <= 32) return {2, 2, 1, 16};
     // 33..48 rows: three row tiles instead of four, a quarter less matrix work
-    // (A 1024x1024x512, m = 48: float32 TN 614 -> 495 us in repeated calls; after
-    // a cache flush NN 636 -> 493 us, TN 720 -> 604 us, float64 1.15 -> 1.03 ms)
+    // (A 1024x1024x512, m = 48, after a cache flush, 64-row -> 48-row blocks:
+    // float32 549 -> 469 us NN and 549 -> 467 us TN, float64 980 -> 836 us NN and
+    // 1072 -> 922 us TN)
     if (is_double && f.m > 32 && f.m <= 48) return {3, 2, 1, 16};
     if (is_double && f.m > 16 && f.m <= 64) return {4, 2, 1, 16};
     if (f.m <= 16) return {1, 4, 1, 16};

@@ -22,7 +22,7 @@ enum class Kernel : int
     tn_stream,  // MFMA 16x16x4, w == 1: rows of A contiguous along the contraction mode
     gemm,       // LDS-staged MFMA blocks (ttm_gemm.hip), NN (w % vec == 0) or TN (w == 1) view
     lowp,       // reduced-precision MFMA blocks (ttm_lowp.hip): bf16, fp16, fp16x2, bf16x3, fp8
-    lowp_generic, // reduced precision, one thread per element: short contractions, no room for planes
+    lowp_generic, // reduced precision, one thread per element: few rows of B, short contractions, no room for planes
     skinny,     // vector-ALU stream of B (ttm_skinny.hip): w == 1 with at most eight columns
     count
 };
